@@ -149,11 +149,17 @@ int ta_merge(const void *part, const float *lse, const int32_t *slots,
 /* One decode-step attention layer on resident pools (replaces attention_matrix,
  * kernels.py:152-168): the large-job segment launches, the small-job launch,
  * the TA_TAIL launch that merges the requests owning a tail job, and the merge
- * of the remaining requests (`rest`).  Pools whose capacity is not a multiple
- * of 8 take the unfused order: every segment kind, then the merge of all
- * requests. */
+ * of the remaining requests (`rest`). */
 int ta_attention_matrix(const void *q, const void *kp, const void *vp,
                         int32_t tcap, const ta_plan *plan, void *out, void *stream);
+
+/* ta_attention_matrix on token-major keys and values, as a prefill leaves them
+ * (replaces pack_kv + attention_matrix, kernels.py:144-149): k, v [tokens, hk, d],
+ * contiguous, 16-byte aligned, physical token t of the plan in row t.  The same
+ * launches and partials as ta_attention_matrix; nothing is packed, and the number of
+ * tokens may be any. */
+int ta_attention_tokens(const void *q, const void *k, const void *v, int32_t tokens, const ta_plan *plan,
+                        void *out, void *stream);
 
 /* ta_attention_matrix without caller-provided partial buffers.  No
  * counterpart in the reference: it is for callers that cannot allocate device

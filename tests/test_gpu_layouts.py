@@ -1,0 +1,95 @@
+"""The segment kernels over pools of any capacity and over token-major K/V.
+
+Pools whose capacity is not a multiple of 8 bring K into LDS through registers
+(its rows start at any 2-byte address); ``attention`` reads token-major K and V
+where they lie.  Both run every work-item kind: small and 64/128/256-row items,
+several kinds in one launch, tails that merge their request.  Sizes sit at the
+edges: capacities below one 8-token chunk, last tiles that end with the pool,
+jobs that start anywhere.  Bars as in test_gpu_parity (0.3 % relative L2 against
+the FP32 oracle, atol .008 / rtol .03).
+"""
+import pytest
+import torch
+
+from oracle.attention_oracle import relative_l2, request_attention
+from tree_attention import CostModel, KVTree, schedule, shapes
+from tree_attention import _native
+from tree_attention.kernels import attention, attention_matrix, pack_kv, prepare
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*args):
+    print(*args, flush=True)
+
+
+# (tree spec, methods): what kinds they lower to is asserted below
+TREES = {
+    "tiny": ([-1, 0, 0], [1, 2, 0], [1, 2]),                                        # 3 tokens in all
+    "one_chunk": ([-1, 0, 0], [5, 1, 3], [1, 2]),                                   # 9 tokens
+    "ragged_tails": shapes.shared_prefix(33, 130, [1 + (29 * r) % 131 for r in range(33)]),
+    "wide_root": shapes.shared_prefix(70, 643, [1 + r % 9 for r in range(70)]),     # 256-row items
+    "branches": ([-1] + [0] * 3 + [1 + i % 3 for i in range(45)], [300, 77, 130, 65] + [3 + 11 * i for i in range(45)],
+                 list(range(4, 49))),                                               # 64-row items and small ones
+}
+
+
+@pytest.mark.parametrize("hq,hk,d,dtype", [(32, 8, 128, torch.bfloat16), (8, 2, 64, torch.float16),
+                                           (8, 2, 32, torch.bfloat16)])
+@pytest.mark.parametrize("name", list(TREES))
+def test_any_capacity_and_token_major(name, hq, hk, d, dtype, device):
+    """Every method's plan over pools of 8n + 1 .. 8n + 7 tokens and over token-major K/V."""
+    tree = shapes.tree(TREES[name])
+    t = tree.storage_tokens
+    pads = [p for p in (0, 1, 4) if (t + p) % 8] or [1]
+    g = torch.Generator().manual_seed(d + t)
+    q = torch.randn(len(tree.paths), hq, d, generator=g).to(dtype)
+    k = torch.randn(t + max(pads), hk, d, generator=g).to(dtype)
+    v = torch.randn(t + max(pads), hk, d, generator=g).to(dtype)
+    ref = request_attention(q.float(), k[:t].float(), v[:t].float(), tree)
+    qd, kd, vd = q.to(device), k.to(device), v.to(device)
+    kinds = set()
+    for method in ("request", "fixed", "cube"):
+        for tile_rows in (256, 128, 64):
+            plan = schedule(tree, hq, hk, d, method, CostModel(kv_split=200, max_query_rows=512))
+            p = prepare(plan, qd, tile_rows=tile_rows, route_items=0)  # the large jobs stay large
+            outs = {f"token-major {tile_rows}": attention(qd, kd[:t], vd[:t], p).clone()}
+            for pad in pads:
+                kp, vp = pack_kv(kd[:t + pad], vd[:t + pad])
+                assert kp.shape[2] % 8
+                outs[f"capacity {t + pad} {tile_rows}"] = attention_matrix(qd, kp, vp, p).clone()
+                kinds |= {i for i in range(_native.TA_NKINDS) if p.for_pools(kp).abi.n_items[i]}
+            torch.cuda.synchronize()
+            for what, out in outs.items():
+                say(name, method, what, list(p.abi.n_items))
+                torch.testing.assert_close(out.cpu(), ref.to(dtype), atol=0.008, rtol=0.03,
+                                           msg=lambda m: f"{method} {what}: {m}")
+                assert relative_l2(out.cpu(), ref) <= 3e-3, (method, what)
+    if name == "wide_root":
+        assert {_native.TA_LARGE64, _native.TA_LARGE128, _native.TA_LARGE256} <= kinds
+    if name == "branches":
+        assert {_native.TA_SMALL, _native.TA_LARGE64} <= kinds
+
+
+def test_token_major_equals_packed(device):
+    """Token-major K/V give the bits of the packed pools of an aligned capacity (same tiles, same
+    order), attachments included; views that are not contiguous are packed as before."""
+    tree = KVTree.synthetic([-1] + [0] * 96, [2043] + [1 + (37 * r) % 200 for r in range(96)], list(range(1, 97)))
+    t = -(-tree.storage_tokens // 8) * 8
+    g = torch.Generator().manual_seed(8)
+    q = torch.randn(96, 32, 128, generator=g).bfloat16().to(device)
+    k = torch.randn(t, 8, 128, generator=g).bfloat16().to(device)
+    v = torch.randn(t, 8, 128, generator=g).bfloat16().to(device)
+    p = prepare(schedule(tree, 32, 8, 128, "cube", CostModel.mi355x()), q)
+    assert p.attached
+    a = attention(q, k, v, p).clone()
+    b = attention_matrix(q, *pack_kv(k, v), p).clone()
+    strided = torch.stack([k, k], dim=1)[:, 0]
+    assert not strided.is_contiguous()
+    c = attention(q, strided, v, p).clone()
+    torch.cuda.synchronize()
+    assert torch.equal(a, b) and torch.equal(a, c)
+    with pytest.raises(ValueError):
+        attention(q, k.half(), v, p)
+    with pytest.raises(ValueError):
+        attention(q[:3], k, v, p)

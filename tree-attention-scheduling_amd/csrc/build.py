@@ -13,6 +13,7 @@ import shutil
 import subprocess
 import sys
 import tempfile
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
@@ -38,9 +39,11 @@ COMMON = [
 # compile to v_max3_f32 chains without a canonicalising v_max per input; the
 # kernel never produces NaN scores (masked tokens are selected to -inf).
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
+# segment_tile.hip is compiled once per K/V layout (enum Layout, ta_common.h).
 SOURCES = [
     (HERE / "tree_attn.hip", VGPR_FORM),
-    (HERE / "segment_tile.hip", VGPR_FORM + ["-fno-honor-nans"]),
+    *[(HERE / "segment_tile.hip", VGPR_FORM + ["-fno-honor-nans", f"-DTA_LAYOUT={layout}"])
+      for layout in ("KV_POOL", "KV_ODD", "KV_TOKEN")],
     (HERE / "decode_append.hip", ["-ffp-contract=off"]),  # each RoPE product rounded, as the eager ops
 ]
 
@@ -67,12 +70,15 @@ def build(verbose: bool = False, out: Path | None = None, defines=()) -> Path:
     target = Path(out) if out is not None else LIB
     tmp = target.with_name(target.name + f".tmp{os.getpid()}")
     with tempfile.TemporaryDirectory() as work:
-        objs = []
-        for src, extra in SOURCES:
-            obj = Path(work) / (src.stem + ".o")
+        def compile_one(i):
+            src, extra = SOURCES[i]
+            obj = Path(work) / f"{src.stem}_{i}.o"
             _run([hipcc(), *COMMON, *extra, *[f"-D{d}" for d in defines], f"-I{INCLUDE}", f"-I{HERE}",
                   "-c", str(src), "-o", str(obj)], verbose)
-            objs.append(str(obj))
+            return str(obj)
+
+        with ThreadPoolExecutor(4) as pool:  # each unit takes up to a minute
+            objs = list(pool.map(compile_one, range(len(SOURCES))))
         _run([hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", str(tmp)], verbose)
     os.replace(tmp, target)
     return target

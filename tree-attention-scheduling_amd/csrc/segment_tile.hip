@@ -35,19 +35,30 @@
 //    operand, so z sums exactly the rounded P that multiplies V.
 //  * Softmax in base 2 with log2(e)/sqrt(D) folded into one FMA; lazy
 //    rescaling (the running maximum moves only by more than TAU).
-// Requirements (checked by the launcher): tcap % 8 == 0 and 16-byte aligned
-// pools, so every 8-token chunk of a K row is one aligned 16-byte copy.
+// The kernels are templates over the layout of K and V (enum Layout): pools whose
+// capacity is a multiple of 8 (every 8-token chunk of a K row is one aligned
+// 16-byte copy), pools of any other capacity (K through registers) and
+// token-major K and V (K's operand read without transposing).  The text above
+// describes the first; TileCopy and KTokens say where the others differ.
 #include "ta_common.h"
 #include "tree_attn.h"
+
+#ifndef TA_LAYOUT
+#define TA_LAYOUT KV_POOL  // the layout this translation unit's kernels are compiled for
+#endif
 
 namespace ta {
 namespace {
 
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(3))) const u16 lds_u16;
 
 // s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding).
 #define TA_VMCNT(n) ((((n)&15) | (7 << 4) | (15 << 8) | ((((n) >> 4) & 3) << 14)))
+
+// s_waitcnt lgkmcnt(0) alone
+#define TA_LGKMCNT0 (15 | (7 << 4) | (0 << 8) | (3 << 14))
 
 // Wait until at most n tiles of this wave's copies (BPW each) are in flight
 // (n = 0 .. 4; the immediate of s_waitcnt must be a constant).
@@ -85,6 +96,7 @@ __device__ inline u32x4 tr_pair(const u16 *lo, const u16 *hi) {
 // 32 KiB and five of them fit the 160 KiB LDS.
 struct LdsOfs {  // per-lane element offsets of the transposing reads (swizzle applied)
     int klo, khi;        // K: the two 8-byte halves of a lane's operand
+    int kt[4];           // KV_TOKEN: K's 16-byte chunk of the lane's token, per 32-wide slice of d
     int vlo[2], vhi[2];  // V: same, by the parity of the 16-row block db of O^T
 };
 
@@ -124,11 +136,156 @@ struct Tile {
             o.vlo[e] = BLK * vb + swz(blo, dbo + vin) - dbo;
             o.vhi[e] = BLK * (vb + 16 / VROWS) + swz(bhi, dbo + vin) - dbo;
         }
+#pragma unroll
+        for (int ks = 0; ks < D / 32; ++ks) o.kt[ks] = row * D + 8 * ((4 * ks + g4) ^ ((row / (128 / D)) % (D / 8)));
         return o;
     }
 };
 
-template <int D, bool FP16, int NB, int NW>
+// K of a KV_TOKEN tile: token rows of D elements, CPR 16-byte chunks each.  The
+// QK operand is 16 contiguous bytes of one token, read without transposing;
+// chunk c of token t sits at chunk c ^ flip(t) of its row, so that the 16 lanes
+// (one chunk of 16 tokens) that read together cover 256 different bytes.
+template <int D>
+struct KTokens {
+    static constexpr int CPR = D / 8;
+    static constexpr int TPL = 16 / CPR;  // token rows of 256 bytes
+    __device__ static int flip(int t) { return (t / TPL) % CPR; }
+};
+
+// Copies of one 64-token tile into an LDS stage by NW waves.  Inside the job
+// (tokens [t0n, t0n + TT) all in [kst, kend)) no index is clamped; at its edges
+// chunks past the pool end read its last chunk and V rows outside the job read
+// a row inside it (finite values; their scores are masked, P = 0).
+//
+// KV_POOL and KV_TOKEN copy both operands by LDS DMA: issue() is all.  A KV_ODD
+// pool's K rows start at any 2-byte address, which the DMA does not take: issue()
+// loads each lane's 16 bytes into registers (unaligned global loads) and starts V's
+// DMA, finish() waits for both and writes K to LDS at the slots the DMA would have
+// filled.  The tile's compute runs between the two and hides the loads.  Moving both
+// operands through registers with an 8 x 8 transpose took twice as long (24 ragged
+// requests in two branches, 10,839 tokens, d = 128: layer 49.2 us, here 26.7 us; 32
+// ragged requests, 1,745 tokens, d = 64: 14.2 us, here 8.4 us).
+template <int D, int NW, int L>
+struct TileCopy {
+    using T = Tile<D>;
+    static constexpr int NK = (T::KBLK + NW - 1) / NW;  // K blocks of a wave, V likewise (D = 32: of some waves)
+    u32x4 k[L == KV_ODD ? NK : 1];
+
+    // V row t of head h
+    __device__ static const u16 *vrow(const SegParams &p, int h, int t) {
+        return p.vp + (L == KV_TOKEN ? (size_t)t * p.hk + h : (size_t)h * p.tcap + t) * D;
+    }
+
+    template <bool CLAMP>
+    __device__ static void copy_v(u16 *st, const SegParams &p, int h, int t0n, int kst, int kend, int vb, int lane) {
+        const int l = lane ^ (8 * ((T::KBLK + vb) & 1));  // logical slot filled by this lane (swizzle)
+        const int rem = l % T::SV;
+        const int s = 2 * (l / T::SV) + ((rem >> 2) & 1);
+        const int j = 4 * (rem >> 3) + (rem & 3);
+        const int t = t0n + vb * T::VROWS + j;
+        const u16 *src = vrow(p, h, CLAMP ? min(max(t, kst), kend - 1) : t) + 8 * s;
+        __builtin_amdgcn_global_load_lds((const void *)src, (lds_void *)(st + (T::KBLK + vb) * T::BLK), 16, 0, 0);
+    }
+
+    template <bool CLAMP>
+    __device__ static void copy_k(u16 *st, const SegParams &p, int h, int t0n, int kst, int kend, int blk, int lane) {
+        const u16 *src;
+        if constexpr (L == KV_TOKEN) {
+            // row-major tile: lane i fills slot i, chunk (i % CPR) ^ f of token row i / CPR (KTokens)
+            const int j = lane / KTokens<D>::CPR, t = blk * T::VROWS + j;
+            const int s = (lane % KTokens<D>::CPR) ^ KTokens<D>::flip(t);
+            const int tok = t0n + t;
+            src = p.kp + ((size_t)(CLAMP ? min(max(tok, kst), kend - 1) : tok) * p.hk + h) * D + 8 * s;
+        } else {
+            const int l = lane ^ (8 * (blk & 1));
+            const int ck = 2 * (l >> 4) + ((l >> 2) & 1);
+            const int d = 8 * blk + 4 * ((l >> 3) & 1) + (l & 3);
+            const int tok = t0n + 8 * ck;
+            src = p.kp + (size_t)(h * D + d) * p.tcap + (CLAMP ? min(tok, p.tcap - 8) : tok);
+        }
+        __builtin_amdgcn_global_load_lds((const void *)src, (lds_void *)(st + blk * T::BLK), 16, 0, 0);
+    }
+
+    template <bool CLAMP>
+    __device__ static void copy_blocks(u16 *st, const SegParams &p, int h, int t0n, int kst, int kend, int w, int lane) {
+#pragma unroll
+        for (int n = 0; n < T::NBLK / NW; ++n) {
+            // One wave alone alternates K (64 tokens of 8 rows, tcap apart) and V (one run of
+            // 1 KiB): 16 strided blocks in a row, then 16 of a run, kept fewer HBM channels
+            // busy (128 x 8192 private tokens, 4.3 GB: 818 us against 776 us).
+            const int i = NW == 1 ? (n & 1) * T::KBLK + (n >> 1) : n;
+            const int blk = w + i * NW;
+            // with KBLK % NW == 0 every wave's i-th block is K for the same i
+            const bool isk = T::KBLK % NW == 0 ? i * NW < T::KBLK : blk < T::KBLK;
+            if (isk)
+                copy_k<CLAMP>(st, p, h, t0n, kst, kend, blk, lane);
+            else
+                copy_v<CLAMP>(st, p, h, t0n, kst, kend, blk - T::KBLK, lane);
+        }
+    }
+
+    // KV_ODD: this wave's K blocks of the tile into registers
+    __device__ void load_k(const SegParams &p, int h, int t0n, int w, int lane) {
+        const bool inside = t0n + T::TT <= p.tcap;
+#pragma unroll
+        for (int i = 0; i < NK; ++i) {
+            const int blk = w + i * NW;
+            if (T::KBLK % NW != 0 && blk >= T::KBLK) continue;
+            const int l = lane ^ (8 * (blk & 1));
+            const int tok = t0n + 8 * (2 * (l >> 4) + ((l >> 2) & 1));
+            const int d = 8 * blk + 4 * ((l >> 3) & 1) + (l & 3);
+            const u16 *src = p.kp + (size_t)(h * D + d) * p.tcap;
+            if (inside) {
+                __builtin_memcpy(&k[i], src + tok, 16);
+            } else {  // the pool's last tile, element by element
+                u32 e[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) e[j] = src[min(tok + j, p.tcap - 1)];
+                k[i] = u32x4{e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16};
+            }
+        }
+    }
+
+    __device__ void issue(u16 *st, const SegParams &p, int h, int t0n, int kst, int kend, int wave, int lane) {
+        const int w = __builtin_amdgcn_readfirstlane(wave);
+        const bool inner = t0n >= kst && t0n + T::TT <= kend;
+        if constexpr (L == KV_ODD) {
+            load_k(p, h, t0n, w, lane);
+#pragma unroll
+            for (int i = 0; i < NK; ++i) {
+                const int vb = w + i * NW;
+                if (T::VBLK % NW != 0 && vb >= T::VBLK) continue;
+                if (inner)
+                    copy_v<false>(st, p, h, t0n, kst, kend, vb, lane);
+                else
+                    copy_v<true>(st, p, h, t0n, kst, kend, vb, lane);
+            }
+        } else if (inner) {
+            copy_blocks<false>(st, p, h, t0n, kst, kend, w, lane);
+        } else {
+            copy_blocks<true>(st, p, h, t0n, kst, kend, w, lane);
+        }
+    }
+
+    // KV_ODD: everything issued has landed; K goes to the stage.  The LDS writes
+    // are done when this returns (a barrier makes them the other waves').
+    __device__ void finish(u16 *st, int wave, int lane) {
+        if constexpr (L == KV_ODD) {
+            const int w = __builtin_amdgcn_readfirstlane(wave);
+            __builtin_amdgcn_s_waitcnt(TA_VMCNT(0));
+#pragma unroll
+            for (int i = 0; i < NK; ++i) {
+                const int blk = w + i * NW;
+                if (T::KBLK % NW != 0 && blk >= T::KBLK) continue;
+                *(u32x4 *)(st + blk * T::BLK + 8 * lane) = k[i];
+            }
+            __builtin_amdgcn_s_waitcnt(TA_LGKMCNT0);
+        }
+    }
+};
+
+template <int D, bool FP16, int NB, int NW, int L>
 struct TileMath {
     static constexpr int DB = D / 16;  // 16-row blocks of O^T
     static constexpr int KS = D / 32;  // 32-wide k slices of QK
@@ -153,57 +310,25 @@ struct TileMath {
     // stages never alias; declaring them restrict in one function lets the
     // compiler keep the copies in flight across the reads of `cur`.
     __device__ void step(const u16 *__restrict__ cur, u16 *__restrict__ nxt, bool copy, bool compute,
-                         const u16 *__restrict__ kp, const u16 *__restrict__ vp, int h, int tcap, int t0n, int kst,
-                         int kend, int wave, int lane, const u32x4 (&qf)[NB][KS], const LdsOfs &of, int lo,
-                         int hi, int g4, float c) {
-        if (copy) this->copy(nxt, kp, vp, h, tcap, t0n, kst, kend, wave, lane);
+                         const SegParams &p, int h, int t0n, int kst, int kend, int wave, int lane,
+                         const u32x4 (&qf)[NB][KS], const LdsOfs &of, int lo, int hi, int g4, float c) {
+        using C = TileCopy<D, NW, L>;
+        C kr;
+        if (copy) kr.issue(nxt, p, h, t0n, kst, kend, wave, lane);
         if (compute) tile(cur, qf, of, lo, hi, g4, c);
-    }
-
-    // Copy the tile at pool token t0n into stage `st` (this wave's blocks).
-    // Inside the job (tokens [t0n, t0n + TT) all in [kst, kend)) no index is
-    // clamped; at its edges chunks past the pool end read its last chunk and
-    // V rows outside the job read a row inside it (finite values; their
-    // scores are masked, P = 0).
-    __device__ static void copy(u16 *st, const u16 *__restrict__ kp, const u16 *__restrict__ vp, int h,
-                                int tcap, int t0n, int kst, int kend, int wave, int lane) {
-        const int w = __builtin_amdgcn_readfirstlane(wave);
-        if (t0n >= kst && t0n + T::TT <= kend)
-            copy_blocks<false>(st, kp, vp, h, tcap, t0n, kst, kend, w, lane);
-        else
-            copy_blocks<true>(st, kp, vp, h, tcap, t0n, kst, kend, w, lane);
-    }
-
-    template <bool CLAMP>
-    __device__ static void copy_blocks(u16 *st, const u16 *__restrict__ kp, const u16 *__restrict__ vp, int h,
-                                       int tcap, int t0n, int kst, int kend, int w, int lane) {
-#pragma unroll
-        for (int i = 0; i < T::NBLK / NW; ++i) {
-            const int blk = w + i * NW;
-            // with KBLK % NW == 0 every wave's i-th block is K for the same i
-            const bool isk = T::KBLK % NW == 0 ? i * NW < T::KBLK : blk < T::KBLK;
-            const u16 *src;
-            const int l = lane ^ (8 * (blk & 1));  // logical slot filled by this lane (swizzle)
-            if (isk) {
-                const int ck = 2 * (l >> 4) + ((l >> 2) & 1);
-                const int d = 8 * blk + 4 * ((l >> 3) & 1) + (l & 3);
-                const int tok = t0n + 8 * ck;
-                src = kp + (size_t)(h * D + d) * tcap + (CLAMP ? min(tok, tcap - 8) : tok);
-            } else {
-                const int vb = blk - T::KBLK;
-                const int rem = l % T::SV;
-                const int s = 2 * (l / T::SV) + ((rem >> 2) & 1);
-                const int j = 4 * (rem >> 3) + (rem & 3);
-                const int t = t0n + vb * T::VROWS + j;
-                src = vp + ((size_t)h * tcap + (CLAMP ? min(max(t, kst), kend - 1) : t)) * D + 8 * s;
-            }
-            __builtin_amdgcn_global_load_lds((const void *)src, (lds_void *)(st + blk * T::BLK), 16, 0, 0);
-        }
+        if (copy) kr.finish(nxt, wave, lane);
     }
 
     // K fragments (A operand of QK) of the 32 tokens base .. base+31:
     // kf[b][ks] covers tokens base+16b .. +15, d = 32*ks .. +31.
     __device__ static void load_k(const u16 *__restrict__ cur, const LdsOfs &of, int base, u32x4 (&kf)[2][KS]) {
+        if constexpr (L == KV_TOKEN) {
+            u32 a[KS];
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) a[ks] = (u32)(uintptr_t)(lds_u16 *)(cur + of.kt[ks] + base * D);
+            read_tokens(a, kf);
+            return;
+        }
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
@@ -212,6 +337,35 @@ struct TileMath {
                 const int e = 4 * T::BLK * ks + 8 * (base + 16 * b);
                 kf[b][ks] = tr_pair(cur + of.klo + e, cur + of.khi + e);
             }
+    }
+
+    // KV_TOKEN: the chunks at LDS byte addresses a[ks] and 16 tokens further.  For
+    // an ordinary LDS read the compiler waits for every LDS DMA in flight (it
+    // cannot tell the stages apart), so these are written out, wait included.
+    __device__ static void read_tokens(const u32 (&a)[KS], u32x4 (&kf)[2][KS]) {
+        constexpr int N = 32 * D;  // bytes of 16 token rows
+        if constexpr (KS == 4)
+            asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %1, %9\n\t"
+                         "ds_read_b128 %2, %10\n\tds_read_b128 %3, %11\n\t"
+                         "ds_read_b128 %4, %8 offset:%12\n\tds_read_b128 %5, %9 offset:%12\n\t"
+                         "ds_read_b128 %6, %10 offset:%12\n\tds_read_b128 %7, %11 offset:%12\n\t"
+                         "s_waitcnt lgkmcnt(0)"
+                         : "=&v"(kf[0][0]), "=&v"(kf[0][1]), "=&v"(kf[0][2]), "=&v"(kf[0][3]), "=&v"(kf[1][0]),
+                           "=&v"(kf[1][1]), "=&v"(kf[1][2]), "=&v"(kf[1][3])
+                         : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "n"(N)
+                         : "memory");
+        else if constexpr (KS == 2)
+            asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\t"
+                         "ds_read_b128 %2, %4 offset:%6\n\tds_read_b128 %3, %5 offset:%6\n\t"
+                         "s_waitcnt lgkmcnt(0)"
+                         : "=&v"(kf[0][0]), "=&v"(kf[0][1]), "=&v"(kf[1][0]), "=&v"(kf[1][1])
+                         : "v"(a[0]), "v"(a[1]), "n"(N)
+                         : "memory");
+        else
+            asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:%3\n\ts_waitcnt lgkmcnt(0)"
+                         : "=&v"(kf[0][0]), "=&v"(kf[1][0])
+                         : "v"(a[0]), "n"(N)
+                         : "memory");
     }
 
     // V^T fragments (A operand of PV) of the 32 tokens base .. base+31: PV
@@ -320,6 +474,14 @@ __device__ inline int xcd_item(int b, int n) {
     return xcd * q8 + min(xcd, rm) + slot;
 }
 
+// First token of the tiles of a job or segment that starts at token t: a KV_POOL
+// K row is copied in aligned chunks of 8 tokens (KV_TOKEN follows it, so that both
+// sum in the same order; KV_ODD starts at the job's first token).
+template <int L>
+__device__ inline int tile_start(int t) {
+    return L == KV_ODD ? t : t & ~7;
+}
+
 // The waves of a work item meet at a barrier, unless one wave works alone on
 // its own LDS stage (SOLO), where its own vmcnt wait orders copy and reads.
 template <bool SOLO>
@@ -330,11 +492,12 @@ __device__ inline void item_barrier() {
 // One work item (job, first row, KV head) of the tile kernels: NW waves, NB
 // 16-row blocks per wave, STAGES LDS stages at `lds`.  The item holds rows
 // [row0, row0 + item_rows) of its job.  SOLO: one wave alone (tid = its lane).
-template <int D, bool FP16, int NB, int NW, int STAGES, bool SOLO = false>
+template <int D, bool FP16, int NB, int NW, int STAGES, int L, bool SOLO = false>
 __device__ __forceinline__ void tile_item(const SegParams &p, const int32_t *__restrict__ items, int item,
                                           u16 *lds, int tid, int item_rows) {
     using T = Tile<D>;
-    using M = TileMath<D, FP16, NB, NW>;
+    using M = TileMath<D, FP16, NB, NW, L>;
+    using C = TileCopy<D, NW, L>;
     constexpr int KS = M::KS;
     constexpr int BPW = T::NBLK / NW;  // copies per wave per tile
     static_assert(T::NBLK % NW == 0, "every wave copies the same number of blocks");
@@ -379,15 +542,17 @@ __device__ __forceinline__ void tile_item(const SegParams &p, const int32_t *__r
     acc.reset();
     const LdsOfs of = T::offsets(row, g4);
 
-    const int tb0 = kst & ~7;
+    const int tb0 = tile_start<L>(kst);
     const int ntiles = ntok > 0 ? (kend - tb0 + T::TT - 1) / T::TT : 0;
     if (STAGES == 1) {
         // one stage (one-wave workgroups, four per CU): copy, wait, compute
         for (int it = 0; it < ntiles; ++it) {
             const int t0 = tb0 + it * T::TT;
             if (it > 0) item_barrier<SOLO>();  // every wave is done with the previous tile
-            acc.copy(lds, p.kp, p.vp, h, p.tcap, t0, kst, kend, wave, lane);
+            C kr;
+            kr.issue(lds, p, h, t0, kst, kend, wave, lane);
             __builtin_amdgcn_s_waitcnt(TA_VMCNT(0));
+            kr.finish(lds, wave, lane);
             item_barrier<SOLO>();
             if (active) acc.tile(lds, qf, of, max(0, kst - t0), min(T::TT, kend - t0), g4, p.scale_log2);
         }
@@ -401,7 +566,7 @@ __device__ __forceinline__ void tile_item(const SegParams &p, const int32_t *__r
         if (it >= 0) {
             // this wave's copies of tile it are done once at most those of the
             // tiles after it (issued, at most AHEAD-1 of them) are pending
-            if (AHEAD == 2 && it + 1 < ntiles)
+            if (AHEAD == 2 && it + 1 < ntiles && L != KV_ODD)  // (KV_ODD: finish() waited for all)
                 __builtin_amdgcn_s_waitcnt(TA_VMCNT(BPW));
             else
                 __builtin_amdgcn_s_waitcnt(TA_VMCNT(0));
@@ -409,9 +574,9 @@ __device__ __forceinline__ void tile_item(const SegParams &p, const int32_t *__r
         }
         const int ns = cs == 0 ? STAGES - 1 : cs - 1;  // stage of tile it+AHEAD (that of tile it-1)
         const int t0 = tb0 + it * T::TT;
-        acc.step(lds + cs * T::ELEMS, lds + ns * T::ELEMS, it + AHEAD < ntiles, it >= 0 && active, p.kp, p.vp, h,
-                 p.tcap, t0 + AHEAD * T::TT, kst, kend, wave, lane, qf, of, max(0, kst - t0),
-                 min(T::TT, kend - t0), g4, p.scale_log2);
+        acc.step(lds + cs * T::ELEMS, lds + ns * T::ELEMS, it + AHEAD < ntiles, it >= 0 && active, p, h,
+                 t0 + AHEAD * T::TT, kst, kend, wave, lane, qf, of, max(0, kst - t0), min(T::TT, kend - t0), g4,
+                 p.scale_log2);
         cs = cs == STAGES - 1 ? 0 : cs + 1;
     }
     }
@@ -428,10 +593,10 @@ __device__ __forceinline__ void tile_item(const SegParams &p, const int32_t *__r
     }
 }
 
-template <int D, bool FP16, int NB, int NW, int STAGES>
+template <int D, bool FP16, int NB, int NW, int STAGES, int L>
 __global__ __launch_bounds__(64 * NW) void seg_tile_kernel(SegParams p) {
     __shared__ __attribute__((aligned(16))) u16 lds[STAGES * Tile<D>::ELEMS];
-    tile_item<D, FP16, NB, NW, STAGES>(p, p.items, xcd_item(blockIdx.x, gridDim.x), lds, threadIdx.x, 16 * NB * NW);
+    tile_item<D, FP16, NB, NW, STAGES, L>(p, p.items, xcd_item(blockIdx.x, gridDim.x), lds, threadIdx.x, 16 * NB * NW);
 }
 
 // ------------------------------------------------------------------------
@@ -449,14 +614,14 @@ __global__ __launch_bounds__(64 * NW) void seg_tile_kernel(SegParams p) {
 // instructions alternate in each wave's instruction stream.  K/V tiles arrive
 // by LDS DMA into five stages: tiles t and t+1 are read while t+2 .. t+4 are
 // in flight, with one barrier per tile.
-template <int D, bool FP16, int NW, int NB_ = 2>
+template <int D, bool FP16, int NW, int NB_, int L>
 struct PipeMath {
     static constexpr int NB = NB_;
     static constexpr int DB = D / 16;
     static constexpr int KS = D / 32;
     using O = Ops<FP16>;
     using T = Tile<D>;
-    using TM = TileMath<D, FP16, NB, NW>;
+    using TM = TileMath<D, FP16, NB, NW, L>;
 
     f32x4 o[NB][DB], z[NB];
     float m[NB], lm[NB], thr[NB];  // running max (scaled), raw row max of the staged step, (m + TAU) / c
@@ -629,17 +794,19 @@ struct PipeMath {
 // the first loop barrier issues the rest of the ring.
 // One 256-row work item of the pipelined kernel, with its attached segments
 // (p.xtail, indexed by the item), STAGES LDS stages at `lds`.
-template <int D, bool FP16, int NW, int NB = 2, int STAGES = TA_PIPE_STAGES, int SYNC = 1, int PRO = TA_PIPE_PRO>
+template <int D, bool FP16, int NW, int NB, int L, int STAGES = TA_PIPE_STAGES, int SYNC = 1, int PRO = TA_PIPE_PRO>
 __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__restrict__ items, int item, u16 *lds,
                                           int tid) {
     using T = Tile<D>;
-    using M = PipeMath<D, FP16, NW, NB>;
-    using TM = TileMath<D, FP16, NB, NW>;
+    using M = PipeMath<D, FP16, NW, NB, L>;
+    using TM = TileMath<D, FP16, NB, NW, L>;
+    using C = TileCopy<D, NW, L>;
     constexpr int KS = M::KS;
     constexpr int BPW = T::NBLK / NW;  // copies per wave per tile
     static_assert(T::NBLK % NW == 0, "every wave copies the same number of blocks");
     static_assert(SYNC >= 1 && STAGES >= 2 * SYNC + 1 && STAGES <= 5,
                   "a group's tiles, the next K and the next group's copies fit the stages");
+    static_assert(L != KV_ODD || SYNC == 1, "KV_ODD sends one tile per group");
     static_assert(PRO >= SYNC + 1 && PRO <= STAGES, "the prologue issues the tiles the first group reads");
     const int job = items[3 * item], row0 = items[3 * item + 1], h = items[3 * item + 2];
 
@@ -652,7 +819,7 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
     const int wrow0 = row0 + 16 * NB * wave;
     const bool active = wrow0 < nrows;
     const float c = p.scale_log2, rc = 1.f / p.scale_log2;
-    const int tb0 = kst & ~7;
+    const int tb0 = tile_start<L>(kst);
     const int ntiles = ntok > 0 ? (kend - tb0 + T::TT - 1) / T::TT : 0;
     const int nsteps = ntok > 0 ? (kend - tb0 + 31) / 32 : 0;
     auto tile_stage = [&](int t) { return lds + (t % STAGES) * T::ELEMS; };
@@ -683,25 +850,31 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
     for (int k = 0; k < XM; ++k) {
         xs[k] = max(0, rec[1 + XF * k]);
         xe[k] = xs[k] + max(0, min(rec[2 + XF * k], p.tcap - xs[k]));
-        xn[k] = k < nx && xe[k] > xs[k] ? (xe[k] - (xs[k] & ~7) + T::TT - 1) / T::TT : 0;
+        xn[k] = k < nx && xe[k] > xs[k] ? (xe[k] - tile_start<L>(xs[k]) + T::TT - 1) / T::TT : 0;
         xfirst[k] = ntot;
         ntot += xn[k];
     }
-    // copy tile t of the sequence into stage st
-    auto copy_tile = [&](int t, u16 *st) {
+    // start the copies of tile t of the sequence into stage st
+    auto start_tile = [&](C &kr, int t, u16 *st) {
         if (t < ntiles) {
-            TM::copy(st, p.kp, p.vp, h, p.tcap, tb0 + t * T::TT, kst, kend, wave, lane);
+            kr.issue(st, p, h, tb0 + t * T::TT, kst, kend, wave, lane);
             return;
         }
         int t0n = 0, cs = 0, ce = 1;
 #pragma unroll
         for (int k = 0; k < XM; ++k)
             if (t >= xfirst[k] && t < xfirst[k] + xn[k]) {
-                t0n = (xs[k] & ~7) + (t - xfirst[k]) * T::TT;
+                t0n = tile_start<L>(xs[k]) + (t - xfirst[k]) * T::TT;
                 cs = xs[k];
                 ce = xe[k];
             }
-        TM::copy(st, p.kp, p.vp, h, p.tcap, t0n, cs, ce, wave, lane);
+        kr.issue(st, p, h, t0n, cs, ce, wave, lane);
+    };
+    // ... and, for KV_ODD, finish them
+    auto copy_tile = [&](int t, u16 *st) {
+        C kr;
+        start_tile(kr, t, st);
+        kr.finish(st, wave, lane);
     };
 
     int issued = 0;  // tiles of the sequence whose copies this wave has issued
@@ -718,7 +891,8 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
     // 1 .. PRO-1 follow.
     const int qb = p.qbase ? p.qbase[job] : -1;
     int rq[NB];
-    if (qb < 0 && ntot > 0) copy_tile(0, lds);
+    C pro[L == KV_ODD ? PRO : 1];  // (KV_ODD: the first tiles' K, until all are on their way)
+    if (qb < 0 && ntot > 0) start_tile(pro[0], 0, lds);
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
         const int rr = max(0, min(wrow0 + 16 * nb + row, nrows - 1));
@@ -732,7 +906,7 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
 #pragma unroll
         for (int k = 0; k < KS; ++k) qf[nb][k] = *(const u32x4 *)(src + 32 * k);
     }
-    if (qb >= 0 && ntot > 0) copy_tile(0, lds);  // behind the Q loads: one wait covers both
+    if (qb >= 0 && ntot > 0) start_tile(pro[0], 0, lds);  // behind the Q loads: one wait covers both
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
         const bool valid = wrow0 + 16 * nb + row < nrows;
@@ -742,7 +916,16 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
             asm volatile("" : "+v"(qf[nb][k]));
         }
     }
-    for (int t = 1; t < PRO && t < ntot; ++t) copy_tile(t, tile_stage(t));
+    if constexpr (L == KV_ODD) {
+#pragma unroll
+        for (int t = 1; t < PRO; ++t)
+            if (t < ntot) start_tile(pro[t], t, tile_stage(t));
+#pragma unroll
+        for (int t = 0; t < PRO; ++t)
+            if (t < ntot) pro[t].finish(tile_stage(t), wave, lane);
+    } else {
+        for (int t = 1; t < PRO && t < ntot; ++t) copy_tile(t, tile_stage(t));
+    }
     issued = min(PRO, ntot);
 
     M acc;
@@ -765,8 +948,22 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
     // at the previous group); the later issued ones may still be in flight.
     // Once every wave passed the barrier the stages of the previous group are
     // free for tiles up to t+STAGES-1.
+    // KV_ODD: one tile per group is on its way, its K in registers (odd_k) since
+    // the previous group; it goes to LDS before the barrier.
+    C odd_k;
+    int odd_tile = -1;
     auto sync_tile = [&](int t) {
         if (t % SYNC != 0 || t + 1 >= ntot) return;
+        if constexpr (L == KV_ODD) {
+            if (odd_tile >= 0) odd_k.finish(tile_stage(odd_tile), wave, lane);
+            odd_tile = -1;
+            __builtin_amdgcn_s_barrier();
+            if (issued < min(t + STAGES, ntot)) {
+                odd_tile = issued++;
+                start_tile(odd_k, odd_tile, tile_stage(odd_tile));
+            }
+            return;
+        }
         wait_tiles<BPW>(max(0, issued - 1 - (t + SYNC)));
         __builtin_amdgcn_s_barrier();
         for (; issued < min(t + STAGES, ntot); ++issued) copy_tile(issued, tile_stage(issued));
@@ -801,7 +998,7 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
     // together: one wait and one barrier per round, then every wave attends
     // the round's tiles of the segments holding its rows, side by side.  The
     // root loop (or the prologue) already issued the first tiles.
-    {
+    if constexpr (L != KV_ODD) {  // (the launcher passes no attachments for KV_ODD)
         for (int r0 = ntiles; r0 < ntot; r0 += STAGES) {
             const int r1 = min(r0 + STAGES, ntot);
             __builtin_amdgcn_s_barrier();  // every wave is done with the tiles before r0
@@ -815,7 +1012,7 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
                 const int rlo = rec[3 + XF * k] - wrow0;
                 if (xn[k] > 0 && active && rlo < 16 * NB && rlo + rec[4 + XF * k] > 0) {
                     for (int i = max(0, r0 - xfirst[k]); i < xn[k] && xfirst[k] + i < r1; ++i) {
-                        const int t0 = (xs[k] & ~7) + i * T::TT;
+                        const int t0 = tile_start<L>(xs[k]) + i * T::TT;
                         acc.tail_tile(tile_stage(xfirst[k] + i), qf, of, max(0, xs[k] - t0), min(T::TT, xe[k] - t0),
                                       rlo, rlo + rec[4 + XF * k], row, g4, c, rc);
                     }
@@ -839,20 +1036,20 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
 // A 256-row work item whose job has at most 8 NW rows from the item's first
 // row on runs 16 rows per wave, so that every wave computes (two per SIMD)
 // instead of half of them 32 rows each; the arithmetic of every row is the same.
-template <int D, bool FP16, int NW>
+template <int D, bool FP16, int NW, int L>
 __device__ __forceinline__ void pipe_item_rows(const SegParams &p, const int32_t *__restrict__ items, int item,
                                                u16 *lds, int tid) {
     const int job = items[3 * item], row0 = items[3 * item + 1];
     if (p.qlen[job] * p.group - row0 <= 16 * NW)
-        pipe_item<D, FP16, NW, 1>(p, items, item, lds, tid);
+        pipe_item<D, FP16, NW, 1, L>(p, items, item, lds, tid);
     else
-        pipe_item<D, FP16, NW, 2>(p, items, item, lds, tid);
+        pipe_item<D, FP16, NW, 2, L>(p, items, item, lds, tid);
 }
 
-template <int D, bool FP16, int NW>
+template <int D, bool FP16, int NW, int L>
 __global__ __launch_bounds__(64 * NW) void seg_pipe_kernel(SegParams p) {
     __shared__ __attribute__((aligned(16))) u16 lds[TA_PIPE_STAGES * Tile<D>::ELEMS];
-    pipe_item_rows<D, FP16, NW>(p, p.items, xcd_item(blockIdx.x, gridDim.x), lds, threadIdx.x);
+    pipe_item_rows<D, FP16, NW, L>(p, p.items, xcd_item(blockIdx.x, gridDim.x), lds, threadIdx.x);
 }
 
 // Work items of several kinds of one layer in one launch of 512-thread
@@ -863,7 +1060,7 @@ __global__ __launch_bounds__(64 * NW) void seg_pipe_kernel(SegParams p) {
 // waves end at once).  The bases are multiples of 8, so that every kind's
 // items map to XCDs as in its own kernel; blocks past a kind's item count end
 // at once.  The kinds run side by side instead of one launch after another.
-template <int D, bool FP16>
+template <int D, bool FP16, int L>
 __global__ __launch_bounds__(512) void seg_mix_kernel(MixParams mp) {
     using T = Tile<D>;
     __shared__ __attribute__((aligned(16))) u16 lds[TA_PIPE_STAGES * T::ELEMS];
@@ -871,15 +1068,15 @@ __global__ __launch_bounds__(512) void seg_mix_kernel(MixParams mp) {
     const int b = blockIdx.x, tid = threadIdx.x;
     if (b < mp.base[1]) {
         if (b >= mp.n[0]) return;
-        pipe_item_rows<D, FP16, 8>(mp.p, mp.items[0], xcd_item(b, mp.n[0]), lds, tid);
+        pipe_item_rows<D, FP16, 8, L>(mp.p, mp.items[0], xcd_item(b, mp.n[0]), lds, tid);
     } else if (b < mp.base[2]) {
         const int lb = b - mp.base[1];
         if (lb >= mp.n[1]) return;
-        tile_item<D, FP16, 1, 8, 3>(mp.p, mp.items[1], xcd_item(lb, mp.n[1]), lds, tid, 64);
+        tile_item<D, FP16, 1, 8, 3, L>(mp.p, mp.items[1], xcd_item(lb, mp.n[1]), lds, tid, 64);
     } else {
         const int wave = tid >> 6, it = 4 * (b - mp.base[2]) + wave;
         if (wave >= 4 || it >= mp.n[2]) return;
-        tile_item<D, FP16, 1, 1, 1, true>(mp.p, mp.items[2], it, lds + wave * T::ELEMS, tid & 63, 16);
+        tile_item<D, FP16, 1, 1, 1, L, true>(mp.p, mp.items[2], it, lds + wave * T::ELEMS, tid & 63, 16);
     }
 }
 
@@ -896,10 +1093,11 @@ __global__ __launch_bounds__(512) void seg_mix_kernel(MixParams mp) {
 //          units u = l + 64k (k < UPL) of the G*D/4 float4 units, unit u =
 //          (row u / (D/4), d = 4 (u % (D/4))).
 // After one barrier wave 1 merges the own partial and writes the output rows.
-template <int D, bool FP16, int UPL>
+template <int D, bool FP16, int UPL, int L>
 __global__ __launch_bounds__(128) void seg_tail_kernel(SegParams p) {
     using T = Tile<D>;
-    using M = TileMath<D, FP16, 1, 1>;
+    using M = TileMath<D, FP16, 1, 1, L>;
+    using C = TileCopy<D, 1, L>;
     constexpr int KS = M::KS, DB = M::DB;
     constexpr int PF = 32;          // units of one merge round
     constexpr int CH = PF / UPL;    // slots per merge round
@@ -921,9 +1119,10 @@ __global__ __launch_bounds__(128) void seg_tail_kernel(SegParams p) {
         const int kst = p.kstart[job];
         const int ntok = max(0, min(p.klen[job], p.tcap - kst));
         const int kend = kst + ntok;
-        const int tb0 = kst & ~7;
+        const int tb0 = tile_start<L>(kst);
         const int ntiles = ntok > 0 ? (kend - tb0 + T::TT - 1) / T::TT : 0;
-        if (ntiles > 0) M::copy(lds, p.kp, p.vp, h, p.tcap, tb0, kst, kend, 0, lane);
+        C kr;
+        if (ntiles > 0) kr.issue(lds, p, h, tb0, kst, kend, 0, lane);
         u32x4 qf[1][KS];
         {
             const int rr = row < G ? row : 0;  // rows past G repeat row 0 and are never stored
@@ -936,8 +1135,9 @@ __global__ __launch_bounds__(128) void seg_tail_kernel(SegParams p) {
         const LdsOfs of = T::offsets(row, g4);
         for (int it = 0; it < ntiles; ++it) {
             const int t0 = tb0 + it * T::TT;
-            if (it > 0) M::copy(lds, p.kp, p.vp, h, p.tcap, t0, kst, kend, 0, lane);
+            if (it > 0) kr.issue(lds, p, h, t0, kst, kend, 0, lane);
             __builtin_amdgcn_s_waitcnt(TA_VMCNT(0));
+            kr.finish(lds, 0, lane);
             acc.tile(lds, qf, of, max(0, kst - t0), min(T::TT, kend - t0), g4, p.scale_log2);
         }
         // the tile's reads fed the MFMAs above, so the stage is free for the partial
@@ -1021,59 +1221,66 @@ __global__ __launch_bounds__(128) void seg_tail_kernel(SegParams p) {
     }
 }
 
-template <int D, bool FP16>
+template <int D, bool FP16, int L>
 hipError_t launch_tail_merge(const SegParams &sp, hipStream_t stream) {
     // float4 units per lane: G*D/4 units over 64 lanes
     const int units = sp.group * (D / 4);
     if (units <= 64)
-        TA_LAUNCH((seg_tail_kernel<D, FP16, 1>), dim3(sp.n_items), dim3(128), stream, sp);
+        TA_LAUNCH((seg_tail_kernel<D, FP16, 1, L>), dim3(sp.n_items), dim3(128), stream, sp);
     else if (units <= 128)
-        TA_LAUNCH((seg_tail_kernel<D, FP16, 2>), dim3(sp.n_items), dim3(128), stream, sp);
+        TA_LAUNCH((seg_tail_kernel<D, FP16, 2, L>), dim3(sp.n_items), dim3(128), stream, sp);
     else if (units <= 256)
-        TA_LAUNCH((seg_tail_kernel<D, FP16, 4>), dim3(sp.n_items), dim3(128), stream, sp);
+        TA_LAUNCH((seg_tail_kernel<D, FP16, 4, L>), dim3(sp.n_items), dim3(128), stream, sp);
     else if (units <= 512)
-        TA_LAUNCH((seg_tail_kernel<D, FP16, 8>), dim3(sp.n_items), dim3(128), stream, sp);
+        TA_LAUNCH((seg_tail_kernel<D, FP16, 8, L>), dim3(sp.n_items), dim3(128), stream, sp);
     else
         return hipErrorNotSupported;
     return hipGetLastError();
 }
 
-template <int D, bool FP16>
+template <int D, bool FP16, int L>
 hipError_t launch_d(const SegParams &sp, int kind, hipStream_t stream) {
     switch (kind) {
-        case TA_SMALL:  // one wave per (job, head); one stage so that four fit on a CU
-            TA_LAUNCH((seg_tile_kernel<D, FP16, 1, 1, 1>), dim3(sp.n_items), dim3(64), stream, sp);
-            break;
         case TA_TAIL:  // as TA_SMALL, merging the request into out when out is given
-            if (sp.out) return launch_tail_merge<D, FP16>(sp, stream);
-            TA_LAUNCH((seg_tile_kernel<D, FP16, 1, 1, 1>), dim3(sp.n_items), dim3(64), stream, sp);
+            if (sp.out) return launch_tail_merge<D, FP16, L>(sp, stream);
+            [[fallthrough]];
+        case TA_SMALL:  // one wave per (job, head); one stage so that five fit on a CU
+            TA_LAUNCH((seg_tile_kernel<D, FP16, 1, 1, 1, L>), dim3(sp.n_items), dim3(64), stream, sp);
             break;
         case TA_LARGE64:
-            TA_LAUNCH((seg_tile_kernel<D, FP16, 1, 4, 3>), dim3(sp.n_items), dim3(256), stream, sp);
+            TA_LAUNCH((seg_tile_kernel<D, FP16, 1, 4, 3, L>), dim3(sp.n_items), dim3(256), stream, sp);
             break;
         case TA_LARGE128:
-            TA_LAUNCH((seg_tile_kernel<D, FP16, 2, 4, 3>), dim3(sp.n_items), dim3(256), stream, sp);
+            TA_LAUNCH((seg_tile_kernel<D, FP16, 2, 4, 3, L>), dim3(sp.n_items), dim3(256), stream, sp);
             break;
         case TA_LARGE256:
-            TA_LAUNCH((seg_pipe_kernel<D, FP16, 8>), dim3(sp.n_items), dim3(512), stream, sp);
+            TA_LAUNCH((seg_pipe_kernel<D, FP16, 8, L>), dim3(sp.n_items), dim3(512), stream, sp);
             break;
         default:
-            return hipErrorNotSupported;
+            return (hipError_t)TA_ERR_ARG;
     }
     return hipGetLastError();
 }
 
-template <int D, bool FP16>
+template <int D, bool FP16, int L>
 hipError_t launch_mix_d(const MixParams &mp, int blocks, hipStream_t stream) {
-    TA_LAUNCH((seg_mix_kernel<D, FP16>), dim3(blocks), dim3(512), stream, mp);
+    TA_LAUNCH((seg_mix_kernel<D, FP16, L>), dim3(blocks), dim3(512), stream, mp);
     return hipGetLastError();
 }
 
+#define TA_BY_SHAPE(FN, L, ...)                                                               \
+    switch (d) {                                                                              \
+        case 128: return fp16 ? FN<128, true, L>(__VA_ARGS__) : FN<128, false, L>(__VA_ARGS__); \
+        case 64: return fp16 ? FN<64, true, L>(__VA_ARGS__) : FN<64, false, L>(__VA_ARGS__);  \
+        case 32: return fp16 ? FN<32, true, L>(__VA_ARGS__) : FN<32, false, L>(__VA_ARGS__);  \
+        default: return hipErrorNotSupported;                                                 \
+    }
+
 }  // namespace
 
-hipError_t launch_tile_mix(const SegParams &sp, const int32_t *const items[3], const int n[3], int d, bool fp16,
-                           hipStream_t stream) {
-    if (sp.tcap % 8 != 0) return hipErrorNotSupported;
+template <>
+hipError_t launch_mix<TA_LAYOUT>(const SegParams &sp, const int32_t *const items[3], const int n[3], int d, bool fp16,
+                                 hipStream_t stream) {
     MixParams mp;
     mp.p = sp;
     int base = 0;
@@ -1086,22 +1293,12 @@ hipError_t launch_tile_mix(const SegParams &sp, const int32_t *const items[3], c
     }
     const int blocks = mp.base[2] + (mp.n[2] + 3) / 4;
     if (blocks <= 0) return hipSuccess;
-    switch (d) {
-        case 128: return fp16 ? launch_mix_d<128, true>(mp, blocks, stream) : launch_mix_d<128, false>(mp, blocks, stream);
-        case 64: return fp16 ? launch_mix_d<64, true>(mp, blocks, stream) : launch_mix_d<64, false>(mp, blocks, stream);
-        case 32: return fp16 ? launch_mix_d<32, true>(mp, blocks, stream) : launch_mix_d<32, false>(mp, blocks, stream);
-        default: return hipErrorNotSupported;
-    }
+    TA_BY_SHAPE(launch_mix_d, TA_LAYOUT, mp, blocks, stream)
 }
 
-hipError_t launch_tile(const SegParams &sp, int kind, int d, bool fp16, hipStream_t stream) {
-    if (sp.tcap % 8 != 0) return hipErrorNotSupported;
-    switch (d) {
-        case 128: return fp16 ? launch_d<128, true>(sp, kind, stream) : launch_d<128, false>(sp, kind, stream);
-        case 64: return fp16 ? launch_d<64, true>(sp, kind, stream) : launch_d<64, false>(sp, kind, stream);
-        case 32: return fp16 ? launch_d<32, true>(sp, kind, stream) : launch_d<32, false>(sp, kind, stream);
-        default: return hipErrorNotSupported;
-    }
+template <>
+hipError_t launch_kind<TA_LAYOUT>(const SegParams &sp, int kind, int d, bool fp16, hipStream_t stream) {
+    TA_BY_SHAPE(launch_d, TA_LAYOUT, sp, kind, stream)
 }
 
 }  // namespace ta

@@ -42,10 +42,6 @@ struct Ops<false> {  // bfloat16
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
                                                        __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
     }
-    __device__ static f32x4 mma_k16(u32x2 a, u32x2 b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a),
-                                                         __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
-    }
     __device__ static u32 pack(float lo, float hi) {
         bf16x2 v = {(__bf16)lo, (__bf16)hi};
         return __builtin_bit_cast(u32, v);
@@ -59,10 +55,6 @@ struct Ops<true> {  // float16
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
                                                       __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
     }
-    __device__ static f32x4 mma_k16(u32x2 a, u32x2 b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, a),
-                                                     __builtin_bit_cast(f16x4, b), c, 0, 0, 0);
-    }
     __device__ static u32 pack(float lo, float hi) {
         f16x2 v = {(_Float16)lo, (_Float16)hi};
         return __builtin_bit_cast(u32, v);
@@ -75,11 +67,6 @@ __device__ inline float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ inline float xor_max(float v) {
     v = fmaxf(v, __shfl_xor(v, 16));
     return fmaxf(v, __shfl_xor(v, 32));
-}
-
-__device__ inline float xor_sum(float v) {
-    v += __shfl_xor(v, 16);
-    return v + __shfl_xor(v, 32);
 }
 
 // Partial outputs.  Row `prow` (= slot * hq + query head) of a segment's
@@ -205,14 +192,33 @@ struct MixParams {
     int base[3];
 };
 
-// Large-job launcher of segment_tile.hip (gfx950 LDS-transpose kernels).
-// Returns hipErrorNotSupported when the shape is outside what it handles.
-hipError_t launch_tile(const SegParams &sp, int kind, int d, bool fp16, hipStream_t stream);
+// Where K and V lie (template argument of the segment kernels).
+//   KV_POOL:  pools kp [hk, d, tcap], vp [hk, tcap, d], tcap % 8 == 0: every
+//             8-token chunk of a K row is 16-byte aligned
+//   KV_ODD:   the same pools of any other capacity: K rows start anywhere
+//   KV_TOKEN: k, v [tokens, hk, d], as a prefill leaves them (kp, vp point at
+//             them, tcap is the number of tokens)
+enum Layout { KV_POOL, KV_ODD, KV_TOKEN };
 
+// Launchers of segment_tile.hip, which is compiled once per layout
+// (hipErrorNotSupported for a head dim they have no kernel for).
+// One segment launch of the work items of one kind; KV_ODD takes no attachments.
+template <int L>
+hipError_t launch_kind(const SegParams &sp, int kind, int d, bool fp16, hipStream_t stream);
 // One launch of the TA_LARGE256, TA_LARGE64 and TA_SMALL items items[k]
-// (n[k] of each) of one layer, side by side (hipErrorNotSupported unless the
-// pool capacity is a multiple of 8).
-hipError_t launch_tile_mix(const SegParams &sp, const int32_t *const items[3], const int n[3], int d, bool fp16,
-                           hipStream_t stream);
+// (n[k] of each) of one layer, side by side.
+template <int L>
+hipError_t launch_mix(const SegParams &sp, const int32_t *const items[3], const int n[3], int d, bool fp16,
+                      hipStream_t stream);
+#define TA_EXTERN_LAYOUT(L)                                                                                          \
+    template <>                                                                                                      \
+    hipError_t launch_kind<L>(const SegParams &sp, int kind, int d, bool fp16, hipStream_t stream);                  \
+    template <>                                                                                                      \
+    hipError_t launch_mix<L>(const SegParams &sp, const int32_t *const items[3], const int n[3], int d, bool fp16,   \
+                             hipStream_t stream);
+TA_EXTERN_LAYOUT(KV_POOL)
+TA_EXTERN_LAYOUT(KV_ODD)
+TA_EXTERN_LAYOUT(KV_TOKEN)
+#undef TA_EXTERN_LAYOUT
 
 }  // namespace ta

@@ -7,28 +7,11 @@
 //   _merge (kernels.py:58-83): per (request, query head) log-sum-exp merge of
 //     the request's partial outputs, cast to the input dtype.
 //
-// Design (MI355X-first, not a translation of the Triton tiling):
-//   * K/V of a job are streamed from HBM once per work item in 64-token tiles
-//     by all 256 threads (coalesced 16-byte loads), transposed 8x8 in
-//     registers and written to LDS as Kt[token][d] and Vt[d][token], the
-//     operand orders the MFMA needs.  The next tile's global loads are issued
-//     before the current tile is computed.
-//   * QK^T is computed transposed, S^T = K Q^T, with
-//     v_mfma_f32_16x16x32_{bf16,f16}: the C layout then gives each lane four
-//     consecutive tokens of one query row, which is exactly the B operand of
-//     the PV product O^T = V^T P^T -- P never leaves registers.
-//   * Small jobs (<= 16 query rows, e.g. one request x 4 GQA heads): the four
-//     waves split every tile's tokens (16 each), keep private (m, z, O) and
-//     combine once through LDS at the end.  PV uses 16x16x16 MFMA.
-//   * Large jobs: the four waves split the query rows (NB blocks of 16 rows per
-//     wave) and share every staged K/V tile; each K/V fragment read from LDS
-//     feeds NB MFMAs.  Work items are (job, row tile, head) and are remapped
-//     so that tiles of the same (job, head) land on the same XCD back to back
-//     and share its L2.
-//   * Softmax runs in base 2 with log2(e)/sqrt(D) folded into one FMA.
+// This file holds the merge kernel, the read-ceiling stream and the C entry points; the
+// segment kernels are in segment_tile.hip.
 //   * Partial rows are stored as fp16 scaled by a power of two per row (the
 //     exponent sits next to the log-sum-exp); the merge reads them with
-//     8-byte loads, one thread per four head-dim elements, and folds the
+//     16-byte loads, one thread per eight head-dim elements, and folds the
 //     scale into each slot's weight.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -41,395 +24,6 @@
 namespace {
 
 using namespace ta;
-
-
-// ------------------------------------------------------- tile staging (LDS)
-// One TTILE-token tile of one KV head: Kt[TTILE][D] (+pad) and Vt[D][TTILE]
-// (+pad), built from 8x8 element blocks that NTHR threads load with 16-byte
-// global loads, transpose in registers and store with 16-byte LDS writes.
-template <int D, int TTILE, int NTHR>
-struct Stage {
-    // Row strides (elements).  Kt rows are read 16 B per lane, 8 lanes per LDS
-    // cycle: D + 8 shifts consecutive rows by 4 banks.  Vt rows are read 8 B per
-    // lane, 16 lanes per cycle: TTILE + 4 shifts consecutive rows by 2 banks, so
-    // 16 rows cover all 32 banks once.
-    static constexpr int KS = D + 8;
-    static constexpr int VS = TTILE + 4;
-    static constexpr int KELEMS = TTILE * KS;
-    static constexpr int ELEMS = KELEMS + D * VS;
-    static constexpr int DG = D / 8;
-    static constexpr int TG = TTILE / 8;
-    static constexpr int KBLK = DG * TG;  // 8x8 blocks per operand
-    static constexpr int NBLK = 2 * KBLK;
-    static constexpr int BPT = (NBLK + NTHR - 1) / NTHR;  // blocks per thread
-
-    u32x4 r[BPT][8];
-
-    __device__ static u32x4 load_tail(const u16 *p, int valid) {
-        u32 w[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const u32 lo = (2 * k < valid) ? (u32)p[2 * k] : 0u;
-            const u32 hi = (2 * k + 1 < valid) ? (u32)p[2 * k + 1] : 0u;
-            w[k] = lo | (hi << 16);
-        }
-        return u32x4{w[0], w[1], w[2], w[3]};
-    }
-
-    // Global -> registers.  Tokens [t0, t0 + nvalid) are read; the rest of the
-    // tile is zero (zero V keeps masked columns finite in PV).
-    __device__ void load(const u16 *__restrict__ kp, const u16 *__restrict__ vp, int h, int tcap, int t0,
-                         int nvalid, bool kaligned, int tid) {
-        if (kaligned && nvalid >= TTILE) {
-            // full, 16-byte aligned tile: unconditional vector loads (wave-uniform branch)
-#pragma unroll
-            for (int j = 0; j < BPT; ++j) {
-                const int b = tid + j * NTHR;
-                if (b < KBLK) {
-                    const int dg = b % DG, tg = b / DG;
-                    const u16 *base = kp + ((size_t)(h * D + 8 * dg) * tcap + t0 + 8 * tg);
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) r[j][i] = *(const u32x4 *)(base + (size_t)i * tcap);
-                } else if (b < NBLK) {
-                    const int u = b - KBLK;
-                    const int tg = u % TG, dg = u / TG;
-                    const u16 *base = vp + ((size_t)(h * tcap + t0 + 8 * tg) * D + 8 * dg);
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) r[j][i] = *(const u32x4 *)(base + i * D);
-                }
-            }
-            return;
-        }
-#pragma unroll
-        for (int j = 0; j < BPT; ++j) {
-            const int b = tid + j * NTHR;
-            if (b < KBLK) {
-                const int dg = b % DG, tg = b / DG;
-                const u16 *base = kp + ((size_t)(h * D + 8 * dg) * tcap + t0 + 8 * tg);
-                const int valid = nvalid - 8 * tg;
-                if (kaligned && valid >= 8) {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) r[j][i] = *(const u32x4 *)(base + (size_t)i * tcap);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) r[j][i] = load_tail(base + (size_t)i * tcap, valid);
-                }
-            } else if (b < NBLK) {
-                const int u = b - KBLK;
-                const int tg = u % TG, dg = u / TG;
-                const u16 *base = vp + ((size_t)(h * tcap + t0 + 8 * tg) * D + 8 * dg);
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    r[j][i] = (8 * tg + i < nvalid) ? *(const u32x4 *)(base + (size_t)i * D) : u32x4{0, 0, 0, 0};
-            }
-        }
-    }
-
-    // 8x8 transpose of 16-bit elements: o[c] = column c of the rows in in[].
-    __device__ static void transpose(const u32x4 (&in)[8], u32x4 (&o)[8]) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            u32 w[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const u32 a = in[2 * k][c >> 1], b = in[2 * k + 1][c >> 1];
-                w[k] = (c & 1) ? ((a >> 16) | (b & 0xffff0000u)) : ((a & 0xffffu) | (b << 16));
-            }
-            o[c] = u32x4{w[0], w[1], w[2], w[3]};
-        }
-    }
-
-    // Registers -> LDS in MFMA operand order.
-    __device__ void store(u16 *lds, int tid) const {
-#pragma unroll
-        for (int j = 0; j < BPT; ++j) {
-            const int b = tid + j * NTHR;
-            if (b >= NBLK) continue;
-            u32x4 o[8];
-            transpose(r[j], o);
-            if (b < KBLK) {
-                const int dg = b % DG, tg = b / DG;
-#pragma unroll
-                for (int c = 0; c < 8; ++c) *(u32x4 *)(lds + (8 * tg + c) * KS + 8 * dg) = o[c];
-            } else {
-                const int u = b - KBLK;
-                const int tg = u % TG, dg = u / TG;
-#pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    u16 *dst = lds + KELEMS + (8 * dg + c) * VS + 8 * tg;  // 8-byte aligned
-                    *(u32x2 *)dst = u32x2{o[c][0], o[c][1]};
-                    *(u32x2 *)(dst + 4) = u32x2{o[c][2], o[c][3]};
-                }
-            }
-        }
-    }
-};
-
-// Query fragment of one 16-row block: lane (row, g4) holds d = 32*ks + 8*g4 .. +7.
-template <int D>
-__device__ inline void load_q(const SegParams &p, int job, int h, int row, int nrows, int g4,
-                              u32x4 (&qf)[D / 32]) {
-    if (row < nrows) {
-        const int lr = row / p.group, gg = row - lr * p.group;
-        const int rq = p.qids[(size_t)job * p.maxr + lr];
-        const u16 *src = p.q + ((size_t)rq * p.hq + h * p.group + gg) * D + 8 * g4;
-#pragma unroll
-        for (int ks = 0; ks < D / 32; ++ks) qf[ks] = *(const u32x4 *)(src + 32 * ks);
-    } else {
-#pragma unroll
-        for (int ks = 0; ks < D / 32; ++ks) qf[ks] = u32x4{0, 0, 0, 0};
-    }
-}
-
-// Online-softmax state of NB 16-row blocks held by one wave.  Lane (row, g4)
-// keeps the shared (stale) maximum m of its row, a partial denominator z over
-// its own columns and O^T[d = 16*db + 4*g4 + i][row] in o[nb][db][i].
-template <int D, int NB>
-struct RowState {
-    float m[NB], z[NB];
-    f32x4 o[NB][D / 16];
-
-    __device__ void reset() {
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            m[nb] = NEG_INF;
-            z[nb] = 0.f;
-#pragma unroll
-            for (int db = 0; db < D / 16; ++db) o[nb][db] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-    }
-};
-
-// S^T = K Q^T for one 32-token step: s[nb][b][i] is the score of token
-// 16*b + 4*g4 + i (relative to kt) against row 16*nb + row.
-template <int D, bool FP16, int NB, int KS>
-__device__ inline void qk_step(const u16 *kt, int row, int g4, const u32x4 (&qf)[NB][D / 32], f32x4 (&s)[NB][2]) {
-    using O = Ops<FP16>;
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) s[nb][0] = s[nb][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-#pragma unroll
-        for (int ks = 0; ks < D / 32; ++ks) {
-            const u32x4 a = *(const u32x4 *)(kt + (16 * b + row) * KS + 32 * ks + 8 * g4);
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) s[nb][b] = O::mma_k32(a, qf[nb][ks], s[nb][b]);
-        }
-    }
-}
-
-// Softmax update and O^T += V^T P^T for one 32-token step with nvs valid
-// tokens.  PV k-slot j of lane group g4 is token 4*g4 + j (j < 4) or
-// 16 + 4*g4 + j - 4 (j >= 4), which is where the QK output left P.
-template <int D, bool FP16, int NB, int VS>
-__device__ inline void pv_step(const u16 *vt, int row, int g4, f32x4 (&s)[NB][2], int nvs, float c,
-                               RowState<D, NB> &st) {
-    using O = Ops<FP16>;
-    u32x4 vf[D / 16];
-#pragma unroll
-    for (int db = 0; db < D / 16; ++db) {
-        const u16 *vr = vt + (16 * db + row) * VS + 4 * g4;
-        const u32x2 lo = *(const u32x2 *)vr;
-        const u32x2 hi = *(const u32x2 *)(vr + 16);
-        vf[db] = u32x4{lo[0], lo[1], hi[0], hi[1]};
-    }
-    const bool full = nvs >= 32;
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        float x[8];
-        float lm = NEG_INF;
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float v = s[nb][b][i];
-                if (!full && 16 * b + 4 * g4 + i >= nvs) v = NEG_INF;
-                x[4 * b + i] = v;
-                lm = fmaxf(lm, v);
-            }
-        const bool need = lm * c > st.m[nb] + TAU;
-        if (__builtin_amdgcn_ballot_w64(need)) {  // wave-uniform, rare after the first step
-            const float mn = fmaxf(st.m[nb], xor_max(lm) * c);
-            const float alpha = fast_exp2(st.m[nb] - mn);
-            st.z[nb] *= alpha;
-#pragma unroll
-            for (int db = 0; db < D / 16; ++db) st.o[nb][db] *= alpha;
-            st.m[nb] = mn;
-        }
-        float pr[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) pr[i] = fast_exp2(__builtin_fmaf(x[i], c, -st.m[nb]));
-        st.z[nb] += ((pr[0] + pr[1]) + (pr[2] + pr[3])) + ((pr[4] + pr[5]) + (pr[6] + pr[7]));
-        const u32x4 pb = {O::pack(pr[0], pr[1]), O::pack(pr[2], pr[3]), O::pack(pr[4], pr[5]),
-                          O::pack(pr[6], pr[7])};
-#pragma unroll
-        for (int db = 0; db < D / 16; ++db) st.o[nb][db] = O::mma_k32(vf[db], pb, st.o[nb][db]);
-    }
-}
-
-// Normalise and store the partial rows of NB 16-row blocks (rows >= nrows skipped).
-template <int D, int NB>
-__device__ inline void store_rows(const SegParams &p, RowState<D, NB> &st, int job, int h, int wrow0, int nrows,
-                                  int row, int g4) {
-    const int rb = p.rowbase[job];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        const float zr = xor_sum(st.z[nb]);
-        const int grow = wrow0 + 16 * nb + row;
-        if (grow >= nrows) continue;
-        const int lr = grow / p.group, gg = grow - lr * p.group;
-        const size_t prow = (size_t)(rb + lr) * p.hq + h * p.group + gg;
-        store_partial<D / 16>(p.part, p.lse, prow, st.o[nb], st.m[nb], zr, g4);
-    }
-}
-
-// --------------------------------------------------------- small segments
-// Jobs with at most 16 query rows (e.g. one request's private tail).  One
-// wave per workgroup walks a strided list of (job, KV head) items; 32-token
-// tiles go through wave-private LDS and the next tile -- of the same item or
-// of the next one -- is already in flight while the current one is computed.
-constexpr int SMALL_TT = 32;
-constexpr int SMALL_NT = 64;
-
-template <int D, bool FP16>
-__global__ __launch_bounds__(SMALL_NT) void seg_small_kernel(SegParams p) {
-    using S = Stage<D, SMALL_TT, SMALL_NT>;
-    __shared__ __attribute__((aligned(16))) u16 lds[S::ELEMS];
-    const int lane = threadIdx.x;
-    const int row = lane & 15, g4 = lane >> 4;
-    const int total = p.n_items;
-    const float c = p.scale_log2;
-    const int stride = gridDim.x;
-
-    struct Item {
-        int job, h, kst, ntok, ntiles;
-        bool kal;
-    };
-    auto decode = [&](int idx) {
-        Item it;
-        it.job = p.items[3 * idx];
-        it.h = p.items[3 * idx + 2];
-        it.kst = p.kstart[it.job];
-        it.ntok = max(0, min(p.klen[it.job], p.tcap - it.kst));
-        it.ntiles = (it.ntok + SMALL_TT - 1) / SMALL_TT;
-        it.kal = ((p.tcap | it.kst) & 7) == 0;
-        return it;
-    };
-
-    S st;
-    // prefetch cursor: (pidx, ptile) is the tile whose loads sit in st.r
-    int pidx = blockIdx.x, ptile = 0;
-    Item pit;
-    while (pidx < total) {
-        pit = decode(pidx);
-        if (pit.ntiles > 0) break;
-        pidx += stride;
-    }
-    if (pidx < total)
-        st.load(p.kp, p.vp, pit.h, p.tcap, pit.kst, min(pit.ntok, SMALL_TT), pit.kal, lane);
-
-    RowState<D, 1> rs;
-    u32x4 qf[1][D / 32];
-    for (int idx = blockIdx.x; idx < total; idx += stride) {
-        const Item it = decode(idx);
-        const int nrows = min(p.qlen[it.job] * p.group, 16);
-        load_q<D>(p, it.job, it.h, row, nrows, g4, qf[0]);
-        rs.reset();
-        for (int t = 0; t < it.ntiles; ++t) {
-            __syncthreads();
-            st.store(lds, lane);
-            __syncthreads();
-            // advance the prefetch cursor and issue the next tile's loads
-            if (++ptile >= pit.ntiles) {
-                ptile = 0;
-                for (pidx += stride; pidx < total; pidx += stride) {
-                    pit = decode(pidx);
-                    if (pit.ntiles > 0) break;
-                }
-            }
-            if (pidx < total) {
-                const int t0 = ptile * SMALL_TT;
-                st.load(p.kp, p.vp, pit.h, p.tcap, pit.kst + t0, min(pit.ntok - t0, SMALL_TT), pit.kal, lane);
-            }
-            f32x4 s[1][2];
-            qk_step<D, FP16, 1, S::KS>(lds, row, g4, qf, s);
-            pv_step<D, FP16, 1, S::VS>(lds + S::KELEMS, row, g4, s, it.ntok - t * SMALL_TT, c, rs);
-        }
-        store_rows<D, 1>(p, rs, it.job, it.h, 0, nrows, row, g4);
-    }
-}
-
-// --------------------------------------------------------- large segments
-// One workgroup (NW waves) per (job, row tile of 16*NB*NW rows, KV head);
-// wave w owns rows [16*NB*w, 16*NB*(w+1)) of the tile.  TT-token K/V tiles
-// are double-buffered in LDS (one barrier per tile) and every K/V fragment
-// read from LDS feeds NB MFMAs.  Within a tile the next 32-token step's QK is
-// issued before the current step's softmax so the matrix cores and the VALU
-// have independent work; with 32 rows per wave everything stays in VGPRs and
-// two waves share each SIMD.
-template <int D, bool FP16, int NB, int NW, int TT>
-__global__ __launch_bounds__(64 * NW) void seg_large_kernel(SegParams p) {
-    constexpr int NTHR = 64 * NW;
-    constexpr int STEPS = TT / 32;
-    using S = Stage<D, TT, NTHR>;
-    __shared__ __attribute__((aligned(16))) u16 lds[2 * S::ELEMS];
-
-    // Linear block L runs on XCD L % 8; give every XCD a contiguous range of
-    // items so neighbouring row tiles of one (job, head) share an L2.
-    const int total = gridDim.x;
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int q8 = total >> 3, rm = total & 7;
-    const int v = xcd * q8 + min(xcd, rm) + slot;
-    const int job = p.items[3 * v], row0 = p.items[3 * v + 1], h = p.items[3 * v + 2];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int row = lane & 15, g4 = lane >> 4;
-    const int kst = p.kstart[job];
-    const int ntok = max(0, min(p.klen[job], p.tcap - kst));
-    const int nrows = p.qlen[job] * p.group;
-    const int wrow0 = row0 + 16 * NB * wave;  // first row of this wave
-    const bool active = wrow0 < nrows;
-    const bool kal = ((p.tcap | kst) & 7) == 0;
-    const float c = p.scale_log2;
-
-    u32x4 qf[NB][D / 32];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) load_q<D>(p, job, h, wrow0 + 16 * nb + row, nrows, g4, qf[nb]);
-    RowState<D, NB> rs;
-    rs.reset();
-
-    const int ntiles = (ntok + TT - 1) / TT;
-    S st;
-    if (ntiles > 0) {
-        st.load(p.kp, p.vp, h, p.tcap, kst, min(ntok, TT), kal, tid);
-        st.store(lds, tid);
-    }
-    if (ntiles > 1) st.load(p.kp, p.vp, h, p.tcap, kst + TT, min(ntok - TT, TT), kal, tid);
-    __syncthreads();
-    for (int it = 0; it < ntiles; ++it) {
-        const u16 *cur = lds + (it & 1) * S::ELEMS;
-        const int nv = ntok - it * TT;
-        if (active) {
-            f32x4 sc[2][NB][2];
-            qk_step<D, FP16, NB, S::KS>(cur, row, g4, qf, sc[0]);
-#pragma unroll
-            for (int k = 0; k < STEPS; ++k) {
-                const int base = 32 * k;
-                if (base >= nv) break;
-                if (k + 1 < STEPS && base + 32 < nv)
-                    qk_step<D, FP16, NB, S::KS>(cur + (base + 32) * S::KS, row, g4, qf, sc[(k + 1) & 1]);
-                pv_step<D, FP16, NB, S::VS>(cur + S::KELEMS + base, row, g4, sc[k & 1], nv - base, c, rs);
-            }
-        }
-        if (it + 1 < ntiles) st.store(lds + ((it + 1) & 1) * S::ELEMS, tid);
-        __syncthreads();
-        if (it + 2 < ntiles) {
-            const int t0 = (it + 2) * TT;
-            st.load(p.kp, p.vp, h, p.tcap, kst + t0, min(ntok - t0, TT), kal, tid);
-        }
-    }
-    if (active) store_rows<D, NB>(p, rs, job, h, wrow0, nrows, row, g4);
-}
 
 // ------------------------------------------------------------------ merge
 // One workgroup of NT threads per (request, group of MH query heads);
@@ -587,40 +181,8 @@ __global__ __launch_bounds__(READ_NT) void read_stream_kernel(const u32x4 *__res
 }
 
 // ------------------------------------------------------------------ launch
-// resident one-wave workgroups on 256 CUs (8 per CU by LDS at d = 128)
-constexpr int SMALL_MAX_BLOCKS = 2048;
-
-template <int D, bool FP16>
-hipError_t launch_segment(const SegParams &sp, int kind, hipStream_t stream) {
-    if (sp.n_items <= 0) return hipSuccess;
-#ifndef TA_LEGACY_LARGE
-    {
-        // LDS-transpose kernels (segment_tile.hip) whenever the pool layout allows them
-        const hipError_t e = launch_tile(sp, kind, D, FP16, stream);
-        if (e != hipErrorNotSupported) return e;
-    }
-#endif
-    switch (kind) {
-        case TA_SMALL:
-        case TA_TAIL: {  // the fused merge exists only on the LDS-transpose path
-            const int blocks = sp.n_items < SMALL_MAX_BLOCKS ? sp.n_items : SMALL_MAX_BLOCKS;
-            TA_LAUNCH((seg_small_kernel<D, FP16>), dim3(blocks), dim3(SMALL_NT), stream, sp);
-            break;
-        }
-        case TA_LARGE64:
-            TA_LAUNCH((seg_large_kernel<D, FP16, 1, 4, 64>), dim3(sp.n_items), dim3(256), stream, sp);
-            break;
-        case TA_LARGE128:
-            TA_LAUNCH((seg_large_kernel<D, FP16, 2, 4, 64>), dim3(sp.n_items), dim3(256), stream, sp);
-            break;
-        case TA_LARGE256:
-            TA_LAUNCH((seg_large_kernel<D, FP16, 2, 8, 128>), dim3(sp.n_items), dim3(512), stream, sp);
-            break;
-        default:
-            return (hipError_t)TA_ERR_ARG;
-    }
-    return hipGetLastError();
-}
+// The layout of pools of `tcap` tokens.
+int pool_layout(int32_t tcap) { return tcap % 8 == 0 ? KV_POOL : KV_ODD; }
 
 // nreq requests: reqs[0 .. nreq) when reqs is given, else 0 .. nreq-1
 template <int D, bool FP16>
@@ -703,7 +265,7 @@ int segment_launch(const void *q, const void *kp, const void *vp, const int32_t 
                    int32_t n_items, int32_t kind, void *part, float *lse, int32_t nreq, int32_t hq, int32_t hk,
                    int32_t d, int32_t tcap, int32_t maxr, int32_t dtype, const int32_t *slots,
                    const int32_t *counts, void *out, int32_t maxs, const int32_t *xtail, int32_t xtail_stride,
-                   const int32_t *qbase, void *stream) {
+                   const int32_t *qbase, int layout, void *stream) {
     if (int e = check_common(hq, hk, d, dtype)) return e;
     if (n_items < 0 || nreq <= 0 || tcap <= 0 || maxr <= 0 || kind < TA_SMALL || kind > TA_TAIL) return TA_ERR_ARG;
     if (n_items == 0) return 0;
@@ -711,25 +273,18 @@ int segment_launch(const void *q, const void *kp, const void *vp, const int32_t 
         return TA_ERR_ARG;
     if (!aligned16(q) || !aligned16(kp) || !aligned16(vp) || !aligned16(part)) return TA_ERR_ALIGN;
     if (out) {
-#ifdef TA_LEGACY_LARGE
-        return TA_ERR_ARG;  // the register-staged kernels have no fused merge
-#endif
-        if (kind != TA_TAIL || tcap % 8 != 0 || !slots || !counts || maxs <= 0) return TA_ERR_ARG;
+        if (kind != TA_TAIL || !slots || !counts || maxs <= 0) return TA_ERR_ARG;
         if (!aligned16(out)) return TA_ERR_ALIGN;
     }
-    if (xtail) {
-#ifdef TA_LEGACY_LARGE
-        return TA_ERR_ARG;  // the register-staged kernels take no attached segments
-#endif
-        if (kind != TA_LARGE256 || tcap % 8 != 0 || xtail_stride != TA_XTAIL_STRIDE) return TA_ERR_ARG;
-    }
+    if (xtail && (kind != TA_LARGE256 || layout == KV_ODD || xtail_stride != TA_XTAIL_STRIDE)) return TA_ERR_ARG;
     SegParams sp;
     fill_params(sp, q, kp, vp, qids, kstart, qlen, klen, rowbase, items, n_items, part, lse, hq, hk, d, tcap, maxr,
                 slots, counts, out, maxs, xtail, xtail_stride, qbase);
     const hipStream_t st = static_cast<hipStream_t>(stream);
-#define TA_SEG(D, F) launch_segment<D, F>(sp, kind, st)
-    return (int)TA_DISPATCH(d, dtype == TA_FP16, TA_SEG);
-#undef TA_SEG
+    const bool fp16 = dtype == TA_FP16;
+    return (int)(layout == KV_POOL  ? ta::launch_kind<KV_POOL>(sp, kind, d, fp16, st)
+                 : layout == KV_ODD ? ta::launch_kind<KV_ODD>(sp, kind, d, fp16, st)
+                                    : ta::launch_kind<KV_TOKEN>(sp, kind, d, fp16, st));
 }
 
 // The launch arguments every segment kernel shares.
@@ -766,12 +321,13 @@ void fill_params(SegParams &sp, const void *q, const void *kp, const void *vp, c
 }
 
 int plan_segment(const void *q, const void *kp, const void *vp, int32_t tcap, const ta_plan *plan, int kind,
-                 void *out, void *stream) {
+                 void *out, int layout, void *stream) {
     const bool xt = kind == TA_LARGE256 && plan->xtail;
     return segment_launch(q, kp, vp, plan->qids, plan->kstart, plan->qlen, plan->klen, plan->rowbase,
                           plan->items[kind], plan->n_items[kind], kind, plan->part, plan->lse, plan->nreq, plan->hq,
                           plan->hk, plan->d, tcap, plan->maxr, plan->dtype, plan->slots, plan->counts, out,
-                          plan->maxs, xt ? plan->xtail : nullptr, xt ? plan->xtail_stride : 0, plan->qbase, stream);
+                          plan->maxs, xt ? plan->xtail : nullptr, xt ? plan->xtail_stride : 0, plan->qbase, layout,
+                          stream);
 }
 
 // The merge of requests reqs[0 .. n) (reqs == NULL: 0 .. n-1) of a prepared
@@ -808,7 +364,7 @@ int ta_segment(const void *q, const void *kp, const void *vp, const int32_t *qid
                int32_t n_items, int32_t kind, void *part, float *lse, int32_t nreq, int32_t hq, int32_t hk,
                int32_t d, int32_t tcap, int32_t maxr, int32_t dtype, void *stream) {
     return segment_launch(q, kp, vp, qids, kstart, qlen, klen, rowbase, items, n_items, kind, part, lse, nreq, hq,
-                          hk, d, tcap, maxr, dtype, nullptr, nullptr, nullptr, 0, nullptr, 0, nullptr, stream);
+                          hk, d, tcap, maxr, dtype, nullptr, nullptr, nullptr, 0, nullptr, 0, nullptr, pool_layout(tcap), stream);
 }
 
 int ta_merge(const void *part, const float *lse, const int32_t *slots, const int32_t *counts, void *out,
@@ -826,13 +382,13 @@ int ta_merge(const void *part, const float *lse, const int32_t *slots, const int
 int ta_segment_plan(const void *q, const void *kp, const void *vp, int32_t tcap, const ta_plan *plan, int32_t kind,
                     void *stream) {
     if (!plan || kind < TA_SMALL || kind > TA_TAIL) return TA_ERR_ARG;
-    return plan_segment(q, kp, vp, tcap, plan, kind, nullptr, stream);
+    return plan_segment(q, kp, vp, tcap, plan, kind, nullptr, pool_layout(tcap), stream);
 }
 
 int ta_tail_merge(const void *q, const void *kp, const void *vp, int32_t tcap, const ta_plan *plan, void *out,
                   void *stream) {
     if (!plan || !out || tcap % 8 != 0) return TA_ERR_ARG;
-    return plan_segment(q, kp, vp, tcap, plan, TA_TAIL, out, stream);
+    return plan_segment(q, kp, vp, tcap, plan, TA_TAIL, out, KV_POOL, stream);
 }
 
 }  // extern "C"
@@ -848,12 +404,10 @@ namespace {
 // The TA_LARGE256, TA_LARGE64 and TA_SMALL items of a plan in one launch
 // (seg_mix_kernel), when at least two of those kinds have items and
 // TA_LARGE128 has none.  Returns -1 when the plan does not qualify.
-int mix_launch(const void *q, const void *kp, const void *vp, int32_t tcap, const ta_plan *plan, void *stream) {
-#ifdef TA_LEGACY_LARGE
-    return -1;
-#endif
+int mix_launch(const void *q, const void *kp, const void *vp, int32_t tcap, const ta_plan *plan, int layout,
+               void *stream) {
     const int n[3] = {plan->n_items[TA_LARGE256], plan->n_items[TA_LARGE64], plan->n_items[TA_SMALL]};
-    if ((n[0] > 0) + (n[1] > 0) + (n[2] > 0) < 2 || plan->n_items[TA_LARGE128] > 0 || tcap % 8 != 0) return -1;
+    if ((n[0] > 0) + (n[1] > 0) + (n[2] > 0) < 2 || plan->n_items[TA_LARGE128] > 0) return -1;
     if (n[0] < 0 || n[1] < 0 || n[2] < 0) return TA_ERR_ARG;
     if (int e = check_common(plan->hq, plan->hk, plan->d, plan->dtype)) return e;
     if (plan->nreq <= 0 || tcap <= 0 || plan->maxr <= 0) return TA_ERR_ARG;
@@ -864,46 +418,36 @@ int mix_launch(const void *q, const void *kp, const void *vp, int32_t tcap, cons
         if (plan->n_items[k] > 0 && !plan->items[k]) return TA_ERR_ARG;
     if (!aligned16(q) || !aligned16(kp) || !aligned16(vp) || !aligned16(plan->part)) return TA_ERR_ALIGN;
     const bool xt = n[0] > 0 && plan->xtail;
-    if (xt && plan->xtail_stride != TA_XTAIL_STRIDE) return TA_ERR_ARG;
+    if (xt && (plan->xtail_stride != TA_XTAIL_STRIDE || layout == KV_ODD)) return TA_ERR_ARG;
     SegParams sp;
     fill_params(sp, q, kp, vp, plan->qids, plan->kstart, plan->qlen, plan->klen, plan->rowbase, nullptr, 0,
                 plan->part, plan->lse, plan->hq, plan->hk, plan->d, tcap, plan->maxr, plan->slots, plan->counts,
                 nullptr, plan->maxs, xt ? plan->xtail : nullptr, xt ? plan->xtail_stride : 0, plan->qbase);
     const int32_t *const items[3] = {plan->items[TA_LARGE256], plan->items[TA_LARGE64], plan->items[TA_SMALL]};
-    if (hipError_t e = ta::launch_tile_mix(sp, items, n, plan->d, plan->dtype == TA_FP16,
-                                           static_cast<hipStream_t>(stream)))
-        return (int)e;
-    return 0;
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    const bool fp16 = plan->dtype == TA_FP16;
+    return (int)(layout == KV_POOL  ? ta::launch_mix<KV_POOL>(sp, items, n, plan->d, fp16, st)
+                 : layout == KV_ODD ? ta::launch_mix<KV_ODD>(sp, items, n, plan->d, fp16, st)
+                                    : ta::launch_mix<KV_TOKEN>(sp, items, n, plan->d, fp16, st));
 }
 
 int attention_layer(const void *q, const void *kp, const void *vp, int32_t tcap, const ta_plan *plan, void *out,
-                    void *stream) {
+                    int layout, void *stream) {
     if (!plan || !out) return TA_ERR_ARG;
-#ifdef TA_LEGACY_LARGE
-    const bool fused = false;
-#else
-    const bool fused = tcap % 8 == 0;  // the LDS-transpose kernels carry the fused merge
-#endif
-    // attached segments exist only on the LDS-transpose path (pools with tcap % 8 == 0)
-    if (plan->xtail && !fused) return TA_ERR_ARG;
+    // attachments are kept to layouts whose K the LDS DMA takes
+    if (plan->xtail && layout == KV_ODD) return TA_ERR_ARG;
     // the partials every merge reads come first: large jobs, then small jobs,
     // in one launch when the kinds allow it
-    const int mixed = mix_launch(q, kp, vp, tcap, plan, stream);
+    const int mixed = mix_launch(q, kp, vp, tcap, plan, layout, stream);
     if (mixed > 0) return mixed;
     static const int order[] = {TA_LARGE256, TA_LARGE128, TA_LARGE64, TA_SMALL};
     for (int kind : order) {
         if (mixed == 0 && kind != TA_LARGE128) continue;
         if (plan->n_items[kind] == 0) continue;
-        if (int e = plan_segment(q, kp, vp, tcap, plan, kind, nullptr, stream)) return e;
-    }
-    if (!fused) {
-        if (plan->n_items[TA_TAIL] > 0)
-            if (int e = plan_segment(q, kp, vp, tcap, plan, TA_TAIL, nullptr, stream)) return e;
-        return ta_merge(plan->part, plan->lse, plan->slots, plan->counts, out, plan->nreq, plan->hq, plan->d,
-                        plan->maxs, plan->dtype, stream);
+        if (int e = plan_segment(q, kp, vp, tcap, plan, kind, nullptr, layout, stream)) return e;
     }
     if (plan->n_items[TA_TAIL] > 0)
-        if (int e = plan_segment(q, kp, vp, tcap, plan, TA_TAIL, out, stream)) return e;
+        if (int e = plan_segment(q, kp, vp, tcap, plan, TA_TAIL, out, layout, stream)) return e;
     if (plan->n_rest <= 0) return 0;
     // rest == NULL with n_rest == nreq: every request
     if (!plan->rest && plan->n_rest != plan->nreq) return TA_ERR_ARG;
@@ -937,7 +481,12 @@ extern "C" {
 
 int ta_attention_matrix(const void *q, const void *kp, const void *vp, int32_t tcap, const ta_plan *plan,
                         void *out, void *stream) {
-    return attention_layer(q, kp, vp, tcap, plan, out, stream);
+    return attention_layer(q, kp, vp, tcap, plan, out, pool_layout(tcap), stream);
+}
+
+int ta_attention_tokens(const void *q, const void *k, const void *v, int32_t tokens, const ta_plan *plan, void *out,
+                        void *stream) {
+    return attention_layer(q, k, v, tokens, plan, out, KV_TOKEN, stream);
 }
 
 int ta_attention_matrix_noalloc(const void *q, const void *kp, const void *vp, int32_t tcap, const ta_plan *plan,
@@ -962,7 +511,7 @@ int ta_attention_matrix_noalloc(const void *q, const void *kp, const void *vp, i
     ta_plan local = *plan;
     local.part = base;
     local.lse = reinterpret_cast<float *>(base + lse_offset);
-    return attention_layer(q, kp, vp, tcap, &local, out, stream);
+    return attention_layer(q, kp, vp, tcap, &local, out, pool_layout(tcap), stream);
 }
 
 int ta_read_stream(const void *src, int64_t bytes, uint32_t *sink, int32_t blocks, void *stream) {

@@ -28,7 +28,7 @@ _c_ptr = ctypes.c_void_p
 
 EXPORTS = ("ta_version", "ta_error_string", "ta_segment", "ta_merge", "ta_attention_matrix",
            "ta_attention_matrix_noalloc", "ta_tail_merge", "ta_segment_plan", "ta_merge_plan", "ta_decode_append", "ta_time_next_launch",
-           "ta_read_stream")
+           "ta_read_stream", "ta_attention_tokens")
 
 
 class TaPlan(ctypes.Structure):
@@ -76,6 +76,9 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
                                  _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_ptr]
         lib.ta_attention_matrix.restype = ctypes.c_int
         lib.ta_attention_matrix.argtypes = [_c_ptr, _c_ptr, _c_ptr, _c_i32, ctypes.POINTER(TaPlan),
+                                            _c_ptr, _c_ptr]
+        lib.ta_attention_tokens.restype = ctypes.c_int
+        lib.ta_attention_tokens.argtypes = [_c_ptr, _c_ptr, _c_ptr, _c_i32, ctypes.POINTER(TaPlan),
                                             _c_ptr, _c_ptr]
         lib.ta_attention_matrix_noalloc.restype = ctypes.c_int
         lib.ta_attention_matrix_noalloc.argtypes = [_c_ptr, _c_ptr, _c_ptr, _c_i32, ctypes.POINTER(TaPlan),

@@ -100,9 +100,9 @@ class PreparedPlan:
 
     def for_pools(self, kp: torch.Tensor) -> "PreparedPlan":
         """The plan to launch on pools like ``kp``: this one, or, when it has
-        attached segments and the pool capacity is not a multiple of 8 (the
-        register-staged kernels, which take no attachments), the same plan
-        prepared without attachments, writing into the same ``out``."""
+        attached segments and the pool capacity is not a multiple of 8 (whose
+        kernels bring K through registers and take no attachments), the same
+        plan prepared without attachments, writing into the same ``out``."""
         if not self.attached or kp.shape[-1] % 8 == 0:
             return self
         if self._unattached is None:
@@ -780,8 +780,30 @@ def pack_kv(k: torch.Tensor, v: torch.Tensor):
 
 
 def attention(q, k, v, prepared):
-    """``attention_matrix`` on pools packed from ``k, v [T,HK,D]`` (kernels.py:148-149)."""
-    return attention_matrix(q, *pack_kv(k, v), prepared)
+    """``attention_matrix`` on ``k, v [T,HK,D]`` (kernels.py:148-149).
+
+    Contiguous K and V are attended where they lie (``ta_attention_tokens``):
+    packing them costs a strided pass over both (one layer of 17,424 tokens:
+    140 us packed, 37 us in place).  Anything else is packed first, and
+    ``attention_matrix`` checks it.
+    """
+    abi = prepared.abi
+    tokens = (k.shape[0], abi.hk, abi.d) if k.dim() == 3 else None
+    if not (tokens and 0 < tokens[0] < 2 ** 31 and tuple(k.shape) == tuple(v.shape) == tokens
+            and k.is_contiguous() and v.is_contiguous() and k.data_ptr() % 16 == 0 and v.data_ptr() % 16 == 0
+            and q.is_cuda and k.device == v.device == q.device and q.dtype in _DTYPES
+            and _DTYPES[q.dtype] == abi.dtype and k.dtype == v.dtype == q.dtype
+            and tuple(q.shape) == (abi.nreq, abi.hq, abi.d)):
+        return attention_matrix(q, *pack_kv(k, v), prepared)
+    if not q.is_contiguous():
+        q = q.contiguous()
+    lib = _native.load()
+    with torch.cuda.device(q.device):
+        stream = torch.cuda.current_stream(q.device).cuda_stream
+        rc = lib.ta_attention_tokens(q.data_ptr(), k.data_ptr(), v.data_ptr(), tokens[0], ctypes.byref(abi),
+                                     prepared.out.data_ptr(), stream)
+    _native.check(rc)
+    return prepared.out
 
 
 def _check_inputs(q, kp, vp, p):
