@@ -15,6 +15,7 @@ from oracle.attention_oracle import relative_l2, request_attention
 from tree_attention import CostModel, KVTree, schedule, shapes
 from tree_attention import _native
 from tree_attention.kernels import attention, attention_matrix, pack_kv, prepare
+from tree_attention.schedule import Job, Plan
 
 pytestmark = pytest.mark.gpu
 
@@ -93,3 +94,34 @@ def test_token_major_equals_packed(device):
         attention(q, k.half(), v, p)
     with pytest.raises(ValueError):
         attention(q[:3], k, v, p)
+
+
+@pytest.mark.parametrize("hk", [8, 4])
+@pytest.mark.parametrize("small", [1, 31, 43, 60])
+def test_one_wave_items_in_any_order(small, hk, device):
+    """Launches of one-wave items on both sides of one round of the GPU (1,280 items), alone and
+    beside 64-row items, over requests that are consecutive or not: every item runs once."""
+    d, group = 128, 4
+    nreq = 2 * small + 16
+    jobs = [Job((r, r + 2) if r % 3 == 0 and r % 4 < 2 and r + 2 < 2 * small else (r,),
+                tuple(range(40 * r, 40 * r + 17 + r % 13))) for r in range(2 * small)]
+    jobs += [Job((r,), tuple(range(40 * r + 31, 40 * r + 34 + r % 4))) for r in range(2 * small)]
+    base = 40 * 2 * small
+    wide = [Job(tuple(range(2 * small, nreq)), tuple(range(base, base + 150)))]
+    rest = [Job((r,), tuple(range(base + 160 + 8 * i + o, base + 161 + 8 * i + o)))
+            for i, r in enumerate(range(2 * small, nreq)) for o in (0, 3)]
+    g = torch.Generator().manual_seed(small)
+    t = base + 160 + 8 * nreq
+    q = torch.randn(nreq, group * hk, d, generator=g).bfloat16()
+    k = torch.randn(t, hk, d, generator=g).bfloat16()
+    v = torch.randn(t, hk, d, generator=g).bfloat16()
+    kp, vp = pack_kv(k.to(device), v.to(device))
+    for plan_jobs in (jobs + rest, jobs + rest + wide):
+        paths = [sum((list(j.tokens) for j in plan_jobs if r in j.requests), []) for r in range(nreq)]
+        p = prepare(Plan(plan_jobs, "x", 0.0, dict(kvheads=hk)), q.to(device), route_items=0)
+        say("one-wave", small, hk, list(p.abi.n_items), -1 in p.qbase_host)
+        assert p.abi.n_items[_native.TA_TAIL] == 0 and (p.abi.n_items[_native.TA_SMALL] > 1280) == (hk == 8 and small > 40)
+        out = attention_matrix(q.to(device), kp, vp, p).cpu()
+        ref = request_attention(q.float(), k.float(), v.float(), KVTree([], [tuple(x) for x in paths]))
+        torch.testing.assert_close(out, ref.bfloat16(), atol=0.008, rtol=0.03)
+        assert relative_l2(out, ref) <= 3e-3

@@ -60,6 +60,11 @@ typedef __attribute__((address_space(3))) const u16 lds_u16;
 // s_waitcnt lgkmcnt(0) alone
 #define TA_LGKMCNT0 (15 | (7 << 4) | (0 << 8) | (3 << 14))
 
+// A uniform load through the scalar unit (constant address space).
+__device__ inline int sload(const int32_t *p, int i) {
+    return ((const __attribute__((address_space(4))) int32_t *)p)[i];
+}
+
 // Wait until at most n tiles of this wave's copies (BPW each) are in flight
 // (n = 0 .. 4; the immediate of s_waitcnt must be a constant).
 template <int BPW>
@@ -514,55 +519,70 @@ __device__ __forceinline__ void tile_item(const SegParams &p, const int32_t *__r
     const int wrow0 = row0 + 16 * NB * wave;
     const bool active = wrow0 < nrows;
 
-    // Q^T fragments (B operand): lane (row, g4) holds d = 32*ks + 8*g4 .. +7.
+    const int rb = sload(p.rowbase, job), qb = p.qbase ? sload(p.qbase, job) : -1;
+    const int tb0 = tile_start<L>(kst);
+    const int ntiles = ntok > 0 ? (kend - tb0 + T::TT - 1) / T::TT : 0;
+
+    // Q^T fragments (B operand): lane (row, g4) holds d = 32*ks + 8*g4 .. +7 (rows
+    // past the item repeat its last row and are never stored).  A job over
+    // consecutive requests (qbase) needs no request-id loads.  The first tile's
+    // copies go out behind the Q loads, so that one wait covers both.
     u32x4 qf[NB][KS];
+    const u16 *qsrc[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-        const int rr = wrow0 + 16 * nb + row;
-        if (rr < nrows) {
-            const int lr = rr / p.group, gg = rr - lr * p.group;
-            const int rq = p.qids[(size_t)job * p.maxr + lr];
-            const u16 *src = p.q + ((size_t)rq * p.hq + h * p.group + gg) * D + 8 * g4;
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) qf[nb][ks] = *(const u32x4 *)(src + 32 * ks);
-        } else {
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) qf[nb][ks] = u32x4{0, 0, 0, 0};
+        const int rr = min(wrow0 + 16 * nb + row, nrows - 1);
+        const int lr = rr / p.group;
+        int rq = qb + lr;
+        if (qb < 0) {
+            rq = p.qids[(size_t)job * p.maxr + lr];
+            asm volatile("" : "+v"(rq));  // waited for in this branch only
         }
+        qsrc[nb] = p.q + ((size_t)rq * p.hq + h * p.group + (rr - lr * p.group)) * D + 8 * g4;
     }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) qf[nb][ks] = *(const u32x4 *)(qsrc[nb] + 32 * ks);
+    asm volatile("" ::: "memory");
+    C first;
+    if (ntiles > 0) first.issue(lds, p, h, tb0, kst, kend, wave, lane);
     // Pin the Q fragments: an empty asm that "redefines" them makes the wave
-    // wait for the Q loads once, here, and not inside the tile loop behind the
-    // copies in flight.
+    // wait for the Q loads (and the first tile) once, here, and not inside the
+    // tile loop behind the copies in flight.
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[nb][ks]));
+    if (ntiles > 0) first.finish(lds, wave, lane);
 
     M acc;
     acc.reset();
     const LdsOfs of = T::offsets(row, g4);
 
-    const int tb0 = tile_start<L>(kst);
-    const int ntiles = ntok > 0 ? (kend - tb0 + T::TT - 1) / T::TT : 0;
     if (STAGES == 1) {
-        // one stage (one-wave workgroups, four per CU): copy, wait, compute
+        // one stage (one-wave workgroups, five per CU): copy, wait, compute
         for (int it = 0; it < ntiles; ++it) {
             const int t0 = tb0 + it * T::TT;
-            if (it > 0) item_barrier<SOLO>();  // every wave is done with the previous tile
-            C kr;
-            kr.issue(lds, p, h, t0, kst, kend, wave, lane);
-            __builtin_amdgcn_s_waitcnt(TA_VMCNT(0));
-            kr.finish(lds, wave, lane);
+            if (it > 0) {
+                item_barrier<SOLO>();  // every wave is done with the previous tile
+                C kr;
+                kr.issue(lds, p, h, t0, kst, kend, wave, lane);
+                __builtin_amdgcn_s_waitcnt(TA_VMCNT(0));
+                kr.finish(lds, wave, lane);
+            } else {
+                __builtin_amdgcn_s_waitcnt(TA_VMCNT(0));
+            }
             item_barrier<SOLO>();
             if (active) acc.tile(lds, qf, of, max(0, kst - t0), min(T::TT, kend - t0), g4, p.scale_log2);
         }
     } else {
     // Iteration it copies tile it+STAGES-1 and computes tile it (stage it %
-    // STAGES); the first STAGES-1 iterations only copy, so every copy comes
-    // from one call site.
+    // STAGES); the first STAGES-2 iterations only copy (tile 0 is under way).
     constexpr int AHEAD = STAGES > 1 ? STAGES - 1 : 1;
-    int cs = STAGES - AHEAD;  // stage of tile it, starting at it = -AHEAD
-    for (int it = -AHEAD; it < ntiles; ++it) {
+    int cs = STAGES > 1 ? STAGES - AHEAD + 1 : 0;  // stage of tile it, starting at it = 1 - AHEAD
+    if (cs == STAGES) cs = 0;
+    for (int it = 1 - AHEAD; it < ntiles; ++it) {
         if (it >= 0) {
             // this wave's copies of tile it are done once at most those of the
             // tiles after it (issued, at most AHEAD-1 of them) are pending
@@ -582,7 +602,6 @@ __device__ __forceinline__ void tile_item(const SegParams &p, const int32_t *__r
     }
 
     if (!active) return;
-    const int rb = p.rowbase[job];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
         const int grow = wrow0 + 16 * nb + row;
@@ -593,10 +612,18 @@ __device__ __forceinline__ void tile_item(const SegParams &p, const int32_t *__r
     }
 }
 
+constexpr int ONE_ROUND = 5 * 256;  // one-wave workgroups that run at once at d = 128 (five 32 KiB tiles per CU)
 template <int D, bool FP16, int NB, int NW, int STAGES, int L>
 __global__ __launch_bounds__(64 * NW) void seg_tile_kernel(SegParams p) {
     __shared__ __attribute__((aligned(16))) u16 lds[STAGES * Tile<D>::ELEMS];
-    tile_item<D, FP16, NB, NW, STAGES, L>(p, p.items, xcd_item(blockIdx.x, gridDim.x), lds, threadIdx.x, 16 * NB * NW);
+    // One-wave items lie job by job with the KV heads inside: with item i on XCD i % 8 an
+    // XCD works on one head of 8 and translates and caches an eighth of the pools.  That
+    // helps a launch whose items all run at once (8 requests, 1024 shared + 64 tokens:
+    // layer 10.1 -> 9.1 us); a launch of several rounds keeps whole jobs on an XCD (128 x
+    // 8192 private tokens: 793 us by heads, 781 us by jobs).
+    const bool by_head = NW == 1 && p.hk % 8 == 0 && gridDim.x <= ONE_ROUND;
+    const int item = by_head ? blockIdx.x : xcd_item(blockIdx.x, gridDim.x);
+    tile_item<D, FP16, NB, NW, STAGES, L>(p, p.items, item, lds, threadIdx.x, 16 * NB * NW);
 }
 
 // ------------------------------------------------------------------------
@@ -1057,9 +1084,13 @@ __global__ __launch_bounds__(64 * NW) void seg_pipe_kernel(SegParams p) {
 // segments), blocks [base[1], base[2]) run 64-row items on eight waves (the
 // upper four copy and meet at the barriers), and the blocks from base[2] on
 // run four small items each, one per wave on its own stage (the upper four
-// waves end at once).  The bases are multiples of 8, so that every kind's
-// items map to XCDs as in its own kernel; blocks past a kind's item count end
+// waves end at once).  The bases are multiples of 8, so that the row tiles map
+// to XCDs as in their own kernels; blocks past a kind's item count end
 // at once.  The kinds run side by side instead of one launch after another.
+// Small items beside 64-row items keep item i on XCD i % 8 (one KV head of 8
+// per XCD; layers of 32 and 24 requests in two branches 43.3 -> 42.5 us and
+// 26.2 -> 25.1 us); beside 256-row items, which fill whole CUs by head already,
+// four neighbours share a workgroup (by head 0.1-0.5 us slower on two layers).
 template <int D, bool FP16, int L>
 __global__ __launch_bounds__(512) void seg_mix_kernel(MixParams mp) {
     using T = Tile<D>;
@@ -1074,7 +1105,8 @@ __global__ __launch_bounds__(512) void seg_mix_kernel(MixParams mp) {
         if (lb >= mp.n[1]) return;
         tile_item<D, FP16, 1, 8, 3, L>(mp.p, mp.items[1], xcd_item(lb, mp.n[1]), lds, tid, 64);
     } else {
-        const int wave = tid >> 6, it = 4 * (b - mp.base[2]) + wave;
+        const int lb = b - mp.base[2], wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int it = mp.n[0] ? 4 * lb + wave : 8 * (4 * (lb >> 3) + wave) + (lb & 7);
         if (wave >= 4 || it >= mp.n[2]) return;
         tile_item<D, FP16, 1, 1, 1, L, true>(mp.p, mp.items[2], it, lds + wave * T::ELEMS, tid & 63, 16);
     }
@@ -1288,10 +1320,10 @@ hipError_t launch_mix<TA_LAYOUT>(const SegParams &sp, const int32_t *const items
         mp.items[k] = items[k];
         mp.n[k] = n[k] > 0 ? n[k] : 0;
         mp.base[k] = base;
-        const int blocks = k < 2 ? mp.n[k] : (mp.n[k] + 3) / 4;
-        base += (blocks + 7) & ~7;
+        base += (mp.n[k] + 7) & ~7;  // (the last kind's is not needed)
     }
-    const int blocks = mp.base[2] + (mp.n[2] + 3) / 4;
+    const int small_blocks = n[0] > 0 ? (mp.n[2] + 3) / 4 : (mp.n[2] + 31) / 32 * 8;
+    const int blocks = mp.base[2] + small_blocks;
     if (blocks <= 0) return hipSuccess;
     TA_BY_SHAPE(launch_mix_d, TA_LAYOUT, mp, blocks, stream)
 }
