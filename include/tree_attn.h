@@ -217,6 +217,12 @@ int ta_decode_append(const void *q, const void *k, const void *v, const void *co
                      int32_t nreq, int32_t hq, int32_t hk, int32_t d, int32_t tcap, int32_t dtype,
                      void *stream);
 
+/* metadata[offsets[i]] = value for i < n: the lengths of a cached plan's growing
+ * tails, one launch per decode step (klen of tail jobs and the tokens fields of
+ * attachment records; kernels.PreparedPlan.grow_offsets lists the positions;
+ * kernels.py:184-186 writes klen).  metadata: the plan's int32 device buffer. */
+int ta_fill_lengths(int32_t *metadata, const int64_t *offsets, int32_t n, int32_t value, void *stream);
+
 /* Kernel timing hook.  No counterpart in the reference, which times kernels
  * with device events around whole launches (scripts/profile_kernel.py:17-33).
  * The next kernel this library launches on the calling host thread records

@@ -1,0 +1,111 @@
+"""The host entry of the per-layer calls (csrc/fastcall.cpp) against the general path.
+
+Every form that the calls accept -- contiguous or not, any slot type, one RoPE row or one per
+request, an output given or not, another stream -- gives the bits that the ctypes path gives,
+and what was refused is refused with the same error.
+"""
+import pytest
+import torch
+
+from tree_attention import CostModel, schedule, shapes
+from tree_attention import _native, kernels
+from tree_attention.kernels import CachedDecodePlan, attention_matrix, decode_append, pack_kv, prepare
+
+pytestmark = pytest.mark.gpu
+
+
+class _General:
+    """Stands in for the module: every call takes the general path."""
+    attention = decode_append = fill = staticmethod(lambda *a: None)
+
+
+@pytest.fixture
+def general(monkeypatch):
+    def run(fn):
+        _native.load()
+        with monkeypatch.context() as m:
+            m.setattr(_native, "fastcall", _General)
+            out = fn()
+        torch.cuda.synchronize()
+        return out
+    return run
+
+
+def test_attention_matrix_forms(device, general):
+    tree = shapes.tree(shapes.shared_prefix(32, 2048, 64))
+    g = torch.Generator().manual_seed(2)
+    q = torch.randn(32, 32, 128, generator=g).bfloat16().to(device)
+    k = torch.randn(tree.storage_tokens, 8, 128, generator=g).bfloat16().to(device)
+    v = torch.randn(tree.storage_tokens, 8, 128, generator=g).bfloat16().to(device)
+    kp, vp = pack_kv(k, v)
+    odd = pack_kv(torch.cat([k, k[:3]]), torch.cat([v, v[:3]]))
+    p = prepare(schedule(tree, 32, 8, 128, "cube", CostModel.mi355x()), q)
+    assert p.attached
+    side = torch.cuda.Stream()
+    for what, qx, pools in (("plain", q, (kp, vp)), ("strided q", q.transpose(0, 1).contiguous().transpose(0, 1), (kp, vp)),
+                            ("odd capacity", q, odd)):
+        fast = attention_matrix(qx, *pools, p).clone()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            on_side = attention_matrix(qx, *pools, p).clone()
+        torch.cuda.current_stream().wait_stream(side)
+        want = general(lambda: attention_matrix(qx, *pools, p).clone())
+        assert torch.equal(fast, want) and torch.equal(on_side, want), what
+    for bad in ((q.half(), kp, vp), (q[:5], kp, vp), (q, kp.transpose(1, 2), vp), (q, kp, vp[:, :-8]), (q.cpu(), kp, vp),
+                (q, kp.cpu(), vp), (q, kp[0], vp)):
+        with pytest.raises(ValueError) as fast_error:
+            attention_matrix(*bad, p)
+        with pytest.raises(ValueError) as general_error:
+            general(lambda: attention_matrix(*bad, p))
+        assert str(fast_error.value) == str(general_error.value)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rope_rows", [1, 6])
+def test_decode_append_forms(dtype, rope_rows, device, general):
+    nreq, hq, hk, d, cap = 6, 8, 2, 64, 40
+    g = torch.Generator().manual_seed(rope_rows)
+
+    def randn(*shape):
+        return torch.randn(*shape, generator=g).to(dtype).to(device)
+
+    q, k, v = randn(nreq, 1, hq, d), randn(nreq, 1, hk, d), randn(nreq, 1, hk, d)
+    cos, sin = randn(rope_rows, 1, d), randn(rope_rows, 1, d)
+    kp, vp = randn(hk, d, cap), randn(hk, cap, d)
+    slots = torch.randperm(cap, generator=g)[:nreq]
+    flat = [t.reshape(nreq, -1, d) for t in (q, k, v)]
+    strided = [torch.stack([t, t], dim=-1)[..., 0] for t in (q, k, v)]
+    for what, qkv, sl in (("plain", (q, k, v), slots.int().to(device)), ("3-d", flat, slots.int().to(device)),
+                          ("strided", strided, slots.int().to(device)), ("int64", (q, k, v), slots.to(device)),
+                          ("host", (q, k, v), slots.tolist())):
+        for given in (False, True):
+            got, pools = [], []
+            for run in (lambda f: f(), general):
+                a, b = kp.clone(), vp.clone()
+                out = torch.empty(nreq, hq, d, device=device, dtype=dtype) if given else None
+                got.append(run(lambda: decode_append(*qkv, cos, sin, sl, a, b, out)))
+                pools.append((a, b))
+            torch.cuda.synchronize()
+            assert torch.equal(got[0], got[1]) and got[0].shape == (nreq, hq, d), what
+            assert all(torch.equal(x, y) for x, y in zip(*pools)), what
+    for bad in (dict(k=k[:, :, :1]), dict(kp=kp.transpose(1, 2)), dict(cos=cos.float()), dict(v=v[:3])):
+        args = {**dict(q=q, k=k, v=v, cos=cos, sin=sin, slots=slots.int().to(device), kp=kp, vp=vp), **bad}
+        errors = []
+        for run in (lambda f: f(), general):
+            with pytest.raises((ValueError, RuntimeError)) as e:
+                run(lambda: decode_append(**args))
+            errors.append((type(e.value), str(e.value)))
+        assert errors[0] == errors[1], bad.keys()
+
+
+@pytest.mark.parametrize("requests", [1, 3, 70])
+def test_fill_growing(requests, device, general):
+    """Every word of the metadata after an update equals the torch op's."""
+    tree = shapes.tree(shapes.shared_prefix(requests, 700, 5))
+    q = torch.empty(requests, 32, 128, dtype=torch.bfloat16, device=device)
+    c = CachedDecodePlan(schedule(tree, 32, 8, 128, "cube", CostModel.mi355x()), q, tree.storage_tokens, 9)
+    for n in (9, 0, 4):
+        fast = c.update(n).metadata.clone()
+        c.update(7)
+        want = general(lambda: c.update(n).metadata.clone())
+        assert torch.equal(fast, want) and kernels._fastcall().fill is not None

@@ -1,5 +1,6 @@
-"""Build ``libtree_attn.so`` (gfx950) and ``libtree_plan.so`` (host planner)
-next to the ``tree_attention`` package.
+"""Build ``libtree_attn.so`` (gfx950), ``libtree_plan.so`` (host planner) and
+``_fastcall.so`` (Python entry of the per-layer calls) next to the
+``tree_attention`` package.
 
     python tree-attention-scheduling_amd/csrc/build.py
 
@@ -21,6 +22,7 @@ PKG = HERE.parent / "tree_attention"
 INCLUDE = HERE.parent.parent / "include"
 LIB = PKG / "libtree_attn.so"
 PLAN_LIB = PKG / "libtree_plan.so"
+FASTCALL = PKG / "_fastcall.so"
 # The planner's costs must round exactly like the Python planner's: no FMA
 # contraction, no fast-math reassociation.
 PLAN_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", "-fno-fast-math", "-Wall"]
@@ -84,6 +86,26 @@ def build(verbose: bool = False, out: Path | None = None, defines=()) -> Path:
     return target
 
 
+def build_fastcall(verbose: bool = False, out: Path | None = None) -> Path:
+    """Compile the Python entry of the per-layer calls (fastcall.cpp) into ``out`` (default:
+    in-tree) with g++ against the installed torch."""
+    import sysconfig
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    target = Path(out) if out is not None else FASTCALL
+    tmp = target.with_name(target.name + f".tmp{os.getpid()}")
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("g++ not found; it is required to build the host module")
+    lib = Path(torch.__file__).parent / "lib"
+    _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          *[f"-isystem{p}" for p in include_paths()], f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}",
+          str(HERE / "fastcall.cpp"), f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-o", str(tmp)],
+         verbose)
+    os.replace(tmp, target)
+    return target
+
+
 def build_planner(verbose: bool = False, out: Path | None = None) -> Path:
     """Compile the host planner (planner.cpp) into ``out`` (default: in-tree) with g++."""
     target = Path(out) if out is not None else PLAN_LIB
@@ -109,3 +131,4 @@ if __name__ == "__main__":
     print(build(verbose=True, out=out, defines=defines))
     if out is None:
         print(build_planner(verbose=True))
+        print(build_fastcall(verbose=True))

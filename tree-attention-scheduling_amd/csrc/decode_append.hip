@@ -87,8 +87,23 @@ __global__ __launch_bounds__(64) void decode_append_kernel(const u16 *__restrict
     }
 }
 
+// The growing tails' lengths of a cached plan: n words of its metadata set to one value.
+__global__ __launch_bounds__(256) void fill_lengths_kernel(int32_t *__restrict__ meta,
+                                                           const int64_t *__restrict__ offsets, int n, int value) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) meta[offsets[i]] = value;
+}
+
 }  // namespace
 }  // namespace ta
+
+extern "C" int ta_fill_lengths(int32_t *metadata, const int64_t *offsets, int32_t n, int32_t value, void *stream) {
+    if (n < 0 || (n > 0 && (!metadata || !offsets))) return TA_ERR_ARG;
+    if (n == 0) return 0;
+    TA_LAUNCH(ta::fill_lengths_kernel, dim3((n + 255) / 256), dim3(256), static_cast<hipStream_t>(stream), metadata,
+              offsets, n, value);
+    return (int)hipGetLastError();
+}
 
 extern "C" int ta_decode_append(const void *q, const void *k, const void *v, const void *cos, const void *sin,
                                 int32_t cs_stride, const int32_t *slots, void *kp, void *vp, void *q_out,

@@ -9,11 +9,14 @@ environment variable ``TREE_ATTN_LIB`` selects another build of the library.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).with_name("libtree_attn.so")
+FASTCALL_PATH = Path(__file__).with_name("_fastcall.so")
 
 TA_BF16, TA_FP16 = 0, 1
 TA_SMALL, TA_LARGE64, TA_LARGE128, TA_LARGE256, TA_TAIL = 0, 1, 2, 3, 4
@@ -28,7 +31,7 @@ _c_ptr = ctypes.c_void_p
 
 EXPORTS = ("ta_version", "ta_error_string", "ta_segment", "ta_merge", "ta_attention_matrix",
            "ta_attention_matrix_noalloc", "ta_tail_merge", "ta_segment_plan", "ta_merge_plan", "ta_decode_append", "ta_time_next_launch",
-           "ta_read_stream", "ta_attention_tokens")
+           "ta_read_stream", "ta_attention_tokens", "ta_fill_lengths")
 
 
 class TaPlan(ctypes.Structure):
@@ -45,6 +48,7 @@ class TaPlan(ctypes.Structure):
 
 
 _lib = None
+fastcall = None  # the host module of the per-layer calls, set by load()
 _lock = threading.Lock()
 
 
@@ -92,13 +96,32 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
         lib.ta_decode_append.restype = ctypes.c_int
         lib.ta_decode_append.argtypes = [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i32, _c_ptr, _c_ptr, _c_ptr,
                                          _c_ptr, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_ptr]
+        lib.ta_fill_lengths.restype = ctypes.c_int
+        lib.ta_fill_lengths.argtypes = [_c_ptr, _c_ptr, _c_i32, _c_i32, _c_ptr]
         lib.ta_time_next_launch.restype = ctypes.c_int
         lib.ta_time_next_launch.argtypes = [_c_ptr, _c_ptr]
         lib.ta_read_stream.restype = ctypes.c_int
         lib.ta_read_stream.argtypes = [_c_ptr, ctypes.c_int64, _c_ptr, _c_i32, _c_ptr]
         if path is None:
+            _bind_fastcall(lib)
             _lib = lib
         return lib
+
+
+def _bind_fastcall(lib) -> None:
+    """Load the host module of the per-layer calls (csrc/fastcall.cpp) and give it ``lib``'s functions."""
+    global fastcall
+    import torch
+    if not FASTCALL_PATH.exists():
+        raise RuntimeError(f"tree_attn host module not found at {FASTCALL_PATH}; build it with "
+                           "`python -c 'import __graft_entry__ as g; g.build()'` from the repository root")
+    loader = importlib.machinery.ExtensionFileLoader("_fastcall", str(FASTCALL_PATH))
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_fastcall", loader))
+    loader.exec_module(module)
+    module.bind(*(ctypes.cast(getattr(lib, name), _c_ptr).value for name in
+                  ("ta_attention_matrix", "ta_attention_tokens", "ta_decode_append", "ta_fill_lengths")),
+                torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice)
+    fastcall = module
 
 
 def check(rc: int) -> None:

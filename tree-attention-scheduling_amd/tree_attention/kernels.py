@@ -93,7 +93,11 @@ class PreparedPlan:
         """Set the length of every growing tail (tokens from ``fixed_from`` on) to
         ``length``, here and in the unattached variant (device-side, no sync)."""
         if self.grow_offsets is not None:
-            self.metadata.index_fill_(0, self.grow_offsets, length)
+            rc = _fastcall().fill(self.metadata, self.grow_offsets, length) if self.metadata.is_cuda else None
+            if rc is None:  # (metadata on the host, or another device current)
+                self.metadata.index_fill_(0, self.grow_offsets, length)
+            elif rc:
+                _native.check(rc)
         self.growing_len = length
         if self._unattached is not None:
             self._unattached.fill_growing(length)
@@ -787,23 +791,19 @@ def attention(q, k, v, prepared):
     140 us packed, 37 us in place).  Anything else is packed first, and
     ``attention_matrix`` checks it.
     """
-    abi = prepared.abi
-    tokens = (k.shape[0], abi.hk, abi.d) if k.dim() == 3 else None
-    if not (tokens and 0 < tokens[0] < 2 ** 31 and tuple(k.shape) == tuple(v.shape) == tokens
-            and k.is_contiguous() and v.is_contiguous() and k.data_ptr() % 16 == 0 and v.data_ptr() % 16 == 0
-            and q.is_cuda and k.device == v.device == q.device and q.dtype in _DTYPES
-            and _DTYPES[q.dtype] == abi.dtype and k.dtype == v.dtype == q.dtype
-            and tuple(q.shape) == (abi.nreq, abi.hq, abi.d)):
+    rc = _fastcall().attention(q, k, v, ctypes.addressof(prepared.abi), prepared.out, True)
+    if rc is None:
         return attention_matrix(q, *pack_kv(k, v), prepared)
-    if not q.is_contiguous():
-        q = q.contiguous()
-    lib = _native.load()
-    with torch.cuda.device(q.device):
-        stream = torch.cuda.current_stream(q.device).cuda_stream
-        rc = lib.ta_attention_tokens(q.data_ptr(), k.data_ptr(), v.data_ptr(), tokens[0], ctypes.byref(abi),
-                                     prepared.out.data_ptr(), stream)
-    _native.check(rc)
+    if rc:
+        _native.check(rc)
     return prepared.out
+
+
+def _fastcall():
+    """The host module of the per-layer calls (csrc/fastcall.cpp)."""
+    if _native.fastcall is None:
+        _native.load()
+    return _native.fastcall
 
 
 def _check_inputs(q, kp, vp, p):
@@ -830,6 +830,11 @@ def attention_matrix(q, kp, vp, prepared):
     Returns ``prepared.out`` (``[R, HQ, D]`` in q's dtype), which every call
     overwrites, as in the reference.
     """
+    rc = _fastcall().attention(q, kp, vp, ctypes.addressof(prepared.abi), prepared.out, False)
+    if rc is not None:  # the ordinary call; None: the general path below
+        if rc:
+            _native.check(rc)
+        return prepared.out
     _check_inputs(q, kp, vp, prepared)
     p = prepared.for_pools(kp)
     if not q.is_contiguous():
@@ -916,6 +921,12 @@ def decode_append(q, k, v, cos, sin, slots, kp, vp, q_out=None):
     would synchronise the host); the kernel then skips a position outside the
     pool, writing nothing for it.
     """
+    if q_out is None and isinstance(slots, torch.Tensor) and slots.is_cuda:
+        out = _fastcall().decode_append(q, k, v, cos, sin, slots, kp, vp)
+        if isinstance(out, torch.Tensor):
+            return out
+        if out is not None:
+            _native.check(out)
     nreq = q.shape[0]
     d = q.shape[-1]
     q2, k2, v2 = q.reshape(nreq, -1, d), k.reshape(nreq, -1, d), v.reshape(nreq, -1, d)
