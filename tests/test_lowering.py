@@ -1,0 +1,92 @@
+"""The lowering of plans (``kernels.prepare``): what each work item holds, read back from its
+metadata the way the kernels read it."""
+import random
+
+import pytest
+import torch
+
+from tree_attention import _native
+from tree_attention.kernels import XTAIL_FIELDS, prepare
+from tree_attention.schedule import Job, Plan
+
+
+def held(p, group, kvheads):
+    """Per (request, KV head): the sorted tokens its work items attend, from the device metadata."""
+    qids, kstart, qlen, klen = (t.tolist() for t in (p.qids, p.kids[:, 0], p.qlen, p.klen))
+    out = {}
+
+    def add(reqs, head, t0, n):
+        for r in reqs:
+            out.setdefault((r, head), []).extend(range(t0, t0 + n))
+
+    for kind in range(_native.TA_NKINDS):
+        items = p.items[kind].view(-1, 3).tolist()
+        for i, (j, row0, head) in enumerate(items):
+            rows = _native.KIND_ROWS.get(kind, 16)
+            per = rows // group if rows >= group else 1
+            add(qids[j][:qlen[j]][row0 // group:row0 // group + per], head, kstart[j], klen[j])
+            if kind == _native.TA_LARGE256 and p.xtail is not None:
+                rec = p.xtail[i].tolist()
+                for k in range(rec[0]):
+                    t0, n, lrow, nrows = rec[1 + XTAIL_FIELDS * k:1 + XTAIL_FIELDS * (k + 1)]
+                    assert row0 <= lrow and lrow + nrows <= min(row0 + 256, qlen[j] * group)
+                    add(qids[j][lrow // group:(lrow + nrows) // group], head, t0, n)
+    return {key: sorted(v) for key, v in out.items()}
+
+
+def check_covers(plan, p, nreq, group, kvheads):
+    want = [[] for _ in range(nreq)]
+    for job in plan.jobs:
+        for r in job.requests:
+            want[r].extend(job.tokens)
+    got = held(p, group, kvheads)
+    for r in range(nreq):
+        for h in range(kvheads):
+            assert got.get((r, h), []) == sorted(want[r]), (r, h)
+
+
+def random_plan(rng, nreq):
+    """A random prefix tree's jobs: a root, uneven branches, nodes of a few requests, tails."""
+    jobs, base = [], rng.randrange(0, 9)
+
+    def job(reqs, n):
+        nonlocal base
+        jobs.append(Job(tuple(reqs), tuple(range(base, base + n))))
+        base += n + rng.choice((0, 0, 3))
+
+    def split(reqs, depth):
+        job(reqs, rng.choice((5, 64, 300, 2100) if depth else (64, 700, 4096)))
+        if depth < 3 and len(reqs) > 1 and rng.random() < 0.9:
+            cuts = sorted(rng.sample(range(1, len(reqs)), min(len(reqs) - 1, rng.choice((1, 1, 2, 5)))))
+            for a, b in zip([0] + cuts, cuts + [len(reqs)]):
+                split(reqs[a:b], depth + 1)
+
+    split(list(range(nreq)), 0)
+    for r in range(nreq):
+        job([r], rng.choice((1, 40, 64, 64, 130)))
+    return Plan(jobs, "x", 0.0, dict(kvheads=2))
+
+
+def test_attachments_follow_their_items_past_attached_nodes():
+    """A node of 8 requests attaches to the root's items and leaves the list of large jobs; the
+    256-row jobs after it keep their own attachments (they are named by their place)."""
+    jobs = [Job(tuple(range(64)), tuple(range(0, 4096))), Job(tuple(range(8)), tuple(range(4096, 4160))),
+            Job(tuple(range(8, 64)), tuple(range(4160, 6208)))]
+    jobs += [Job((r,), tuple(range(6208 + 64 * r, 6272 + 64 * r))) for r in range(64)]
+    plan = Plan(jobs, "x", 0.0, dict(kvheads=8))
+    p = prepare(plan, torch.empty(64, 32, 128, dtype=torch.bfloat16))
+    assert any(len(seg.requests) == 8 for segs in p.attached.values() for seg, _ in segs)
+    assert {p.jobs[j].requests[0] for j, _ in p.attached} == {0, 8}
+    check_covers(plan, p, 64, 4, 8)
+
+
+@pytest.mark.parametrize("seed", range(40))
+def test_random_trees_cover_every_token(seed):
+    """Every request's work items hold its path once, per KV head."""
+    rng = random.Random(seed)
+    nreq = rng.choice((1, 3, 17, 40, 72, 130))
+    plan = random_plan(rng, nreq)
+    group = rng.choice((4, 4, 8))
+    q = torch.empty(nreq, 2 * group, 128, dtype=torch.bfloat16)
+    for opts in ({}, dict(attach_tails=False), dict(tile_rows=64)):
+        check_covers(plan, prepare(plan, q, **opts), nreq, group, 2)

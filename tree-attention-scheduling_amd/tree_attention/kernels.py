@@ -647,7 +647,10 @@ def prepare(plan: Plan, q: torch.Tensor, tile_rows: int = 256, fixed_from: int |
             small = [j for j in left if len(j.requests) * group <= SMALL_ROWS]
             if mids:
                 gone = {id(job) for segs in attached.values() for job, _ in segs}
-                large = [j for j in large if id(j) not in gone]
+                stay = [i for i, j in enumerate(large) if id(j) not in gone]
+                place = {old: new for new, old in enumerate(stay)}  # attachments name jobs by their place
+                attached = {(place[i], row0): segs for (i, row0), segs in attached.items()}
+                large = [large[i] for i in stay]
         return small, large, attached
 
     def lowering(min_tiles, fill=None):
