@@ -80,6 +80,28 @@ int tp_attach_tails(int32_t n_large, const int32_t *is256, const int32_t *tiles,
                     int32_t *item_job, int32_t *item_row0, int32_t *n_items);
 
 /*
+ * The execution jobs and attachments of a plan (the backend's prepare(), no
+ * counterpart in the reference): fusing jobs over one token run, re-cutting,
+ * attaching, consolidating and routing, as tree_attention/kernels.py's _lower.
+ * Jobs j < njobs: requests req[req_off[j] .. req_off[j+1]) in [0, nreq), tokens
+ * [start[j], start[j] + ntok[j]).  options[19]: kvheads, group, tile_rows,
+ * attach_tails, consolidate_rows, large_target, large_min_tiles, CUs,
+ * fixed_from (-1: none), xtail_max, wave_rows, attach_min_cap, small_target,
+ * tokens per tile, route_items, fuse_rows, tail_keep_tiles,
+ * tail_keep_items_per_cu, small_pairs.
+ * Returns a handle and sizes[7]: jobs, small jobs, request groups, their
+ * requests in all, items with attachments, attached segments, ints that
+ * tp_lower_take writes; NULL for invalid arguments (nothing to free).
+ * tp_lower_take writes per job its group, per job its first token, per job its
+ * tokens, the groups' sizes, the groups' requests, (large job, first row,
+ * segments) of each item with attachments, then (group, first token, tokens,
+ * first job row) of each segment, and frees the handle (out NULL: frees only).
+ */
+void *tp_lower(int32_t njobs, const int32_t *req_off, const int32_t *req, const int32_t *start, const int32_t *ntok,
+               int32_t nreq, const int64_t *options, int32_t *sizes);
+void tp_lower_take(void *handle, int32_t *out);
+
+/*
  * Device metadata of a prepared plan (the backend's prepare(), cf. the
  * reference's kernels.py:103-141), every int32 section in one buffer:
  *   qids[njobs*maxr] kstart[njobs] qlen[njobs] klen[njobs] slots[nreq*maxs]

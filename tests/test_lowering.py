@@ -90,3 +90,38 @@ def test_random_trees_cover_every_token(seed):
     q = torch.empty(nreq, 2 * group, 128, dtype=torch.bfloat16)
     for opts in ({}, dict(attach_tails=False), dict(tile_rows=64)):
         check_covers(plan, prepare(plan, q, **opts), nreq, group, 2)
+
+
+@pytest.mark.parametrize("seed", range(60))
+def test_native_lowering_equals_python(seed):
+    """tp_lower gives the jobs and attachments of kernels._lower_py, in the same order, over random
+    trees, head groups and every option."""
+    from tree_attention import _planner, kernels
+    assert _planner.available()
+    rng = random.Random(1000 + seed)
+    nreq = rng.choice((1, 3, 17, 40, 72, 130))
+    plan = random_plan(rng, nreq)
+    tokens = max(j.tokens[-1] for j in plan.jobs)
+    group = rng.choice((1, 2, 4, 4, 8, 16, 24))
+    opts = dict(kvheads=rng.choice((1, 2, 8)), group=group, tile_rows=rng.choice((256, 256, 128, 64)),
+                fixed_from=rng.choice((None, None, 0, tokens // 2)), attach_tails=rng.random() < 0.8,
+                route_items=rng.choice((0, 768, 5000)), fuse_rows=rng.choice((0, 64, 256)),
+                consolidate_rows=rng.choice((0, 128, 256)), large_target=rng.choice((0, 1, 64, 256)),
+                small_target=rng.choice((0, 64, 2048)), large_min_tiles=rng.choice((1, 2, 4)))
+    jobs = list(plan.jobs)
+    if rng.random() < 0.5:  # jobs over one token run, split by requests, and chunks of one group
+        wide = jobs[0]
+        cut = len(wide.requests) // 2
+        half = len(wide.tokens) // 2
+        jobs = [Job(r, t) for r in (wide.requests[:cut], wide.requests[cut:]) if r
+                for t in (wide.tokens[:half], wide.tokens[half:]) if t] + jobs[1:]
+    want = kernels._lower_py(jobs, 256, **opts)
+    got = kernels._lower(jobs, nreq, 256, **opts)
+    assert got[1] == want[1] and got[0] == want[0]
+    assert list(got[2].items()) == list(want[2].items())
+
+
+def test_native_lowering_leaves_bad_requests_to_prepare():
+    plan = Plan([Job((0, 5), (0, 1, 2))], "x", 0.0, dict(kvheads=1))
+    with pytest.raises(ValueError, match="names request 5"):
+        prepare(plan, torch.empty(2, 4, 32, dtype=torch.float16))

@@ -25,7 +25,10 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <map>
+#include <memory>
 #include <unordered_map>
+#include <utility>
 #include <vector>
 
 namespace {
@@ -635,4 +638,375 @@ extern "C" int tp_build_metadata(int32_t njobs, int32_t small_jobs, const int32_
     }
     std::copy(qbase.begin(), qbase.end(), p);
     return 0;
+}
+
+// ---------------------------------------------------------------- lowering
+// The execution jobs and attachments of a plan: tree_attention/kernels.py's
+// _lower, step for step (the comments there say why each rule stands; a test
+// compares both on random plans).  Request groups are interned, so that equal
+// groups compare as ints.
+namespace {
+
+struct Lowering {
+    using Reqs = std::vector<int32_t>;
+    struct LJob {
+        int32_t group, t0, n;
+    };
+    struct Seg {
+        LJob job;
+        int32_t lrow;
+    };
+    struct Att {
+        int32_t job, row0;
+        std::vector<Seg> segs;
+    };
+    struct Lowered {
+        std::vector<LJob> small, large;
+        std::vector<Att> att;
+    };
+
+    const int64_t *o;  // options, in tp_lower's order
+    int32_t nreq;
+    std::vector<Reqs> groups;
+    std::map<Reqs, int32_t> index;
+    std::vector<LJob> small0, large0, routed;
+    std::vector<LJob> jobs;
+    int32_t small_jobs = 0;
+    std::vector<Att> att;
+
+    int64_t kvheads() const { return o[0]; }
+    int64_t group() const { return o[1]; }
+    int64_t tile_rows() const { return o[2]; }
+    int64_t n_cu() const { return o[7]; }
+    int64_t quantum() const { return o[13]; }
+    int64_t item_rows() const { return 256; }
+
+    int32_t intern(const Reqs &r) {
+        const auto it = index.emplace(r, (int32_t)groups.size());
+        if (it.second) groups.push_back(r);
+        return it.first->second;
+    }
+    int64_t size(const LJob &j) const { return (int64_t)groups[j.group].size(); }
+    int64_t rows(const LJob &j) const { return size(j) * group(); }
+    int64_t tiles(const LJob &j) const { return ((int64_t)j.t0 + j.n - (j.t0 & ~7) + quantum() - 1) / quantum(); }
+    bool growing(const LJob &j) const { return o[8] >= 0 && j.t0 >= o[8]; }
+    int kind(int64_t r) const { return r <= 64 || tile_rows() <= 64 ? 1 : tile_rows() <= 128 ? 2 : 3; }
+    static int64_t up(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+    void slices(const LJob &j, int64_t per, std::vector<LJob> &out) {
+        const Reqs all = groups[j.group];
+        for (size_t i = 0; i < all.size(); i += per)
+            out.push_back({intern(Reqs(all.begin() + i, all.begin() + std::min(all.size(), i + (size_t)per))), j.t0, j.n});
+    }
+
+    void fuse(std::vector<LJob> &in, int64_t min_rows) {
+        std::map<std::pair<int32_t, int32_t>, std::vector<size_t>> runs;
+        for (size_t i = 0; i < in.size(); ++i)
+            if (rows(in[i]) > 16) runs[{in[i].t0, in[i].n}].push_back(i);
+        std::map<std::pair<int32_t, int32_t>, int32_t> fused;  // group, or -1 once placed
+        for (const auto &run : runs) {
+            if (run.second.size() < 2) continue;
+            Reqs all;
+            for (size_t i : run.second) all.insert(all.end(), groups[in[i].group].begin(), groups[in[i].group].end());
+            if ((int64_t)all.size() * group() < min_rows) continue;
+            std::sort(all.begin(), all.end());
+            if (std::adjacent_find(all.begin(), all.end()) == all.end()) fused[run.first] = intern(all);
+        }
+        if (fused.empty()) return;
+        std::vector<LJob> out;
+        for (const LJob &j : in) {
+            const auto it = fused.find({j.t0, j.n});
+            if (it == fused.end() || rows(j) <= 16) {
+                out.push_back(j);
+            } else if (it->second >= 0) {
+                out.push_back({it->second, j.t0, j.n});
+                it->second = -1;
+            }
+        }
+        in.swap(out);
+    }
+
+    template <class Items, class Fixed>
+    std::vector<LJob> recut(const std::vector<LJob> &in, Items items, int64_t target, Fixed is_fixed, int64_t min_tiles,
+                            int64_t floor_items, bool one_round, bool pairs) {
+        struct Run {
+            LJob j;
+            bool fixed;
+            int64_t w;
+        };
+        std::vector<Run> runs;
+        for (size_t i = 0; i < in.size(); ++i) {
+            const bool fixed = is_fixed(i);
+            if (!runs.empty() && !fixed && !runs.back().fixed && runs.back().j.group == in[i].group &&
+                runs.back().j.t0 + runs.back().j.n == in[i].t0)
+                runs.back().j.n += in[i].n;
+            else
+                runs.push_back({in[i], fixed, items(in[i])});
+        }
+        int64_t fixed_items = 0, longest = 0;
+        for (const Run &r : runs) {
+            if (r.fixed)
+                fixed_items += r.w;
+            else
+                longest = std::max<int64_t>(longest, r.j.n);
+        }
+        if (longest == 0) return in;
+        auto count = [&](int64_t limit) {
+            int64_t c = fixed_items;
+            for (const Run &r : runs)
+                if (!r.fixed) c += r.w * up(r.j.n, limit);
+            return c;
+        };
+        const int64_t q = quantum();
+        int64_t lo = 1, hi = up(longest, q);
+        if (count(hi * q) >= target) lo = hi;
+        while (hi - lo > 1) {
+            const int64_t mid = (lo + hi) / 2;
+            (count(mid * q) >= target ? lo : hi) = mid;
+        }
+        if (one_round && hi > lo) {
+            const int64_t rounds = up(count(lo * q), target);
+            if (rounds > 1 && hi < rounds * lo) lo = hi;
+        }
+        if (pairs && lo == 1 && hi == 2 && 20 * count(q) >= 9 * target) lo = 2;
+        if (lo < min_tiles && count(min_tiles * q) >= floor_items) lo = min_tiles;
+        const int64_t limit = lo * q;
+        std::vector<LJob> out;
+        for (const Run &r : runs) {
+            if (r.fixed) {
+                out.push_back(r.j);
+                continue;
+            }
+            const int64_t step = up(up(r.j.n, up(r.j.n, limit)), 8) * 8;
+            for (int64_t a = 0; a < r.j.n; a += step)
+                out.push_back({r.j.group, (int32_t)(r.j.t0 + a), (int32_t)std::min<int64_t>(step, r.j.n - a)});
+        }
+        return out;
+    }
+
+    // Candidates that joined an item go to `att`; returns which did.
+    std::vector<char> attach(const std::vector<LJob> &cand, const std::vector<LJob> &large, int64_t min_cap,
+                             std::vector<Att> &out) {
+        std::vector<char> gone(cand.size(), 0);
+        std::vector<int32_t> is256, tl, off{0}, req, soff{0}, sreq, ts;
+        int64_t cap = 0;
+        for (const LJob &j : large) {
+            is256.push_back(kind(rows(j)) == 3);
+            if (is256.back()) cap += up(rows(j), item_rows());
+            tl.push_back((int32_t)tiles(j));
+            req.insert(req.end(), groups[j.group].begin(), groups[j.group].end());
+            off.push_back((int32_t)req.size());
+        }
+        if (cand.empty() || cap == 0) return gone;
+        for (const LJob &j : cand) {
+            sreq.insert(sreq.end(), groups[j.group].begin(), groups[j.group].end());
+            soff.push_back((int32_t)sreq.size());
+            ts.push_back((int32_t)tiles(j));
+        }
+        const std::vector<int8_t> fixed(cand.size(), 0);
+        std::vector<int32_t> item(cand.size()), lrow(cand.size()), ij(cap), ir(cap), place(cap, -1);
+        int32_t n = 0;
+        if (tp_attach_tails((int32_t)large.size(), is256.data(), tl.data(), off.data(), req.data(), (int32_t)group(),
+                            (int32_t)cand.size(), soff.data(), sreq.data(), ts.data(), fixed.data(), nreq,
+                            (int32_t)o[9], (int32_t)o[10], (int32_t)item_rows(), (int32_t)min_cap, item.data(),
+                            lrow.data(), ij.data(), ir.data(), &n))
+            return gone;
+        for (size_t s = 0; s < cand.size(); ++s) {
+            if (item[s] < 0) continue;
+            gone[s] = 1;
+            int32_t &at = place[item[s]];
+            if (at < 0) {
+                at = (int32_t)out.size();
+                out.push_back({ij[item[s]], ir[item[s]], {}});
+            }
+            out[at].segs.push_back({cand[s], lrow[s]});
+        }
+        return gone;
+    }
+
+    Lowered lower(const std::vector<LJob> &small, const std::vector<LJob> &large, int64_t min_tiles) {
+        static const int64_t tile_of[4] = {0, 64, 128, 256};
+        Lowered r;
+        r.large = recut(
+            large, [&](const LJob &j) { return up(rows(j), tile_of[kind(rows(j))]) * kvheads(); }, o[5],
+            [&](size_t i) { return growing(large[i]); }, min_tiles, o[5] / 2, true, false);
+        std::stable_sort(r.large.begin(), r.large.end(), [&](const LJob &a, const LJob &b) {
+            return a.t0 != b.t0 ? a.t0 < b.t0 : groups[a.group][0] < groups[b.group][0];
+        });
+        r.small = small;
+        if (!o[3]) return r;
+        std::vector<LJob> cand = small;
+        std::vector<size_t> mids;
+        for (size_t i = 0; i < r.large.size(); ++i)
+            if (rows(r.large[i]) <= o[10]) {
+                mids.push_back(i);
+                cand.push_back(r.large[i]);
+            }
+        std::vector<char> gone = attach(cand, r.large, o[11], r.att);
+        bool launch = false;  // the small-job kernel launches anyway
+        for (size_t s = 0; s < cand.size(); ++s) launch |= !gone[s] && rows(cand[s]) <= 16;
+        if (launch) {
+            r.att.clear();
+            gone = attach(cand, r.large, 0, r.att);
+        }
+        r.small.clear();
+        for (size_t s = 0; s < cand.size(); ++s)
+            if (!gone[s] && rows(cand[s]) <= 16) r.small.push_back(cand[s]);
+        std::vector<int32_t> place(r.large.size(), 0);
+        for (size_t m = 0; m < mids.size(); ++m)
+            if (gone[small.size() + m]) place[mids[m]] = -1;
+        std::vector<LJob> stay;
+        for (size_t i = 0; i < r.large.size(); ++i)
+            if (place[i] == 0) {
+                place[i] = (int32_t)stay.size();
+                stay.push_back(r.large[i]);
+            }
+        r.large.swap(stay);
+        for (Att &a : r.att) a.job = place[a.job];
+        return r;
+    }
+
+    Lowered lowering(int64_t min_tiles, int &fill) {
+        Lowered r = lower(small0, large0, min_tiles);
+        const int64_t per64 = 64 / group(), limit = o[4];
+        bool wide = false, fits = true;
+        for (const LJob &j : large0)
+            if (rows(j) > 64) {
+                wide = true;
+                fits &= rows(j) <= limit;
+            }
+        bool any64 = false;
+        for (const LJob &j : r.large) any64 |= kind(rows(j)) == 1;
+        if (fill < 0) {
+            int64_t items = 0;
+            for (const LJob &j : r.large)
+                if (kind(rows(j)) == 3) items += up(rows(j), 256);
+            items *= kvheads();
+            bool one_tile = true;
+            for (const LJob &j : small0) one_tile &= tiles(j) <= 1;
+            fill = min_tiles == 1 && n_cu() / 4 < items && items <= n_cu() / 2 && one_tile;
+        }
+        if (limit && per64 && wide && fits && (any64 || fill)) {
+            std::vector<LJob> split, small = small0, large;
+            for (const LJob &j : large0) {
+                if (rows(j) > 64)
+                    slices(j, per64, split);
+                else
+                    split.push_back(j);
+            }
+            for (const LJob &j : split) (rows(j) <= 16 ? small : large).push_back(j);
+            r = lower(small, large, min_tiles);
+        }
+        if (!r.small.empty() && !routed.empty()) {
+            int64_t units = 0;
+            for (const LJob &j : routed) units += tiles(j);
+            if (units * kvheads() <= o[14]) {
+                r.small = small0;
+                r.small.insert(r.small.end(), routed.begin(), routed.end());
+                r.large.clear();
+                r.att.clear();
+            }
+        }
+        return r;
+    }
+
+    int kinds(const Lowered &r) const {
+        int k = r.small.empty() ? 0 : 1;
+        for (const LJob &j : r.large) k |= 2 << kind(rows(j));
+        return k;
+    }
+
+    void run(std::vector<LJob> in) {
+        if (o[15] > 0) fuse(in, o[15]);
+        for (const LJob &j : in) (rows(j) <= 16 ? small0 : large0).push_back(j);
+        const int64_t per = 16 / group();
+        if (per && !small0.empty())
+            for (const LJob &j : large0) slices(j, per, routed);
+        int fill = -1;
+        Lowered r = lowering(1, fill);
+        const int64_t min_tiles = o[6];
+        bool shorter = false;
+        for (const LJob &j : r.large) shorter |= j.n < min_tiles * quantum();
+        if (min_tiles > 1 && shorter) {
+            Lowered alt = lowering(min_tiles, fill);
+            if (kinds(alt) == kinds(r) && alt.small.size() <= r.small.size()) std::swap(r, alt);
+        }
+        std::vector<int32_t> owners(nreq, 0);
+        for (const LJob &j : r.small)
+            for (int32_t x : groups[j.group]) ++owners[x];
+        std::vector<char> keep(r.small.size(), 0);
+        int64_t longest = 0, tails = 0;
+        for (size_t i = 0; i < r.small.size(); ++i) {
+            const Reqs &g = groups[r.small[i].group];
+            if (g.size() != 1 || owners[g[0]] != 1) continue;
+            keep[i] = 1;
+            ++tails;
+            longest = std::max(longest, tiles(r.small[i]));
+        }
+        if (tails * kvheads() < n_cu() * (longest <= o[16] ? 1 : o[17])) std::fill(keep.begin(), keep.end(), 0);
+        const std::vector<LJob> small = r.small;
+        r.small = recut(
+            small, [&](const LJob &) { return kvheads(); }, o[12], [&](size_t i) { return growing(small[i]) || keep[i]; }, 1,
+            0, false, o[18] && r.large.empty());
+        small_jobs = (int32_t)r.small.size();
+        jobs = r.small;
+        jobs.insert(jobs.end(), r.large.begin(), r.large.end());
+        att = std::move(r.att);
+    }
+};
+
+}  // namespace
+
+extern "C" void *tp_lower(int32_t njobs, const int32_t *req_off, const int32_t *req, const int32_t *start,
+                          const int32_t *ntok, int32_t nreq, const int64_t *options, int32_t *sizes) {
+    if (njobs <= 0 || nreq <= 0 || !req_off || !req || !start || !ntok || !options || !sizes) return nullptr;
+    if (options[0] <= 0 || options[1] <= 0 || options[13] <= 0) return nullptr;
+    for (int32_t j = 0; j < njobs; ++j) {
+        if (req_off[j + 1] <= req_off[j] || ntok[j] <= 0 || start[j] < 0) return nullptr;
+        for (int32_t i = req_off[j]; i < req_off[j + 1]; ++i)
+            if (req[i] < 0 || req[i] >= nreq) return nullptr;
+    }
+    try {
+        std::unique_ptr<Lowering> l(new Lowering);
+        l->o = options;
+        l->nreq = nreq;
+        std::vector<Lowering::LJob> in(njobs);
+        for (int32_t j = 0; j < njobs; ++j)
+            in[j] = {l->intern(Lowering::Reqs(req + req_off[j], req + req_off[j + 1])), start[j], ntok[j]};
+        l->run(std::move(in));
+        l->o = nullptr;
+        int64_t greq = 0, segs = 0;
+        for (const auto &g : l->groups) greq += (int64_t)g.size();
+        for (const auto &a : l->att) segs += (int64_t)a.segs.size();
+        const int64_t total = 3 * (int64_t)l->jobs.size() + (int64_t)l->groups.size() + greq + 3 * (int64_t)l->att.size() + 4 * segs;
+        if (total > INT32_MAX) return nullptr;
+        const int64_t s[7] = {(int64_t)l->jobs.size(), l->small_jobs, (int64_t)l->groups.size(), greq,
+                              (int64_t)l->att.size(), segs, total};
+        for (int i = 0; i < 7; ++i) sizes[i] = (int32_t)s[i];
+        return l.release();
+    } catch (...) {  // out of memory: the caller's own code takes over
+        return nullptr;
+    }
+}
+
+extern "C" void tp_lower_take(void *handle, int32_t *out) {
+    std::unique_ptr<Lowering> l(static_cast<Lowering *>(handle));
+    if (!l || !out) return;
+    for (const auto &j : l->jobs) *out++ = j.group;
+    for (const auto &j : l->jobs) *out++ = j.t0;
+    for (const auto &j : l->jobs) *out++ = j.n;
+    for (const auto &g : l->groups) *out++ = (int32_t)g.size();
+    for (const auto &g : l->groups) out = std::copy(g.begin(), g.end(), out);
+    for (const auto &a : l->att) {
+        *out++ = a.job;
+        *out++ = a.row0;
+        *out++ = (int32_t)a.segs.size();
+    }
+    for (const auto &a : l->att)
+        for (const auto &s : a.segs) {
+            *out++ = s.job.group;
+            *out++ = s.job.t0;
+            *out++ = s.job.n;
+            *out++ = s.lrow;
+        }
 }

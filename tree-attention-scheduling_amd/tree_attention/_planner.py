@@ -13,13 +13,14 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
-from itertools import chain
+from array import array
+from itertools import accumulate, chain
 from pathlib import Path
 
 import numpy as np
 
 LIB_PATH = Path(__file__).with_name("libtree_plan.so")
-EXPORTS = ("tp_grouped_plan", "tp_attach_tails", "tp_build_metadata")
+EXPORTS = ("tp_grouped_plan", "tp_attach_tails", "tp_build_metadata", "tp_lower", "tp_lower_take")
 METHODS = {"greedy": 0, "cube": 1}
 
 _lib = None
@@ -52,6 +53,10 @@ def load(required: bool = True):
             lib.tp_build_metadata.restype = ctypes.c_int
             lib.tp_build_metadata.argtypes = [i32, i32, _p, _p, _p, _p, i32, i32, i32, i32, i32, _p, _p, _p, i32,
                                               _p, _p, ctypes.c_int64]
+            lib.tp_lower.restype = _p
+            lib.tp_lower.argtypes = [i32, _p, _p, _p, _p, i32, _p, _p]
+            lib.tp_lower_take.restype = None
+            lib.tp_lower_take.argtypes = [_p, _p]
             _lib = lib
     return _lib
 
@@ -61,7 +66,42 @@ def available() -> bool:
 
 
 def _ptr(a: np.ndarray):
-    return a.ctypes.data_as(_p)
+    return a.__array_interface__["data"][0]  # (an int: ctypes.data_as costs four times as much)
+
+
+def lower(jobs, nreq, options):
+    """``tp_lower`` over job objects: (jobs as (requests, first token, tokens) triples, small jobs,
+    attachments as ``(large job, first row, [(requests, first token, tokens, first job row)])``), or
+    ``None`` for arguments it does not take."""
+    lib = load()
+    off = array("i", accumulate((len(j.requests) for j in jobs), initial=0))
+    req = array("i", chain.from_iterable(j.requests for j in jobs))
+    start = array("i", (j.tokens[0] for j in jobs))
+    ntok = array("i", (len(j.tokens) for j in jobs))
+    opts = array("q", options)
+    sizes = array("i", bytes(28))
+    at = [a.buffer_info()[0] for a in (off, req, start, ntok, opts, sizes)]
+    handle = lib.tp_lower(len(jobs), at[0], at[1], at[2], at[3], nreq, at[4], at[5])
+    if not handle:
+        return None
+    n, small, n_groups, n_req, n_att, n_seg, total = sizes
+    out = array("i", bytes(4 * total))
+    lib.tp_lower_take(handle, out.buffer_info()[0])
+    o = out.tolist()
+    p = 3 * n
+    groups, q = [], p + n_groups
+    for size in o[p:q]:
+        groups.append(tuple(o[q:q + size]))
+        q += size
+    triples = [(groups[g], t0, k) for g, t0, k in zip(o[:n], o[n:2 * n], o[2 * n:p])]
+    att, s = [], q + 3 * n_att
+    for i in range(q, q + 3 * n_att, 3):
+        segs = []
+        for _ in range(o[i + 2]):
+            segs.append((groups[o[s]], o[s + 1], o[s + 2], o[s + 3]))
+            s += 4
+        att.append((o[i], o[i + 1], segs))
+    return triples, small, att
 
 
 def grouped_decisions(tree, method: str, model, qheads: int, kvheads: int, dim: int, node_runs):
@@ -72,29 +112,22 @@ def grouped_decisions(tree, method: str, model, qheads: int, kvheads: int, dim: 
     lib = load()
     nodes = tree.nodes
     n = len(nodes)
-    parent = np.fromiter((nd.parent for nd in nodes), dtype=np.int32, count=n)
-    child_off = np.zeros(n + 1, dtype=np.int32)
-    np.cumsum([len(nd.children) for nd in nodes], out=child_off[1:])
-    child_idx = np.fromiter((c for nd in nodes for c in nd.children), dtype=np.int32, count=int(child_off[-1]))
-    nreq = np.fromiter((len(nd.requests) for nd in nodes), dtype=np.int32, count=n)
-    run_off = np.zeros(n + 1, dtype=np.int64)
-    np.cumsum([len(r) for r in node_runs], out=run_off[1:])
-    flat = np.array([x for r in node_runs for run in r for x in run], dtype=np.int64).reshape(-1, 2)
-    run_start = np.ascontiguousarray(flat[:, 0]) if len(flat) else np.zeros(1, np.int64)
-    run_len = np.ascontiguousarray(flat[:, 1]) if len(flat) else np.zeros(1, np.int64)
-    fparams = np.array([model.bandwidth, model.cube_flops, model.task_us, model.merge_us], dtype=np.float64)
-    iparams = np.array([model.cube_rows, model.key_tile, model.kv_split, model.max_query_rows,
-                        qheads, kvheads, dim], dtype=np.int64)
-    pushed = np.zeros(n, dtype=np.int8)
-    total = np.zeros(1, dtype=np.float64)
-    if len(child_idx) == 0:
-        child_idx = np.zeros(1, dtype=np.int32)
-    rc = lib.tp_grouped_plan(METHODS[method], n, _ptr(parent), _ptr(child_off), _ptr(child_idx), _ptr(nreq),
-                             _ptr(run_off), _ptr(run_start), _ptr(run_len), _ptr(fparams), _ptr(iparams),
-                             _ptr(pushed), _ptr(total))
+    parent = array("i", [nd.parent for nd in nodes])
+    child_off = array("i", accumulate((len(nd.children) for nd in nodes), initial=0))
+    child_idx = array("i", [c for nd in nodes for c in nd.children] or [0])
+    nreq = array("i", [len(nd.requests) for nd in nodes])
+    run_off = array("q", accumulate(map(len, node_runs), initial=0))
+    run_start = array("q", [s for runs in node_runs for s, _ in runs] or [0])
+    run_len = array("q", [k for runs in node_runs for _, k in runs] or [0])
+    fparams = array("d", (model.bandwidth, model.cube_flops, model.task_us, model.merge_us))
+    iparams = array("q", (model.cube_rows, model.key_tile, model.kv_split, model.max_query_rows, qheads, kvheads, dim))
+    pushed = array("b", bytes(n))
+    total = array("d", (0.0,))
+    rc = lib.tp_grouped_plan(METHODS[method], n, *(a.buffer_info()[0] for a in (
+        parent, child_off, child_idx, nreq, run_off, run_start, run_len, fparams, iparams, pushed, total)))
     if rc != 0:
         raise ValueError(f"tp_grouped_plan rejected its arguments (code {rc})")
-    return pushed, float(total[0])
+    return pushed, total[0]
 
 
 def attach_tails(large, small, group, is256, large_tiles, small_tiles, fixed, nreq, xtail_max, wave_rows,

@@ -465,12 +465,12 @@ def _metadata_sections(njobs, maxr, nreq, maxs, n_rest, n_l256, attached, xstrid
 def _metadata_native(jobs, small_jobs, nreq, group, kvheads, tile_rows, attached, xstride):
     """The metadata sections through the host library (``tp_build_metadata``)."""
     from . import _planner
-    qlen = np.fromiter((len(j.requests) for j in jobs), dtype=np.int32, count=len(jobs))
-    req = np.fromiter(chain.from_iterable(j.requests for j in jobs), dtype=np.int32, count=int(qlen.sum()))
-    kstart = np.fromiter((j.tokens[0] for j in jobs), dtype=np.int32, count=len(jobs))
-    klen = np.fromiter((len(j.tokens) for j in jobs), dtype=np.int32, count=len(jobs))
-    att_job = np.fromiter((j + small_jobs for j, _ in attached), dtype=np.int32, count=len(attached))
-    att_row0 = np.fromiter((r0 for _, r0 in attached), dtype=np.int32, count=len(attached))
+    qlen = np.array([len(j.requests) for j in jobs], dtype=np.int32)
+    req = np.array(list(chain.from_iterable(j.requests for j in jobs)), dtype=np.int32)
+    kstart = np.array([j.tokens[0] for j in jobs], dtype=np.int32)
+    klen = np.array([len(j.tokens) for j in jobs], dtype=np.int32)
+    att_job = np.array([j + small_jobs for j, _ in attached], dtype=np.int32)
+    att_row0 = np.array([r0 for _, r0 in attached], dtype=np.int32)
     att_rec = np.zeros((len(attached), xstride), dtype=np.int32)
     for i, segs in enumerate(attached.values()):
         att_rec[i, :1 + XTAIL_FIELDS * len(segs)] = _xtail_record(segs, group)
@@ -564,55 +564,35 @@ def _metadata_numpy(jobs, small_jobs, nreq, group, kvheads, tile_rows, attached,
             "contiguous_q": contiguous_q, "slot_stride": slot_stride, "qbase": qbase}
 
 
-def prepare(plan: Plan, q: torch.Tensor, tile_rows: int = 256, fixed_from: int | None = None,
-            attach_tails: bool = True, route_items: int = ROUTE_ITEMS, fuse_rows: int = FUSE_ROWS,
-            consolidate_rows: int = CONSOLIDATE_ROWS, large_target: int | None = None,
-            small_target: int | None = None, large_min_tiles: int = LARGE_MIN_TILES) -> PreparedPlan:
-    """Lower ``plan`` to device metadata and scratch for queries shaped like ``q``.
+def _lower(jobs, nreq, n_cu, **options):
+    """``_lower_py`` through the host library (``tp_lower``) when it is built and takes the jobs;
+    both give the same jobs and attachments in the same order."""
+    from . import _planner
+    if _planner.available() and all(0 <= j.tokens[0] and j.tokens[0] + len(j.tokens) < 2 ** 31 for j in jobs):
+        o = options
+        got = _planner.lower(jobs, nreq, (
+            o["kvheads"], o["group"], o["tile_rows"], bool(o["attach_tails"]), o["consolidate_rows"], o["large_target"],
+            o["large_min_tiles"], n_cu, -1 if o["fixed_from"] is None else o["fixed_from"], XTAIL_MAX, WAVE_ROWS,
+            ATTACH_MIN_CAP, o["small_target"], TOKEN_QUANTUM, o["route_items"], o["fuse_rows"], TAIL_KEEP_TILES,
+            TAIL_KEEP_ITEMS_PER_CU, bool(SMALL_PAIRS)))
+        if got is not None:
+            triples, small_jobs, att = got
+            out, new, put = [], object.__new__, object.__setattr__
+            for reqs, t0, n in triples:
+                job = new(Job)
+                put(job, "requests", reqs)
+                put(job, "tokens", id_run(t0, t0 + n))
+                out.append(job)
+            return out, small_jobs, {(j, row0): [(Job(reqs, id_run(t0, t0 + n)), lrow) for reqs, t0, n, lrow in segs]
+                                     for j, row0, segs in att}
+    return _lower_py(jobs, n_cu, **options)
 
-    Mirrors kernels.py:103-141: physical jobs, stable small-first order, one
-    host-to-device copy of all int32 metadata, scratch allocated once.
-    ``tile_rows`` (64, 128 or 256) caps the query rows one workgroup of the
-    large-job kernels handles; it changes the work split, not the result.
-    Large jobs over the same token run that together hold at least ``fuse_rows``
-    query rows (0: never) run as one (``_fuse_same_tokens``).  Runs of jobs over one request group are re-cut for the
-    GPU (``_recut``), so ``jobs`` holds the execution jobs; ``fixed_from`` keeps jobs whose tokens
-    start at or after it (decode tails whose length changes) as they are.
-    ``attach_tails`` folds private single-request jobs into the 256-row work
-    items of the large jobs holding their request (``_attach_tails``); those
-    tails are then in ``attached``, not in ``jobs``.  When small jobs are left for
-    the small-job kernel and the large jobs, cut into 16-row request groups, stream
-    at most ``route_items`` (tile, KV head) units, the large jobs run as those
-    groups in the small-job kernel instead (one segment launch less).
-    ``large_target`` and ``small_target`` are the work items the re-cut aims at
-    for the large kinds and the small-job kind (default: one and eight per CU);
-    a large re-cut that would leave a few items for a second round takes the
-    next longer chunks when one round of them is shorter.
-    Large chunks of one tile are lengthened to ``large_min_tiles`` tiles when
-    that keeps the kernel kinds and the attachments and gives at least half of
-    ``large_target`` work items.  Jobs of at most ``consolidate_rows`` rows run
-    as 64-row request groups when 64-row items run anyway, or when their
-    256-row items would fill only a quarter to a half of the CUs and every
-    small job is one tile long (0: never).  Raises
-    ``ValueError`` for jobs without requests or tokens, request ids outside
-    ``q`` and token runs that are not consecutive physical ids.
-    """
-    if q.dim() != 3:
-        raise ValueError("q must be [requests, query heads, head dim]")
-    nreq, hq, dim = q.shape
-    kvheads = plan.settings["kvheads"]
-    if hq % kvheads:
-        raise ValueError("Query heads must be divisible by KV heads")
-    group = hq // kvheads
-    jobs = physical_jobs(plan.jobs)
-    for i, job in enumerate(jobs):
-        toks = job.tokens
-        if not job.requests or not toks:
-            raise ValueError("Every job needs requests and tokens")
-        if toks[0] < 0 or (len(toks) > 1 and toks != id_run(toks[0], toks[0] + len(toks))):
-            raise ValueError(f"Job {i} tokens are not one run of consecutive physical ids")
-    if not jobs:
-        raise ValueError("Plan has no jobs")
+
+def _lower_py(jobs, n_cu, *, kvheads, group, tile_rows, fixed_from, attach_tails, route_items, fuse_rows,
+              consolidate_rows, large_target, small_target, large_min_tiles):
+    """The execution jobs of a plan's physical jobs (see ``prepare``): (jobs, small ones first; how many
+    are small; attachments ``{(large job, first row): [(job, first job row)]}``, large jobs counted
+    from the first large one)."""
     if fuse_rows > 0:
         jobs = _fuse_same_tokens(jobs, group, fuse_rows)
     small = [j for j in jobs if len(j.requests) * group <= SMALL_ROWS]
@@ -621,9 +601,6 @@ def prepare(plan: Plan, q: torch.Tensor, tile_rows: int = 256, fixed_from: int |
     routed = [Job(j.requests[i:i + per], j.tokens) for j in large for i in range(0, len(j.requests), per)] \
         if per and small and large else []
     small0 = small
-    n_cu = _cu_count(q.device)
-    large_target = n_cu if large_target is None else large_target
-    small_target = 8 * n_cu if small_target is None else small_target
 
     def growing(job):
         return fixed_from is not None and job.tokens[0] >= fixed_from
@@ -634,7 +611,7 @@ def prepare(plan: Plan, q: torch.Tensor, tile_rows: int = 256, fixed_from: int |
                        * kvheads, large_target, growing, min_tiles, large_target // 2, one_round=True)
         # chunks of one token range side by side: a root split into request groups then gives
         # request r its k-th slot at r + k * (requests of a chunk), the layout the merge computes
-        large.sort(key=lambda j: (j.tokens[0], j.requests[0]))
+        large = sorted(large, key=lambda j: (j.tokens[0], j.requests[0]))
         attached = {}
         if attach_tails:  # growing tails too: their records' token fields are rewritten by fill_growing
             # candidates: the small jobs, then the large ones whose rows fit one wave
@@ -717,8 +694,65 @@ def prepare(plan: Plan, q: torch.Tensor, tile_rows: int = 256, fixed_from: int |
     keep = {id(j) for j in tails} if enough else set()
     small = _recut(small, lambda r: kvheads, small_target, lambda j: growing(j) or id(j) in keep,
                    pairs=SMALL_PAIRS and not large)
-    jobs = small + large
-    small_jobs = len(small)
+    return small + large, len(small), attached
+
+
+def prepare(plan: Plan, q: torch.Tensor, tile_rows: int = 256, fixed_from: int | None = None,
+            attach_tails: bool = True, route_items: int = ROUTE_ITEMS, fuse_rows: int = FUSE_ROWS,
+            consolidate_rows: int = CONSOLIDATE_ROWS, large_target: int | None = None,
+            small_target: int | None = None, large_min_tiles: int = LARGE_MIN_TILES) -> PreparedPlan:
+    """Lower ``plan`` to device metadata and scratch for queries shaped like ``q``.
+
+    Mirrors kernels.py:103-141: physical jobs, stable small-first order, one
+    host-to-device copy of all int32 metadata, scratch allocated once.
+    ``tile_rows`` (64, 128 or 256) caps the query rows one workgroup of the
+    large-job kernels handles; it changes the work split, not the result.
+    Large jobs over the same token run that together hold at least ``fuse_rows``
+    query rows (0: never) run as one (``_fuse_same_tokens``).  Runs of jobs over one request group are re-cut for the
+    GPU (``_recut``), so ``jobs`` holds the execution jobs; ``fixed_from`` keeps jobs whose tokens
+    start at or after it (decode tails whose length changes) as they are.
+    ``attach_tails`` folds private single-request jobs into the 256-row work
+    items of the large jobs holding their request (``_attach_tails``); those
+    tails are then in ``attached``, not in ``jobs``.  When small jobs are left for
+    the small-job kernel and the large jobs, cut into 16-row request groups, stream
+    at most ``route_items`` (tile, KV head) units, the large jobs run as those
+    groups in the small-job kernel instead (one segment launch less).
+    ``large_target`` and ``small_target`` are the work items the re-cut aims at
+    for the large kinds and the small-job kind (default: one and eight per CU);
+    a large re-cut that would leave a few items for a second round takes the
+    next longer chunks when one round of them is shorter.
+    Large chunks of one tile are lengthened to ``large_min_tiles`` tiles when
+    that keeps the kernel kinds and the attachments and gives at least half of
+    ``large_target`` work items.  Jobs of at most ``consolidate_rows`` rows run
+    as 64-row request groups when 64-row items run anyway, or when their
+    256-row items would fill only a quarter to a half of the CUs and every
+    small job is one tile long (0: never).  Raises
+    ``ValueError`` for jobs without requests or tokens, request ids outside
+    ``q`` and token runs that are not consecutive physical ids.
+    """
+    if q.dim() != 3:
+        raise ValueError("q must be [requests, query heads, head dim]")
+    nreq, hq, dim = q.shape
+    kvheads = plan.settings["kvheads"]
+    if hq % kvheads:
+        raise ValueError("Query heads must be divisible by KV heads")
+    group = hq // kvheads
+    jobs = physical_jobs(plan.jobs)
+    for i, job in enumerate(jobs):
+        toks = job.tokens
+        if not job.requests or not toks:
+            raise ValueError("Every job needs requests and tokens")
+        if toks[0] < 0 or (len(toks) > 1 and toks != id_run(toks[0], toks[0] + len(toks))):
+            raise ValueError(f"Job {i} tokens are not one run of consecutive physical ids")
+    if not jobs:
+        raise ValueError("Plan has no jobs")
+    n_cu = _cu_count(q.device)
+    large_target = n_cu if large_target is None else large_target
+    small_target = 8 * n_cu if small_target is None else small_target
+    jobs, small_jobs, attached = _lower(
+        jobs, nreq, n_cu, kvheads=kvheads, group=group, tile_rows=tile_rows, fixed_from=fixed_from,
+        attach_tails=attach_tails, route_items=route_items, fuse_rows=fuse_rows, consolidate_rows=consolidate_rows,
+        large_target=large_target, small_target=small_target, large_min_tiles=large_min_tiles)
     njobs = len(jobs)
     xstride = 1 + XTAIL_FIELDS * XTAIL_MAX
     from . import _planner
@@ -761,9 +795,11 @@ def prepare(plan: Plan, q: torch.Tensor, tile_rows: int = 256, fixed_from: int |
     # the token field of the attachment record of every item holding it when it is
     # attached.  fill_growing writes all of them with one device-side fill.
     offs = np.cumsum([0] + sizes)
-    grow = [int(offs[3]) + j for j, job in enumerate(jobs) if growing(job)]
+    grow = [int(offs[3]) + j for j, job in enumerate(jobs) if job.tokens[0] >= fixed_from] \
+        if fixed_from is not None else []
     if attached and fixed_from is not None:
-        slots_of = {key: [k for k, (job, _) in enumerate(segs) if growing(job)] for key, segs in keyed.items()}
+        slots_of = {key: [k for k, (job, _) in enumerate(segs) if job.tokens[0] >= fixed_from]
+                    for key, segs in keyed.items()}
         if any(slots_of.values()):
             k256 = 10 + _native.TA_LARGE256
             big = meta["buf"][offs[k256]:offs[k256 + 1]].reshape(-1, 3)

@@ -30,7 +30,7 @@ in the reference).
 """
 from __future__ import annotations
 
-from dataclasses import asdict, dataclass
+from dataclasses import asdict, dataclass, fields
 from itertools import chain
 from math import ceil
 
@@ -200,15 +200,33 @@ def schedule(tree: KVTree, qheads=32, kvheads=8, dim=128, method="cube", model=N
     kv_split = model.kv_split
     nodes = tree.nodes
 
+    new, put = object.__new__, object.__setattr__  # what the frozen dataclass's __init__ does
+
     def split(requests, tokens):
-        return [Job(tuple(requests[q:q + req_tile]), tuple(tokens[k:k + kv_split]))
-                for q in range(0, len(requests), req_tile)
-                for k in range(0, len(tokens), kv_split)]
+        out = []
+        for q in range(0, len(requests), req_tile):
+            reqs = tuple(requests[q:q + req_tile])
+            for k in range(0, len(tokens), kv_split):
+                job = new(Job)
+                put(job, "requests", reqs)
+                put(job, "tokens", tuple(tokens[k:k + kv_split]))
+                out.append(job)
+        return out
+
+    # the reference's cost depends on the two counts alone: one evaluation per pair
+    by_counts = {} if type(model).cost is CostModel.cost else None
 
     def plan_cost(jobs):
         total = 0
         for job in physical_jobs(jobs):
-            total = total + model.cost(job.requests, job.tokens, qheads, kvheads, dim)
+            if by_counts is None:
+                total = total + model.cost(job.requests, job.tokens, qheads, kvheads, dim)
+                continue
+            counts = (len(job.requests), len(job.tokens))
+            cost = by_counts.get(counts)
+            if cost is None:
+                cost = by_counts[counts] = model.cost(job.requests, job.tokens, qheads, kvheads, dim)
+            total = total + cost
         return total
 
     if method == "request":
@@ -219,7 +237,9 @@ def schedule(tree: KVTree, qheads=32, kvheads=8, dim=128, method="cube", model=N
         jobs = _grouped_jobs(tree, method, model, split, plan_cost, qheads, kvheads, dim, req_tile, native)
     else:
         raise ValueError(f"Unknown scheduling method: {method}")
-    settings = asdict(model)
+    settings = {f.name: getattr(model, f.name) for f in fields(model)}
+    if not all(type(x) in (int, float) for x in settings.values()):
+        settings = asdict(model)  # (a model with fields of its own)
     settings.update(qheads=qheads, kvheads=kvheads, head_dim=dim)
     return Plan(jobs, method, plan_cost(jobs), settings)
 
@@ -246,6 +266,7 @@ def _grouped_jobs(tree, method, model, split, plan_cost, qheads, kvheads, dim, r
             raise ValueError("the C++ planner covers the reference cost formula over increasing id chains only")
         if covered and (native or _planner.available()):
             pushed, _ = _planner.grouped_decisions(tree, method, model, qheads, kvheads, dim, all_runs)
+            pushed = pushed.tolist()
             return _materialise(nodes, split, lambda v, top: {c for c in nodes[v].children if pushed[c]})
 
     # --- token chains ------------------------------------------------------
@@ -395,8 +416,10 @@ def _materialise(nodes, split, pushed_of):
         v, top = todo.pop()
         node = nodes[v]
         pushed = pushed_of(v, top)
-        detached = {r for c in pushed for r in nodes[c].requests}
-        remaining = tuple(r for r in node.requests if r not in detached)
+        remaining = node.requests
+        if pushed:
+            detached = {r for c in pushed for r in nodes[c].requests}
+            remaining = tuple(r for r in node.requests if r not in detached)
         jobs.extend(split(remaining, chain_tokens(v, top)))
         ct = v if top is None else top
         for c in reversed(node.children):
