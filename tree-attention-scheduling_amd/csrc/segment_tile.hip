@@ -171,45 +171,69 @@ struct KTokens {
 // operands through registers with an 8 x 8 transpose took twice as long (24 ragged
 // requests in two branches, 10,839 tokens, d = 128: layer 49.2 us, here 26.7 us; 32
 // ragged requests, 1,745 tokens, d = 64: 14.2 us, here 8.4 us).
-template <int D, int NW, int L>
+constexpr int SHORT_CAP = 1 << 28;
+template <int D, int NW, int L, bool SHORT = false>
 struct TileCopy {
     using T = Tile<D>;
     static constexpr int NK = (T::KBLK + NW - 1) / NW;  // K blocks of a wave, V likewise (D = 32: of some waves)
     u32x4 k[L == KV_ODD ? NK : 1];
 
-    // V row t of head h
-    __device__ static const u16 *vrow(const SegParams &p, int h, int t) {
-        return p.vp + (L == KV_TOKEN ? (size_t)t * p.hk + h : (size_t)h * p.tcap + t) * D;
+    // SHORT: a copy's source is a scalar base per block plus a 32-bit lane offset that all tiles
+    // of an item share (8 K rows span 14 tcap bytes, so tcap <= SHORT_CAP); else a 64-bit address
+    // per lane.  In the one-wave kernel the short form streams 128 x 8192 private tokens in 768
+    // us against 782 us; in the mixed kernel, whose scalar registers are full, it is the slower
+    // one (32 requests x 4096 tokens: 42.8 us against 41.8 us).
+    __device__ static void dma(u16 *dst, const u16 *base, u32 ofs) {
+        __builtin_amdgcn_global_load_lds((const void *)((const char *)base + ofs), (lds_void *)dst, 16, 0, 0);
+    }
+
+    // Row t of head h of V (and of token-major K).
+    __device__ static const u16 *row(const u16 *x, const SegParams &p, int h, int t) {
+        return x + (L == KV_TOKEN ? (size_t)t * p.hk + h : (size_t)h * p.tcap + t) * D;
+    }
+    __device__ static u32 row_bytes(const SegParams &p) { return 2u * D * (L == KV_TOKEN ? p.hk : 1); }
+
+    // Row t0n + t of a tile, chunk s; `base`: a row of the tile that is the same for all lanes.
+    template <bool CLAMP>
+    __device__ static void copy_row(u16 *dst, const u16 *x, const SegParams &p, int h, int t0n, int kst, int kend,
+                                    int first, int j, int s) {
+        if constexpr (SHORT) {
+            const int from = CLAMP ? max(t0n, kst) : t0n + first;
+            const int r = CLAMP ? min(max(t0n + first + j, kst), kend - 1) - from : j;
+            dma(dst, row(x, p, h, from), r * row_bytes(p) + 16 * s);
+        } else {
+            const int t = t0n + first + j;
+            dma(dst, row(x, p, h, CLAMP ? min(max(t, kst), kend - 1) : t) + 8 * s, 0);
+        }
     }
 
     template <bool CLAMP>
     __device__ static void copy_v(u16 *st, const SegParams &p, int h, int t0n, int kst, int kend, int vb, int lane) {
         const int l = lane ^ (8 * ((T::KBLK + vb) & 1));  // logical slot filled by this lane (swizzle)
         const int rem = l % T::SV;
-        const int s = 2 * (l / T::SV) + ((rem >> 2) & 1);
-        const int j = 4 * (rem >> 3) + (rem & 3);
-        const int t = t0n + vb * T::VROWS + j;
-        const u16 *src = vrow(p, h, CLAMP ? min(max(t, kst), kend - 1) : t) + 8 * s;
-        __builtin_amdgcn_global_load_lds((const void *)src, (lds_void *)(st + (T::KBLK + vb) * T::BLK), 16, 0, 0);
+        copy_row<CLAMP>(st + (T::KBLK + vb) * T::BLK, p.vp, p, h, t0n, kst, kend, vb * T::VROWS,
+                        4 * (rem >> 3) + (rem & 3), 2 * (l / T::SV) + ((rem >> 2) & 1));
     }
 
     template <bool CLAMP>
     __device__ static void copy_k(u16 *st, const SegParams &p, int h, int t0n, int kst, int kend, int blk, int lane) {
-        const u16 *src;
+        u16 *dst = st + blk * T::BLK;
         if constexpr (L == KV_TOKEN) {
             // row-major tile: lane i fills slot i, chunk (i % CPR) ^ f of token row i / CPR (KTokens)
-            const int j = lane / KTokens<D>::CPR, t = blk * T::VROWS + j;
-            const int s = (lane % KTokens<D>::CPR) ^ KTokens<D>::flip(t);
-            const int tok = t0n + t;
-            src = p.kp + ((size_t)(CLAMP ? min(max(tok, kst), kend - 1) : tok) * p.hk + h) * D + 8 * s;
+            const int j = lane / KTokens<D>::CPR;
+            copy_row<CLAMP>(dst, p.kp, p, h, t0n, kst, kend, blk * T::VROWS, j,
+                            (lane % KTokens<D>::CPR) ^ KTokens<D>::flip(blk * T::VROWS + j));
         } else {
             const int l = lane ^ (8 * (blk & 1));
-            const int ck = 2 * (l >> 4) + ((l >> 2) & 1);
-            const int d = 8 * blk + 4 * ((l >> 3) & 1) + (l & 3);
-            const int tok = t0n + 8 * ck;
-            src = p.kp + (size_t)(h * D + d) * p.tcap + (CLAMP ? min(tok, p.tcap - 8) : tok);
+            const int tok = 8 * (2 * (l >> 4) + ((l >> 2) & 1));
+            const int j = 4 * ((l >> 3) & 1) + (l & 3);
+            const int last = p.tcap - 8;  // (a tile starts inside the pool, at a multiple of 8 like its capacity)
+            if constexpr (SHORT)
+                dma(dst, p.kp + (size_t)(h * D + 8 * blk) * p.tcap + t0n,
+                    2u * ((u32)j * (u32)p.tcap + (u32)(CLAMP ? min(tok, last - t0n) : tok)));
+            else
+                dma(dst, p.kp + (size_t)(h * D + 8 * blk + j) * p.tcap + (CLAMP ? min(t0n + tok, last) : t0n + tok), 0);
         }
-        __builtin_amdgcn_global_load_lds((const void *)src, (lds_void *)(st + blk * T::BLK), 16, 0, 0);
     }
 
     template <bool CLAMP>
@@ -337,11 +361,13 @@ struct TileMath {
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                // block 4*ks + g4, chunk pair base/16 + b, block rows 0-3 / 4-7
-                const int e = 4 * T::BLK * ks + 8 * (base + 16 * b);
-                kf[b][ks] = tr_pair(cur + of.klo + e, cur + of.khi + e);
-            }
+            for (int ks = 0; ks < KS; ++ks) kf[b][ks] = k_pair(cur, of, base, b, ks);
+    }
+
+    // one of them (not KV_TOKEN): block 4*ks + g4, chunk pair base/16 + b, block rows 0-3 / 4-7
+    __device__ static u32x4 k_pair(const u16 *__restrict__ cur, const LdsOfs &of, int base, int b, int ks) {
+        const int e = 4 * T::BLK * ks + 8 * (base + 16 * b);
+        return tr_pair(cur + of.klo + e, cur + of.khi + e);
     }
 
     // KV_TOKEN: the chunks at LDS byte addresses a[ks] and 16 tokens further.  For
@@ -379,10 +405,13 @@ struct TileMath {
     __device__ static void load_v(const u16 *__restrict__ st, const LdsOfs &of, int base, u32x4 (&v)[DB]) {
         const u16 *vrow = st + T::BLK * (T::KBLK + base / T::VROWS);
 #pragma unroll
-        for (int db = 0; db < DB; ++db) {
-            const u16 *va = vrow + 8 * T::SV * db;
-            v[db] = tr_pair(va + of.vlo[db & 1], va + of.vhi[db & 1]);
-        }
+        for (int db = 0; db < DB; ++db) v[db] = v_pair(vrow, of, db);
+    }
+
+    // one of them; vrow: the stage's first V block of the step
+    __device__ static u32x4 v_pair(const u16 *__restrict__ vrow, const LdsOfs &of, int db) {
+        const u16 *va = vrow + 8 * T::SV * db;
+        return tr_pair(va + of.vlo[db & 1], va + of.vhi[db & 1]);
     }
 
     // S^T = K Q^T: s[nb][b] holds tokens base+16b+4*g4+i of row block nb.
@@ -497,12 +526,12 @@ __device__ inline void item_barrier() {
 // One work item (job, first row, KV head) of the tile kernels: NW waves, NB
 // 16-row blocks per wave, STAGES LDS stages at `lds`.  The item holds rows
 // [row0, row0 + item_rows) of its job.  SOLO: one wave alone (tid = its lane).
-template <int D, bool FP16, int NB, int NW, int STAGES, int L, bool SOLO = false>
+template <int D, bool FP16, int NB, int NW, int STAGES, int L, bool SOLO = false, bool SHORT = false>
 __device__ __forceinline__ void tile_item(const SegParams &p, const int32_t *__restrict__ items, int item,
                                           u16 *lds, int tid, int item_rows) {
     using T = Tile<D>;
     using M = TileMath<D, FP16, NB, NW, L>;
-    using C = TileCopy<D, NW, L>;
+    using C = TileCopy<D, NW, L, SHORT>;
     constexpr int KS = M::KS;
     constexpr int BPW = T::NBLK / NW;  // copies per wave per tile
     static_assert(T::NBLK % NW == 0, "every wave copies the same number of blocks");
@@ -613,8 +642,8 @@ __device__ __forceinline__ void tile_item(const SegParams &p, const int32_t *__r
 }
 
 constexpr int ONE_ROUND = 5 * 256;  // one-wave workgroups that run at once at d = 128 (five 32 KiB tiles per CU)
-template <int D, bool FP16, int NB, int NW, int STAGES, int L>
-__global__ __launch_bounds__(64 * NW) void seg_tile_kernel(SegParams p) {
+template <int D, bool FP16, int NB, int NW, int STAGES, int L, bool SHORT = false>
+__global__ __launch_bounds__(64 * NW) void seg_tile_kernel(const int32_t *items, SegParams p) {
     __shared__ __attribute__((aligned(16))) u16 lds[STAGES * Tile<D>::ELEMS];
     // One-wave items lie job by job with the KV heads inside: with item i on XCD i % 8 an
     // XCD works on one head of 8 and translates and caches an eighth of the pools.  That
@@ -623,7 +652,7 @@ __global__ __launch_bounds__(64 * NW) void seg_tile_kernel(SegParams p) {
     // 8192 private tokens: 793 us by heads, 781 us by jobs).
     const bool by_head = NW == 1 && p.hk % 8 == 0 && gridDim.x <= ONE_ROUND;
     const int item = by_head ? blockIdx.x : xcd_item(blockIdx.x, gridDim.x);
-    tile_item<D, FP16, NB, NW, STAGES, L>(p, p.items, item, lds, threadIdx.x, 16 * NB * NW);
+    tile_item<D, FP16, NB, NW, STAGES, L, false, SHORT>(p, items, item, lds, threadIdx.x, 16 * NB * NW);
 }
 
 // ------------------------------------------------------------------------
@@ -637,8 +666,8 @@ __global__ __launch_bounds__(64 * NW) void seg_tile_kernel(SegParams p) {
 //                                          row maxima of step g+1
 //
 // and the rare online-softmax rescale runs between blocks.  The order inside
-// a block is pinned with sched_group_barrier so that MFMAs and VALU
-// instructions alternate in each wave's instruction stream.  K/V tiles arrive
+// a block is written out so that MFMAs, LDS reads and VALU instructions
+// alternate in each wave's instruction stream (see block()).  K/V tiles arrive
 // by LDS DMA into five stages: tiles t and t+1 are read while t+2 .. t+4 are
 // in flight, with one barrier per tile.
 template <int D, bool FP16, int NW, int NB_, int L>
@@ -726,15 +755,85 @@ struct PipeMath {
     // ks / kbase: of K(g+2) (any resident step when there is none); lo / hi:
     // valid tokens of step g+1.  Every fragment register set is reloaded only
     // after its last reader: V(g) during QK(g+1), K(g+2) during PV(g).
+    //
+    // With MORE the order is written out, one matrix instruction per slot, and each
+    // slot is closed by a sched_barrier: left to the compiler, sched_group_barrier
+    // or not, all 16 K reads ended up behind the PV MFMAs and all V reads behind
+    // half of QK's, so that every wave waited for LDS twice per step, all eight at
+    // once (root kernel at 128 x 8192 28.1 -> 27.5 us by dispatch stamps).  What is
+    // left per 64-token tile, 2.27 us on random data, is the matrix cores' own 1.36
+    // us (that loop without copies, barrier, LDS reads and exponentials) plus about
+    // 0.4 us each for the tile's copies and the LDS reads, 0.15 us each for the
+    // exponentials and the barrier.
     template <bool MORE, bool MASKN, bool ROWMASK = false>
     __device__ __forceinline__ void block(const u16 *__restrict__ vs, int vbase, const u16 *__restrict__ ks,
                                           int kbase, const u32x4 (&qf)[NB][KS], const LdsOfs &of, int lo,
                                           int hi, int g4, float c, unsigned keep = ~0u) {
         const u32x4 ones = {O::ONE2, O::ONE2, O::ONE2, O::ONE2};
-        f32x4 sn[NB][2];
-        if (MORE) TM::qk(kf, qf, sn);
-        TM::load_v(vs, of, vbase, vf);
         u32x4 pb[NB];
+        if constexpr (MORE) {
+            constexpr int NQ = 2 * KS * NB;      // MFMAs of QK
+            constexpr int EXPS = 8 * NB / NQ;    // exponentials per slot (1, 2, 4)
+            f32x4 sn[NB][2];
+            float pr[NB][8];
+            const u16 *vrow = vs + T::BLK * (T::KBLK + vbase / T::VROWS);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) {
+                const int k = i / (2 * NB), b = i / NB % 2, nb = i % NB;
+                sn[nb][b] = O::mma_k32(kf[b][k], qf[nb][k], k == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sn[nb][b]);
+                if (i < DB) vf[i] = TM::v_pair(vrow, of, i);
+#pragma unroll
+                for (int e = i * EXPS; e < (i + 1) * EXPS; ++e) {
+                    const int n = e / 8, x = e % 8;
+                    pr[n][x] = fast_exp2(__builtin_fmaf(s[n][x >> 2][x & 3], c, -m[n]));
+                    if (x == 7)
+                        pb[n] = u32x4{O::pack(pr[n][0], pr[n][1]), O::pack(pr[n][2], pr[n][3]),
+                                      O::pack(pr[n][4], pr[n][5]), O::pack(pr[n][6], pr[n][7])};
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // V has landed by now; waited for here, the K reads below stay in flight behind PV
+            __builtin_amdgcn_s_waitcnt(TA_LGKMCNT0);
+            // the next step's maxima, two scores at a time, in the slots after the K reads
+            constexpr int NP = DB * NB, FROM = NP > 4 * NB ? NP - 4 * NB : 0;
+            float mx[NB];
+#pragma unroll
+            for (int j = 0; j < NP; ++j) {
+                const int db = j / NB, nb = j % NB;
+                o[nb][db] = O::mma_k32(vf[db], pb[nb], o[nb][db]);
+                if (L == KV_TOKEN ? j == 0 : j < 2 * KS) {
+                    if constexpr (L == KV_TOKEN)
+                        TM::load_k(ks, of, kbase, kf);
+                    else
+                        kf[j % 2][j / 2] = TM::k_pair(ks, of, kbase, j % 2, j / 2);
+                }
+                if (!MASKN && j >= FROM) {
+#pragma unroll
+                    for (int u = (j - FROM) * 4 * NB / (NP - FROM); u < (j - FROM + 1) * 4 * NB / (NP - FROM); ++u) {
+                        const int n = u % NB, x = 2 * (u / NB);
+                        const float a0 = sn[n][x >> 2][x & 3], a1 = sn[n][x >> 2][(x & 3) + 1];
+                        mx[n] = x == 0 ? fmaxf(a0, a1) : fmaxf(fmaxf(mx[n], a0), a1);
+                        asm volatile("" : "+v"(mx[n]));  // in this slot, not at its last use
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) z[nb] = O::mma_k32(ones, pb[nb], z[nb]);
+            if constexpr (MASKN) {
+                finish_scores<true>(sn, lo, hi, g4);
+            } else {
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) {
+                    lm[nb] = mx[nb];
+                    s[nb][0] = sn[nb][0];
+                    s[nb][1] = sn[nb][1];
+                }
+            }
+            return;
+        }
+        TM::load_v(vs, of, vbase, vf);
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             float pr[8];
@@ -744,38 +843,12 @@ struct PipeMath {
                            O::pack(pr[6], pr[7])};
             if (ROWMASK && !((keep >> nb) & 1)) pb[nb] = u32x4{0u, 0u, 0u, 0u};
         }
-        if (MORE) {
-            // 2*KS*NB QK MFMAs; the V reads go out with the first half of them
-#pragma unroll
-            for (int i = 0; i < 2 * KS * NB; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-                if (i < DB) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // DS read
-                __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
-                __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);  // transcendental
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);  // K(g+1) is dead only after QK(g+1)
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) o[nb][db] = O::mma_k32(vf[db], pb[nb], o[nb][db]);
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) z[nb] = O::mma_k32(ones, pb[nb], z[nb]);
-        if (MORE) {
-            TM::load_k(ks, of, kbase, kf);
-            finish_scores<MASKN>(sn, lo, hi, g4);
-        }
-        // instruction order: QK MFMAs alternate with the exponentials and the
-        // V reads, then PV MFMAs alternate with the K reads and the score epilogue
-        if (MORE) {
-            // DB*NB PV MFMAs; the K reads go out with the first half of them
-#pragma unroll
-            for (int i = 0; i < DB * NB; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);  // MFMA
-                if (i < 2 * KS) __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);  // DS read
-                __builtin_amdgcn_sched_group_barrier(0x002, 1, 1);  // VALU
-            }
-        }
     }
 
     // One staged tile of an attached private segment (after the pipeline has
@@ -1074,9 +1147,9 @@ __device__ __forceinline__ void pipe_item_rows(const SegParams &p, const int32_t
 }
 
 template <int D, bool FP16, int NW, int L>
-__global__ __launch_bounds__(64 * NW) void seg_pipe_kernel(SegParams p) {
+__global__ __launch_bounds__(64 * NW) void seg_pipe_kernel(const int32_t *items, SegParams p) {
     __shared__ __attribute__((aligned(16))) u16 lds[TA_PIPE_STAGES * Tile<D>::ELEMS];
-    pipe_item_rows<D, FP16, NW, L>(p, p.items, xcd_item(blockIdx.x, gridDim.x), lds, threadIdx.x);
+    pipe_item_rows<D, FP16, NW, L>(p, items, xcd_item(blockIdx.x, gridDim.x), lds, threadIdx.x);
 }
 
 // Work items of several kinds of one layer in one launch of 512-thread
@@ -1092,23 +1165,24 @@ __global__ __launch_bounds__(64 * NW) void seg_pipe_kernel(SegParams p) {
 // 26.2 -> 25.1 us); beside 256-row items, which fill whole CUs by head already,
 // four neighbours share a workgroup (by head 0.1-0.5 us slower on two layers).
 template <int D, bool FP16, int L>
-__global__ __launch_bounds__(512) void seg_mix_kernel(MixParams mp) {
+__global__ __launch_bounds__(512) void seg_mix_kernel(const int32_t *items0, const int32_t *items1, const int32_t *items2,
+                                                      MixParams mp) {
     using T = Tile<D>;
     __shared__ __attribute__((aligned(16))) u16 lds[TA_PIPE_STAGES * T::ELEMS];
     static_assert(TA_PIPE_STAGES >= 4 && 3 <= TA_PIPE_STAGES, "four small stages and three 64-row stages fit");
     const int b = blockIdx.x, tid = threadIdx.x;
     if (b < mp.base[1]) {
         if (b >= mp.n[0]) return;
-        pipe_item_rows<D, FP16, 8, L>(mp.p, mp.items[0], xcd_item(b, mp.n[0]), lds, tid);
+        pipe_item_rows<D, FP16, 8, L>(mp.p, items0, xcd_item(b, mp.n[0]), lds, tid);
     } else if (b < mp.base[2]) {
         const int lb = b - mp.base[1];
         if (lb >= mp.n[1]) return;
-        tile_item<D, FP16, 1, 8, 3, L>(mp.p, mp.items[1], xcd_item(lb, mp.n[1]), lds, tid, 64);
+        tile_item<D, FP16, 1, 8, 3, L>(mp.p, items1, xcd_item(lb, mp.n[1]), lds, tid, 64);
     } else {
         const int lb = b - mp.base[2], wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int it = mp.n[0] ? 4 * lb + wave : 8 * (4 * (lb >> 3) + wave) + (lb & 7);
         if (wave >= 4 || it >= mp.n[2]) return;
-        tile_item<D, FP16, 1, 1, 1, L, true>(mp.p, mp.items[2], it, lds + wave * T::ELEMS, tid & 63, 16);
+        tile_item<D, FP16, 1, 1, 1, L, true>(mp.p, items2, it, lds + wave * T::ELEMS, tid & 63, 16);
     }
 }
 
@@ -1277,16 +1351,20 @@ hipError_t launch_d(const SegParams &sp, int kind, hipStream_t stream) {
             if (sp.out) return launch_tail_merge<D, FP16, L>(sp, stream);
             [[fallthrough]];
         case TA_SMALL:  // one wave per (job, head); one stage so that five fit on a CU
-            TA_LAUNCH((seg_tile_kernel<D, FP16, 1, 1, 1, L>), dim3(sp.n_items), dim3(64), stream, sp);
+            if (L != KV_ODD && sp.tcap <= SHORT_CAP)
+                TA_LAUNCH((seg_tile_kernel<D, FP16, 1, 1, 1, L, L != KV_ODD>), dim3(sp.n_items), dim3(64), stream,
+                          sp.items, sp);
+            else
+                TA_LAUNCH((seg_tile_kernel<D, FP16, 1, 1, 1, L>), dim3(sp.n_items), dim3(64), stream, sp.items, sp);
             break;
         case TA_LARGE64:
-            TA_LAUNCH((seg_tile_kernel<D, FP16, 1, 4, 3, L>), dim3(sp.n_items), dim3(256), stream, sp);
+            TA_LAUNCH((seg_tile_kernel<D, FP16, 1, 4, 3, L>), dim3(sp.n_items), dim3(256), stream, sp.items, sp);
             break;
         case TA_LARGE128:
-            TA_LAUNCH((seg_tile_kernel<D, FP16, 2, 4, 3, L>), dim3(sp.n_items), dim3(256), stream, sp);
+            TA_LAUNCH((seg_tile_kernel<D, FP16, 2, 4, 3, L>), dim3(sp.n_items), dim3(256), stream, sp.items, sp);
             break;
         case TA_LARGE256:
-            TA_LAUNCH((seg_pipe_kernel<D, FP16, 8, L>), dim3(sp.n_items), dim3(512), stream, sp);
+            TA_LAUNCH((seg_pipe_kernel<D, FP16, 8, L>), dim3(sp.n_items), dim3(512), stream, sp.items, sp);
             break;
         default:
             return (hipError_t)TA_ERR_ARG;
@@ -1296,7 +1374,7 @@ hipError_t launch_d(const SegParams &sp, int kind, hipStream_t stream) {
 
 template <int D, bool FP16, int L>
 hipError_t launch_mix_d(const MixParams &mp, int blocks, hipStream_t stream) {
-    TA_LAUNCH((seg_mix_kernel<D, FP16, L>), dim3(blocks), dim3(512), stream, mp);
+    TA_LAUNCH((seg_mix_kernel<D, FP16, L>), dim3(blocks), dim3(512), stream, mp.items[0], mp.items[1], mp.items[2], mp);
     return hipGetLastError();
 }
 
