@@ -125,3 +125,31 @@ def test_one_wave_items_in_any_order(small, hk, device):
         ref = request_attention(q.float(), k.float(), v.float(), KVTree([], [tuple(x) for x in paths]))
         torch.testing.assert_close(out, ref.bfloat16(), atol=0.008, rtol=0.03)
         assert relative_l2(out, ref) <= 3e-3
+
+
+@pytest.mark.parametrize("d,hq,hk,dtype", [(128, 32, 8, torch.bfloat16), (64, 8, 2, torch.float16)])
+@pytest.mark.parametrize("n", [319, 320, 321, 384, 385, 449, 1000])
+def test_copies_spread_over_steps(n, d, hq, hk, dtype, device):
+    """256-row items of packed pools from just under five whole tiles (the ring) on: the loop that
+    starts a tile's copies inside the steps (pools) gives the bits of the one that starts them behind
+    the barrier (token-major), at starts on and off a tile chunk, with idle waves, with attachments."""
+    g = torch.Generator().manual_seed(n)
+    for start, nreq, attach in ((0, 64, False), (3, 70, False), (8, 66, True), (16, 34, False)):
+        jobs = [Job(tuple(range(nreq)), tuple(range(start, start + n)))]
+        base = start + n + 5
+        jobs += [Job((r,), tuple(range(base + 20 * r, base + 20 * r + 9 + r % 11))) for r in range(nreq)]
+        t = -(-(base + 20 * nreq) // 8) * 8
+        q = torch.randn(nreq, hq, d, generator=g).to(dtype)
+        k = torch.randn(t, hk, d, generator=g).to(dtype)
+        v = torch.randn(t, hk, d, generator=g).to(dtype)
+        qd, kd, vd = q.to(device), k.to(device), v.to(device)
+        p = prepare(Plan(jobs, "x", 0.0, dict(kvheads=hk)), qd, route_items=0, consolidate_rows=0, large_target=1,
+                    attach_tails=attach)
+        say("spread", n, start, nreq, list(p.abi.n_items), len(p.attached))
+        assert p.abi.n_items[_native.TA_LARGE256]
+        out = attention_matrix(qd, *pack_kv(kd, vd), p).cpu()
+        assert torch.equal(out, attention(qd, kd, vd, p).cpu())
+        paths = [sum((list(j.tokens) for j in jobs if r in j.requests), []) for r in range(nreq)]
+        ref = request_attention(q.float(), k.float(), v.float(), KVTree([], [tuple(x) for x in paths]))
+        torch.testing.assert_close(out, ref.to(dtype), atol=0.008, rtol=0.03)
+        assert relative_l2(out, ref) <= 3e-3

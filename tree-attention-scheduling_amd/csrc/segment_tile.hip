@@ -193,6 +193,19 @@ struct TileCopy {
     }
     __device__ static u32 row_bytes(const SegParams &p) { return 2u * D * (L == KV_TOKEN ? p.hk : 1); }
 
+    // Byte offsets of this lane's 16 bytes in a KV_POOL tile's copies of wave w from the first
+    // row of the block copied: K block w + n NW, and V block w + n NW (NW and KBLK even, so
+    // that a block's parity, which the swizzle follows, is w's).
+    __device__ static u32 k_offset(const SegParams &p, int w, int lane) {
+        const int l = lane ^ (8 * (w & 1));
+        return 2u * ((u32)(4 * ((l >> 3) & 1) + (l & 3)) * (u32)p.tcap + 8 * (2 * (l >> 4) + ((l >> 2) & 1)));
+    }
+    __device__ static u32 v_offset(int w, int lane) {
+        static_assert(NW % 2 == 0 || NW == 1, "one parity per wave");
+        const int l = lane ^ (8 * (w & 1)), rem = l % T::SV;
+        return 2u * ((4 * (rem >> 3) + (rem & 3)) * D + 8 * (2 * (l / T::SV) + ((rem >> 2) & 1)));
+    }
+
     // Row t0n + t of a tile, chunk s; `base`: a row of the tile that is the same for all lanes.
     template <bool CLAMP>
     __device__ static void copy_row(u16 *dst, const u16 *x, const SegParams &p, int h, int t0n, int kst, int kend,
@@ -760,15 +773,19 @@ struct PipeMath {
     // slot is closed by a sched_barrier: left to the compiler, sched_group_barrier
     // or not, all 16 K reads ended up behind the PV MFMAs and all V reads behind
     // half of QK's, so that every wave waited for LDS twice per step, all eight at
-    // once (root kernel at 128 x 8192 28.1 -> 27.5 us by dispatch stamps).  What is
-    // left per 64-token tile, 2.27 us on random data, is the matrix cores' own 1.36
+    // once (root kernel at 128 x 8192 28.1 -> 27.5 us by dispatch stamps).  What was
+    // left per 64-token tile, 2.27 us on random data, was the matrix cores' own 1.36
     // us (that loop without copies, barrier, LDS reads and exponentials) plus about
-    // 0.4 us each for the tile's copies and the LDS reads, 0.15 us each for the
-    // exponentials and the barrier.
-    template <bool MORE, bool MASKN, bool ROWMASK = false>
+    // 0.4 us each for the tile's copies, all sent behind the barrier, and the LDS
+    // reads, 0.15 us each for the exponentials and the barrier.
+    // `copy`, called with the slot's number, may start a copy of a later tile there.
+    struct NoCopy {
+        __device__ void operator()(int) const {}
+    };
+    template <bool MORE, bool MASKN, bool ROWMASK = false, class Copy = NoCopy>
     __device__ __forceinline__ void block(const u16 *__restrict__ vs, int vbase, const u16 *__restrict__ ks,
                                           int kbase, const u32x4 (&qf)[NB][KS], const LdsOfs &of, int lo,
-                                          int hi, int g4, float c, unsigned keep = ~0u) {
+                                          int hi, int g4, float c, unsigned keep = ~0u, Copy copy = Copy()) {
         const u32x4 ones = {O::ONE2, O::ONE2, O::ONE2, O::ONE2};
         u32x4 pb[NB];
         if constexpr (MORE) {
@@ -783,6 +800,7 @@ struct PipeMath {
                 const int k = i / (2 * NB), b = i / NB % 2, nb = i % NB;
                 sn[nb][b] = O::mma_k32(kf[b][k], qf[nb][k], k == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sn[nb][b]);
                 if (i < DB) vf[i] = TM::v_pair(vrow, of, i);
+                copy(i);
 #pragma unroll
                 for (int e = i * EXPS; e < (i + 1) * EXPS; ++e) {
                     const int n = e / 8, x = e % 8;
@@ -1070,6 +1088,45 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
     };
     // steady state: steps whose successor is neither the last nor masked
     int g = 0;
+    // ... and, while a whole tile is left to copy per tile attended, that tile's copies
+    // spread over the two steps: K's in the slots of the first, V's in those of the second,
+    // from a scalar base that the step selects and one lane offset each (8 K rows span
+    // 14 tcap bytes, see SHORT_CAP).  All eight waves used to send their four copies at
+    // once behind the barrier, with 64-bit lane addresses and the tests for a tile's place
+    // in the sequence (128 requests x 8192: kernel 27.6 -> 26.7 us, layer 34.1 -> 33.2 us;
+    // every 4th, 8th or 12th slot alike; the branch per tile instead of per loop spilled
+    // 590 registers).  Items of fewer than STAGES whole tiles stay with the loop below.
+    constexpr int NH = T::KBLK / NW;  // copies of K, and of V, of one wave
+    if constexpr (L == KV_POOL && SYNC == 1 && T::KBLK % NW == 0 && NH * NW == T::VBLK) {
+        // (readfirstlane: a lane-dependent branch here would move `issued` to vector registers)
+        if (__builtin_amdgcn_readfirstlane(active) && p.tcap <= SHORT_CAP && tb0 + STAGES * T::TT <= kend) {
+            constexpr int EVERY = 4;  // slots from one copy to the next
+            static_assert(EVERY * NH <= 2 * KS * NB, "the copies fit the step's QK slots");
+            const int w = __builtin_amdgcn_readfirstlane(wave);
+            const u32 kofs = C::k_offset(p, w, lane), vofs = C::v_offset(w, lane);
+            const u16 *kb = p.kp + (size_t)(h * D + 8 * w) * p.tcap + tb0;
+            const u16 *vb = p.vp + ((size_t)h * p.tcap + tb0 + w * T::VROWS) * D;
+            for (; issued < STAGES - 1; ++issued) copy_tile(issued, tile_stage(issued));
+            for (; tb0 + ((g >> 1) + STAGES) * T::TT <= kend; ++g) {
+                const int nt = (g >> 1) + STAGES - 1, odd = g & 1;  // nt: tile copied, inside the job
+                if (!odd) {
+                    wait_tiles<BPW>(STAGES - 3);  // tile (g >> 1) + 1 landed
+                    __builtin_amdgcn_s_barrier();
+                    ++issued;
+                }
+                const u16 *src = odd ? vb + (size_t)nt * (T::TT * D) : kb + nt * T::TT;
+                const size_t next = odd ? (size_t)NW * T::VROWS * D : (size_t)8 * NW * p.tcap;
+                const u32 ofs = odd ? vofs : kofs;
+                u16 *dst = tile_stage(nt) + (odd ? T::KBLK + w : w) * T::BLK;
+                acc.template block<true, false, false>(
+                    stage(g), 32 * odd, stage(g + 2), 32 * odd, qf, of, 0, 32, g4, c, ~0u, [&](int slot) {
+                        const int n = slot / EVERY;
+                        if (slot % EVERY == EVERY / 2 && n < NH) C::dma(dst + n * NW * T::BLK, src + n * next, ofs);
+                    });
+                acc.rescale(c, rc);
+            }
+        }
+    }
     for (; g + 2 < nsteps; ++g) {
         if (!(g & 1)) sync_tile(g >> 1);
         if (active) {
