@@ -14,8 +14,9 @@
 //    x 64 tokens each) and D/8 of V, each copied by one wave with one
 //    global_load_lds_dwordx4 (lane i fills bytes 16i..16i+15 of the block).
 //    Three LDS stages keep two tiles in flight while one is computed (one-wave
-//    workgroups of small jobs use one stage, so that four share a CU); each wave waits for its own copies with s_waitcnt vmcnt
-//    and the waves meet at one barrier per tile.
+//    workgroups of small jobs use one stage, so that five fit a CU); each wave
+//    waits for its own copies with s_waitcnt vmcnt and the waves meet at one
+//    barrier per tile.
 //  * The lane -> 16-byte-chunk assignment inside a block is chosen so that the
 //    eight chunks one 16-lane group reads together are 128 contiguous bytes,
 //    and odd blocks swap the two 128-byte halves of every 256 bytes so that
