@@ -149,7 +149,9 @@ int ta_merge(const void *part, const float *lse, const int32_t *slots,
 /* One decode-step attention layer on resident pools (replaces attention_matrix,
  * kernels.py:152-168): the large-job segment launches, the small-job launch,
  * the TA_TAIL launch that merges the requests owning a tail job, and the merge
- * of the remaining requests (`rest`). */
+ * of the remaining requests (`rest`).  Pools whose capacity is not a multiple
+ * of 8 take the unfused order: every segment kind, then the merge of all
+ * requests. */
 int ta_attention_matrix(const void *q, const void *kp, const void *vp,
                         int32_t tcap, const ta_plan *plan, void *out, void *stream);
 

@@ -8,6 +8,8 @@ edges: capacities below one 8-token chunk, last tiles that end with the pool,
 jobs that start anywhere.  Bars as in test_gpu_parity (0.3 % relative L2 against
 the FP32 oracle, atol .008 / rtol .03).
 """
+import math
+
 import pytest
 import torch
 
@@ -70,6 +72,63 @@ def test_any_capacity_and_token_major(name, hq, hk, d, dtype, device):
         assert {_native.TA_LARGE64, _native.TA_LARGE128, _native.TA_LARGE256} <= kinds
     if name == "branches":
         assert {_native.TA_SMALL, _native.TA_LARGE64} <= kinds
+
+
+def _rounding_case(nreq, n, device):
+    """One job of ``nreq`` requests over ``n`` tokens whose probabilities lie between two bf16
+    values: one token scores 0, the others p = 0.5013, which bf16 rounds to 0.5."""
+    q = torch.zeros(nreq, 32, 128)
+    q[..., 0] = 8.0
+    k = torch.zeros(n, 8, 128)
+    k[1:, :, 0] = -0.9765625
+    p = math.exp(-8 * 0.9765625 / math.sqrt(128))
+    lse = math.log(1 + (n - 1) * p)
+    assert lse - math.log(1 + (n - 1) * float(torch.tensor(p).bfloat16())) > 1e-3  # what rounded P would give
+    jobs = [Job(tuple(range(nreq)), tuple(range(n)))]
+    return q.bfloat16().to(device), k.bfloat16().to(device), Plan(jobs, "x", 0.0, dict(kvheads=8)), lse
+
+
+@pytest.mark.parametrize("nreq,tile_rows,kind", [(3, 256, _native.TA_SMALL), (14, 256, _native.TA_LARGE64),
+                                                 (30, 128, _native.TA_LARGE128), (40, 256, _native.TA_LARGE256),
+                                                 (64, 256, _native.TA_LARGE256)])
+@pytest.mark.parametrize("n", [29, 197])
+def test_odd_capacity_sums_fp32_probabilities(n, nreq, tile_rows, kind, device):
+    """The log-sum-exp of pools of other capacities carries no rounding of the probabilities
+    (they are summed in FP32, as in the reference's kernel); 1e-4 is ten times what 197 FP32
+    additions and the exponential's last bit can move it."""
+    q, k, plan, lse = _rounding_case(nreq, n, device)
+    v = torch.randn(n, 8, 128, device=device).bfloat16()
+    prepared = prepare(plan, q, tile_rows=tile_rows, route_items=0, consolidate_rows=0, large_target=1, small_target=1)
+    say("fp32 sums", n, nreq, list(prepared.abi.n_items))
+    assert prepared.abi.n_items[kind] and len(prepared.jobs) == 1
+    attention_matrix(q, *pack_kv(k, v), prepared)
+    got = prepared.lse[..., 0].cpu()
+    assert (got - lse).abs().max() < 1e-4
+
+
+@pytest.mark.parametrize("n", [5, 45, 75, 333])
+@pytest.mark.parametrize("nreq", [2, 14, 40, 64])
+def test_odd_capacity_same_bits_in_every_kind(n, nreq, device):
+    """A row's result on pools of other capacities does not depend on the kind of work item it
+    is in, and an infinite value counts once (its row also pads the job's last tile)."""
+    g = torch.Generator().manual_seed(n)
+    q = torch.randn(nreq, 32, 128, generator=g).mul(4).bfloat16().to(device)
+    k = torch.randn(n, 8, 128, generator=g).bfloat16().to(device)
+    v = torch.randn(n, 8, 128, generator=g).bfloat16().to(device)
+    inf = v.clone()
+    inf[-1, :, 3] = float("inf")
+    plan = Plan([Job(tuple(range(nreq)), tuple(range(n)))], "x", 0.0, dict(kvheads=8))
+    outs, kinds = [], set()
+    for tile_rows in (64, 128, 256):
+        p = prepare(plan, q, tile_rows=tile_rows, route_items=0, consolidate_rows=0, large_target=1, small_target=1)
+        kinds |= {i for i in range(_native.TA_NKINDS) if p.abi.n_items[i]}
+        outs.append(attention_matrix(q, *pack_kv(k, v), p).clone())
+        attention_matrix(q, *pack_kv(k, inf), p)
+        assert not p.part.isnan().any() and int(p.part.isposinf().sum()) == nreq * 32
+    say("kinds", n, nreq, kinds)
+    assert all(torch.equal(outs[0], o) for o in outs[1:])
+    ref = request_attention(q.float().cpu(), k.float().cpu(), v.float().cpu(), KVTree([], [tuple(range(n))] * nreq))
+    assert relative_l2(outs[0].cpu(), ref) <= 3e-3
 
 
 def test_token_major_equals_packed(device):

@@ -33,7 +33,8 @@
 //    consecutive tokens of one query row, which is the B operand of the PV
 //    product O^T = V^T P^T, so P never leaves registers.
 //  * The softmax denominator is one more PV MFMA against an all-ones A
-//    operand, so z sums exactly the rounded P that multiplies V.
+//    operand, so z sums exactly the rounded P that multiplies V (RowSum; pools of
+//    other capacities sum the FP32 exponentials).
 //  * Softmax in base 2 with log2(e)/sqrt(D) folded into one FMA; lazy
 //    rescaling (the running maximum moves only by more than TAU).
 // The kernels are templates over the layout of K and V (enum Layout): pools whose
@@ -328,21 +329,70 @@ struct TileCopy {
     }
 };
 
+// The softmax denominator of a lane's row.  KV_POOL and KV_TOKEN: one more PV MFMA against
+// an all-ones A operand, so that it sums exactly the rounded P that multiplies V.  KV_ODD:
+// the FP32 exponentials themselves, each lane its own tokens, added over the four lanes of
+// the row at the end -- the log-sum-exp then carries no rounding of P.  Against the ones
+// product: 24 ragged requests in two branches, 10,839 tokens, 25.7 us (25.5); 128 requests x
+// 8192 in 256-row items, where the additions share the step's slots, 54.3 us (48.1).
+template <int L>
+struct RowSum {
+    static constexpr bool FP32 = L == KV_ODD;
+    f32x4 v;  // FP32: v[0] alone
+    __device__ void reset() { v = f32x4{0.f, 0.f, 0.f, 0.f}; }
+    __device__ void scale(float a) {
+        if constexpr (FP32)
+            v[0] *= a;
+        else
+            v *= a;
+    }
+    __device__ void add(const float (&p)[8]) {
+        if constexpr (FP32) v[0] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+    }
+    template <class O>
+    __device__ void add_rounded(u32x4 pb) {
+        if constexpr (!FP32) v = O::mma_k32(u32x4{O::ONE2, O::ONE2, O::ONE2, O::ONE2}, pb, v);
+    }
+    __device__ float total() const {  // all four lanes of the row active
+        if constexpr (FP32) {
+            const float s = v[0] + __shfl_xor(v[0], 16);
+            return s + __shfl_xor(s, 32);
+        }
+        return v[0];
+    }
+};
+
+// KV_ODD: V^T fragments of a step of which only the first n tokens are the job's, the others
+// zero (the stage holds a row of the job there, which P = 0 would not cancel if it is infinite).
+template <int DB>
+__device__ inline void mask_v(u32x4 (&vf)[DB], int n, int g4) {
+    u32x4 keep;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int t = 16 * (j >> 1) + 4 * g4 + 2 * (j & 1);
+        keep[j] = (t < n ? 0xffffu : 0u) | (t + 1 < n ? 0xffff0000u : 0u);
+    }
+#pragma unroll
+    for (int db = 0; db < DB; ++db) vf[db] &= keep;
+}
+
 template <int D, bool FP16, int NB, int NW, int L>
 struct TileMath {
     static constexpr int DB = D / 16;  // 16-row blocks of O^T
     static constexpr int KS = D / 32;  // 32-wide k slices of QK
     using O = Ops<FP16>;
     using T = Tile<D>;
+    using Z = RowSum<L>;
 
-    f32x4 o[NB][DB], z[NB];
+    f32x4 o[NB][DB];
+    Z z[NB];
     float m[NB];
 
     __device__ void reset() {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             m[nb] = NEG_INF;
-            z[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+            z[nb].reset();
 #pragma unroll
             for (int db = 0; db < DB; ++db) o[nb][db] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
@@ -448,7 +498,6 @@ struct TileMath {
     __device__ void tile(const u16 *__restrict__ cur, const u32x4 (&qf)[NB][KS], const LdsOfs &of, int lo,
                          int hi, int g4, float c) {
         constexpr int STEPS = T::TT / 32;
-        const u32x4 ones = {O::ONE2, O::ONE2, O::ONE2, O::ONE2};
         f32x4 s[NB][2];
         {
             u32x4 kf[2][KS];
@@ -474,6 +523,7 @@ struct TileMath {
                             const int tok = base + 16 * b + 4 * g4 + i;
                             if (tok < lo || tok >= hi) s[nb][b][i] = NEG_INF;
                         }
+                if constexpr (Z::FP32) mask_v(vf, hi - base, g4);
             }
             // ---- softmax of every row block -> P^T fragments (B operand of PV)
             u32x4 pb[NB];
@@ -490,7 +540,7 @@ struct TileMath {
                 if (__builtin_amdgcn_ballot_w64(need)) {  // wave-uniform, rare after the first step
                     const float mn = fmaxf(m[nb], xor_max(lm) * c);
                     const float alpha = fast_exp2(m[nb] - mn);
-                    z[nb] *= alpha;
+                    z[nb].scale(alpha);
 #pragma unroll
                     for (int db = 0; db < DB; ++db) o[nb][db] *= alpha;
                     m[nb] = mn;
@@ -498,6 +548,7 @@ struct TileMath {
                 float pr[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) pr[i] = fast_exp2(__builtin_fmaf(x[i], c, -m[nb]));
+                z[nb].add(pr);
                 pb[nb] = u32x4{O::pack(pr[0], pr[1]), O::pack(pr[2], pr[3]), O::pack(pr[4], pr[5]),
                                O::pack(pr[6], pr[7])};
             }
@@ -507,7 +558,7 @@ struct TileMath {
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) o[nb][db] = O::mma_k32(vf[db], pb[nb], o[nb][db]);
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) z[nb] = O::mma_k32(ones, pb[nb], z[nb]);
+            for (int nb = 0; nb < NB; ++nb) z[nb].template add_rounded<O>(pb[nb]);
             if (more) qk(kf, qf, s);
         }
     }
@@ -648,10 +699,11 @@ __device__ __forceinline__ void tile_item(const SegParams &p, const int32_t *__r
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
         const int grow = wrow0 + 16 * nb + row;
+        const float z = acc.z[nb].total();
         if (grow >= nrows) continue;
         const int lr = grow / p.group, gg = grow - lr * p.group;
         const size_t prow = (size_t)(rb + lr) * p.hq + h * p.group + gg;
-        store_partial<M::DB>(p.part, p.lse, prow, acc.o[nb], acc.m[nb], acc.z[nb][0], g4);
+        store_partial<M::DB>(p.part, p.lse, prow, acc.o[nb], acc.m[nb], z, g4);
     }
 }
 
@@ -692,8 +744,10 @@ struct PipeMath {
     using O = Ops<FP16>;
     using T = Tile<D>;
     using TM = TileMath<D, FP16, NB, NW, L>;
+    using Z = RowSum<L>;
 
-    f32x4 o[NB][DB], z[NB];
+    f32x4 o[NB][DB];
+    Z z[NB];
     float m[NB], lm[NB], thr[NB];  // running max (scaled), raw row max of the staged step, (m + TAU) / c
     f32x4 s[NB][2];      // scores of the step whose exponentials come next
     u32x4 kf[2][KS];     // K fragments of the next QK step
@@ -703,7 +757,7 @@ struct PipeMath {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             m[nb] = thr[nb] = NEG_INF;
-            z[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+            z[nb].reset();
 #pragma unroll
             for (int db = 0; db < DB; ++db) o[nb][db] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
@@ -737,6 +791,7 @@ struct PipeMath {
     // zero, so the maxima are set without the pass over O that rescale makes
     // (the values equal rescale's from the initial state).
     __device__ void first_max(float c, float rc) {
+        if constexpr (Z::FP32) return rescale(c, rc);
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             const float mn = xor_max(lm[nb]) * c;
@@ -746,8 +801,23 @@ struct PipeMath {
     }
 
     // Raise the running maxima where a score of the staged step exceeds them
-    // by more than TAU (wave-uniform branch, rare after the first step).
+    // by more than TAU (wave-uniform branch, rare after the first step).  KV_ODD
+    // decides it per row block as tile() does, so that a row's result does not
+    // depend on the kind of item it is in.
     __device__ void rescale(float c, float rc) {  // rc = 1 / c
+        if constexpr (Z::FP32) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                if (!__builtin_amdgcn_ballot_w64(lm[nb] * c > m[nb] + TAU)) continue;
+                const float mn = fmaxf(m[nb], xor_max(lm[nb]) * c);
+                const float alpha = fast_exp2(m[nb] - mn);
+                z[nb].scale(alpha);
+#pragma unroll
+                for (int db = 0; db < DB; ++db) o[nb][db] *= alpha;
+                m[nb] = mn;
+            }
+            return;
+        }
         bool need = false;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) need |= lm[nb] > thr[nb];
@@ -756,7 +826,7 @@ struct PipeMath {
             for (int nb = 0; nb < NB; ++nb) {
                 const float mn = fmaxf(m[nb], xor_max(lm[nb]) * c);
                 const float alpha = mn == NEG_INF ? 1.f : fast_exp2(m[nb] - mn);
-                z[nb] *= alpha;
+                z[nb].scale(alpha);
 #pragma unroll
                 for (int db = 0; db < DB; ++db) o[nb][db] *= alpha;
                 m[nb] = mn;
@@ -767,7 +837,7 @@ struct PipeMath {
 
     // One pipeline block (see above).  vs / vbase: stage and offset of V(g);
     // ks / kbase: of K(g+2) (any resident step when there is none); lo / hi:
-    // valid tokens of step g+1.  Every fragment register set is reloaded only
+    // valid tokens of step g+1 (without MORE: of step g, for KV_ODD).  Every fragment register set is reloaded only
     // after its last reader: V(g) during QK(g+1), K(g+2) during PV(g).
     //
     // With MORE the order is written out, one matrix instruction per slot, and each
@@ -787,7 +857,6 @@ struct PipeMath {
     __device__ __forceinline__ void block(const u16 *__restrict__ vs, int vbase, const u16 *__restrict__ ks,
                                           int kbase, const u32x4 (&qf)[NB][KS], const LdsOfs &of, int lo,
                                           int hi, int g4, float c, unsigned keep = ~0u, Copy copy = Copy()) {
-        const u32x4 ones = {O::ONE2, O::ONE2, O::ONE2, O::ONE2};
         u32x4 pb[NB];
         if constexpr (MORE) {
             constexpr int NQ = 2 * KS * NB;      // MFMAs of QK
@@ -806,9 +875,11 @@ struct PipeMath {
                 for (int e = i * EXPS; e < (i + 1) * EXPS; ++e) {
                     const int n = e / 8, x = e % 8;
                     pr[n][x] = fast_exp2(__builtin_fmaf(s[n][x >> 2][x & 3], c, -m[n]));
-                    if (x == 7)
+                    if (x == 7) {
+                        z[n].add(pr[n]);
                         pb[n] = u32x4{O::pack(pr[n][0], pr[n][1]), O::pack(pr[n][2], pr[n][3]),
                                       O::pack(pr[n][4], pr[n][5]), O::pack(pr[n][6], pr[n][7])};
+                    }
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -839,7 +910,7 @@ struct PipeMath {
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) z[nb] = O::mma_k32(ones, pb[nb], z[nb]);
+            for (int nb = 0; nb < NB; ++nb) z[nb].template add_rounded<O>(pb[nb]);
             if constexpr (MASKN) {
                 finish_scores<true>(sn, lo, hi, g4);
             } else {
@@ -853,11 +924,14 @@ struct PipeMath {
             return;
         }
         TM::load_v(vs, of, vbase, vf);
+        if constexpr (Z::FP32)
+            if (hi < 32) mask_v(vf, hi, g4);
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             float pr[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) pr[i] = fast_exp2(__builtin_fmaf(s[nb][i >> 2][i & 3], c, -m[nb]));
+            z[nb].add(pr);
             pb[nb] = u32x4{O::pack(pr[0], pr[1]), O::pack(pr[2], pr[3]), O::pack(pr[4], pr[5]),
                            O::pack(pr[6], pr[7])};
             if (ROWMASK && !((keep >> nb) & 1)) pb[nb] = u32x4{0u, 0u, 0u, 0u};
@@ -867,7 +941,7 @@ struct PipeMath {
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) o[nb][db] = O::mma_k32(vf[db], pb[nb], o[nb][db]);
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) z[nb] = O::mma_k32(ones, pb[nb], z[nb]);
+        for (int nb = 0; nb < NB; ++nb) z[nb].template add_rounded<O>(pb[nb]);
     }
 
     // One staged tile of an attached private segment (after the pipeline has
@@ -1149,7 +1223,9 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
     }
     if (g < nsteps) {
         if (!(g & 1)) sync_tile(g >> 1);
-        if (active) acc.template block<false, false>(stage(g), 32 * (g & 1), stage(g), 0, qf, of, 0, 32, g4, c);
+        if (active)
+            acc.template block<false, false>(stage(g), 32 * (g & 1), stage(g), 0, qf, of, 0, kend - (tb0 + 32 * g), g4,
+                                             c);
     }
 
     // Attached segments, in rounds of up to STAGES tiles that are resident
@@ -1184,10 +1260,11 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
         const int grow = wrow0 + 16 * nb + row;
+        const float z = acc.z[nb].total();
         if (grow >= nrows) continue;
         const int lr = grow / p.group, gg = grow - lr * p.group;
         const size_t prow = (size_t)(rb + lr) * p.hq + h * p.group + gg;
-        store_partial<M::DB>(p.part, p.lse, prow, acc.o[nb], acc.m[nb], acc.z[nb][0], g4);
+        store_partial<M::DB>(p.part, p.lse, prow, acc.o[nb], acc.m[nb], z, g4);
     }
 }
 
@@ -1306,7 +1383,7 @@ __global__ __launch_bounds__(128) void seg_tail_kernel(SegParams p) {
         }
         // the tile's reads fed the MFMAs above, so the stage is free for the partial
         const bool any = acc.m[0] != NEG_INF;
-        const float zr = acc.z[0][0];
+        const float zr = acc.z[0].total();
         const float inv = any ? 1.f / zr : 0.f;
         if (row < G) {
 #pragma unroll
@@ -1406,7 +1483,12 @@ template <int D, bool FP16, int L>
 hipError_t launch_d(const SegParams &sp, int kind, hipStream_t stream) {
     switch (kind) {
         case TA_TAIL:  // as TA_SMALL, merging the request into out when out is given
-            if (sp.out) return launch_tail_merge<D, FP16, L>(sp, stream);
+            if (sp.out) {
+                if constexpr (L == KV_ODD)
+                    return (hipError_t)TA_ERR_ARG;
+                else
+                    return launch_tail_merge<D, FP16, L>(sp, stream);
+            }
             [[fallthrough]];
         case TA_SMALL:  // one wave per (job, head); one stage so that five fit on a CU
             if (L != KV_ODD && sp.tcap <= SHORT_CAP)

@@ -273,7 +273,7 @@ int segment_launch(const void *q, const void *kp, const void *vp, const int32_t 
         return TA_ERR_ARG;
     if (!aligned16(q) || !aligned16(kp) || !aligned16(vp) || !aligned16(part)) return TA_ERR_ALIGN;
     if (out) {
-        if (kind != TA_TAIL || !slots || !counts || maxs <= 0) return TA_ERR_ARG;
+        if (kind != TA_TAIL || layout == KV_ODD || !slots || !counts || maxs <= 0) return TA_ERR_ARG;
         if (!aligned16(out)) return TA_ERR_ALIGN;
     }
     if (xtail && (kind != TA_LARGE256 || layout == KV_ODD || xtail_stride != TA_XTAIL_STRIDE)) return TA_ERR_ARG;
@@ -446,8 +446,12 @@ int attention_layer(const void *q, const void *kp, const void *vp, int32_t tcap,
         if (plan->n_items[kind] == 0) continue;
         if (int e = plan_segment(q, kp, vp, tcap, plan, kind, nullptr, layout, stream)) return e;
     }
+    // the fused merge takes a tail's partial in FP32; pools of other capacities store every
+    // partial and merge all requests alike
+    const bool fused = layout != KV_ODD;
     if (plan->n_items[TA_TAIL] > 0)
-        if (int e = plan_segment(q, kp, vp, tcap, plan, TA_TAIL, out, layout, stream)) return e;
+        if (int e = plan_segment(q, kp, vp, tcap, plan, TA_TAIL, fused ? out : nullptr, layout, stream)) return e;
+    if (!fused) return plan_merge(plan, nullptr, plan->nreq, out, stream);
     if (plan->n_rest <= 0) return 0;
     // rest == NULL with n_rest == nreq: every request
     if (!plan->rest && plan->n_rest != plan->nreq) return TA_ERR_ARG;
