@@ -157,9 +157,9 @@ int ta_attention_matrix(const void *q, const void *kp, const void *vp,
 
 /* ta_attention_matrix on token-major keys and values, as a prefill leaves them
  * (replaces pack_kv + attention_matrix, kernels.py:144-149): k, v [tokens, hk, d],
- * contiguous, 16-byte aligned, physical token t of the plan in row t.  The same
- * launches and partials as ta_attention_matrix; nothing is packed, and the number of
- * tokens may be any. */
+ * contiguous, 16-byte aligned, physical token t of the plan in row t.  The launches and
+ * the bits of ta_attention_matrix on pools packed from them (a number of tokens that is
+ * no multiple of 8 takes no attachments and the unfused order); nothing is packed. */
 int ta_attention_tokens(const void *q, const void *k, const void *v, int32_t tokens, const ta_plan *plan,
                         void *out, void *stream);
 

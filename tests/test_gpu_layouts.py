@@ -101,9 +101,10 @@ def test_odd_capacity_sums_fp32_probabilities(n, nreq, tile_rows, kind, device):
     prepared = prepare(plan, q, tile_rows=tile_rows, route_items=0, consolidate_rows=0, large_target=1, small_target=1)
     say("fp32 sums", n, nreq, list(prepared.abi.n_items))
     assert prepared.abi.n_items[kind] and len(prepared.jobs) == 1
-    attention_matrix(q, *pack_kv(k, v), prepared)
-    got = prepared.lse[..., 0].cpu()
-    assert (got - lse).abs().max() < 1e-4
+    for layer in (lambda: attention_matrix(q, *pack_kv(k, v), prepared), lambda: attention(q, k, v, prepared)):
+        prepared.lse.zero_()
+        layer()
+        assert (prepared.lse[..., 0].cpu() - lse).abs().max() < 1e-4
 
 
 @pytest.mark.parametrize("n", [5, 45, 75, 333])
@@ -153,6 +154,30 @@ def test_token_major_equals_packed(device):
         attention(q, k.half(), v, p)
     with pytest.raises(ValueError):
         attention(q[:3], k, v, p)
+
+
+@pytest.mark.parametrize("hq,hk,d,dtype", [(32, 8, 128, torch.bfloat16), (8, 2, 64, torch.float16),
+                                           (8, 8, 32, torch.bfloat16)])
+@pytest.mark.parametrize("shared,nreq", [(2043, 96), (77, 9), (0, 300)])
+def test_token_major_of_any_count_equals_packed(shared, nreq, hq, hk, d, dtype, device):
+    """Numbers of tokens that are no multiple of 8: the bits of the packed pools, also under a
+    plan with attachments (both run it without) and with tails of their own, without packing."""
+    spec = shapes.shared_prefix(nreq, shared, [1 + (37 * r) % 60 for r in range(nreq)])
+    tree = shapes.tree(spec)
+    t = tree.storage_tokens + (1 if tree.storage_tokens % 8 == 0 else 0)
+    g = torch.Generator().manual_seed(shared)
+    q = torch.randn(nreq, hq, d, generator=g).to(dtype).to(device)
+    k = torch.randn(t, hk, d, generator=g).to(dtype).to(device)
+    v = torch.randn(t, hk, d, generator=g).to(dtype).to(device)
+    for method in ("cube", "request"):
+        p = prepare(schedule(tree, hq, hk, d, method, CostModel.mi355x()), q)
+        a = attention(q, k, v, p).clone()
+        b = attention_matrix(q, *pack_kv(k, v), p).clone()
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        attention(q, k, v, p)
+        assert torch.cuda.memory_stats()["allocation.all.allocated"] == before  # nothing packed
+        say("any count", t, method, list(p.abi.n_items), len(p.attached))
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("hk", [8, 4])

@@ -47,13 +47,13 @@ COMMON = [
 # kernel never produces NaN scores (masked tokens are selected to -inf).
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 # segment_tile.hip is compiled once per K/V layout (enum Layout, ta_common.h); the
-# flag stays off for the pools of other capacities, whose row maxima pass over a NaN
+# flag stays off for the layouts of token counts that are no multiple of 8, whose row maxima pass over a NaN
 # score wherever it stands (at most 0.4 % of a layer's time either way, 2 % in 256-row items).
 SOURCES = [
     (HERE / "tree_attn.hip", VGPR_FORM),
     *[(HERE / "segment_tile.hip", VGPR_FORM + ["-fno-honor-nans", f"-DTA_LAYOUT={layout}"])
       for layout in ("KV_POOL", "KV_TOKEN")],
-    (HERE / "segment_tile.hip", VGPR_FORM + ["-DTA_LAYOUT=KV_ODD"]),
+    *[(HERE / "segment_tile.hip", VGPR_FORM + [f"-DTA_LAYOUT={layout}"]) for layout in ("KV_ODD", "KV_TOKEN_ODD")],
     (HERE / "decode_append.hip", ["-ffp-contract=off"]),  # each RoPE product rounded, as the eager ops
 ]
 
@@ -87,7 +87,7 @@ def build(verbose: bool = False, out: Path | None = None, defines=()) -> Path:
                   "-c", str(src), "-o", str(obj)], verbose)
             return str(obj)
 
-        with ThreadPoolExecutor(4) as pool:  # each unit takes up to a minute
+        with ThreadPoolExecutor(5) as pool:  # each unit takes up to a minute
             objs = list(pool.map(compile_one, range(len(SOURCES))))
         _run([hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", str(tmp)], verbose)
     os.replace(tmp, target)

@@ -110,10 +110,10 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
             if (!sizes(k, cap, plan->hk, plan->d) || !sizes(v, cap, plan->hk, plan->d)) return general();
             // (a view may start anywhere; a packed copy would not)
             if ((uintptr_t)k.data_ptr() % 16 || (uintptr_t)v.data_ptr() % 16) return general();
-        } else {
-            if (!sizes(k, plan->hk, plan->d, cap) || !sizes(v, plan->hk, cap, plan->d)) return general();
-            if (plan->xtail && cap % 8) return general();  // PreparedPlan.for_pools
+        } else if (!sizes(k, plan->hk, plan->d, cap) || !sizes(v, plan->hk, cap, plan->d)) {
+            return general();
         }
+        if (plan->xtail && cap % 8) return general();  // PreparedPlan.for_capacity
         void *stream;
         if (!stream_of(device, &stream)) return general();
         const void *qp = q.data_ptr(), *kp = k.data_ptr(), *vp = v.data_ptr();

@@ -191,9 +191,9 @@ struct TileCopy {
 
     // Row t of head h of V (and of token-major K).
     __device__ static const u16 *row(const u16 *x, const SegParams &p, int h, int t) {
-        return x + (L == KV_TOKEN ? (size_t)t * p.hk + h : (size_t)h * p.tcap + t) * D;
+        return x + (token_major(L) ? (size_t)t * p.hk + h : (size_t)h * p.tcap + t) * D;
     }
-    __device__ static u32 row_bytes(const SegParams &p) { return 2u * D * (L == KV_TOKEN ? p.hk : 1); }
+    __device__ static u32 row_bytes(const SegParams &p) { return 2u * D * (token_major(L) ? p.hk : 1); }
 
     // Byte offsets of this lane's 16 bytes in a KV_POOL tile's copies of wave w from the first
     // row of the block copied: K block w + n NW, and V block w + n NW (NW and KBLK even, so
@@ -233,7 +233,7 @@ struct TileCopy {
     template <bool CLAMP>
     __device__ static void copy_k(u16 *st, const SegParams &p, int h, int t0n, int kst, int kend, int blk, int lane) {
         u16 *dst = st + blk * T::BLK;
-        if constexpr (L == KV_TOKEN) {
+        if constexpr (token_major(L)) {
             // row-major tile: lane i fills slot i, chunk (i % CPR) ^ f of token row i / CPR (KTokens)
             const int j = lane / KTokens<D>::CPR;
             copy_row<CLAMP>(dst, p.kp, p, h, t0n, kst, kend, blk * T::VROWS, j,
@@ -330,14 +330,14 @@ struct TileCopy {
 };
 
 // The softmax denominator of a lane's row.  KV_POOL and KV_TOKEN: one more PV MFMA against
-// an all-ones A operand, so that it sums exactly the rounded P that multiplies V.  KV_ODD:
-// the FP32 exponentials themselves, each lane its own tokens, added over the four lanes of
+// an all-ones A operand, so that it sums exactly the rounded P that multiplies V.  The
+// others (odd_count): the FP32 exponentials themselves, each lane its own tokens, added over the four lanes of
 // the row at the end -- the log-sum-exp then carries no rounding of P.  Against the ones
 // product: 24 ragged requests in two branches, 10,839 tokens, 25.7 us (25.5); 128 requests x
 // 8192 in 256-row items, where the additions share the step's slots, 54.3 us (48.1).
 template <int L>
 struct RowSum {
-    static constexpr bool FP32 = L == KV_ODD;
+    static constexpr bool FP32 = odd_count(L);
     f32x4 v;  // FP32: v[0] alone
     __device__ void reset() { v = f32x4{0.f, 0.f, 0.f, 0.f}; }
     __device__ void scale(float a) {
@@ -362,7 +362,7 @@ struct RowSum {
     }
 };
 
-// KV_ODD: V^T fragments of a step of which only the first n tokens are the job's, the others
+// odd_count layouts: V^T fragments of a step of which only the first n tokens are the job's, the others
 // zero (the stage holds a row of the job there, which P = 0 would not cancel if it is infinite).
 template <int DB>
 __device__ inline void mask_v(u32x4 (&vf)[DB], int n, int g4) {
@@ -415,7 +415,7 @@ struct TileMath {
     // K fragments (A operand of QK) of the 32 tokens base .. base+31:
     // kf[b][ks] covers tokens base+16b .. +15, d = 32*ks .. +31.
     __device__ static void load_k(const u16 *__restrict__ cur, const LdsOfs &of, int base, u32x4 (&kf)[2][KS]) {
-        if constexpr (L == KV_TOKEN) {
+        if constexpr (token_major(L)) {
             u32 a[KS];
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) a[ks] = (u32)(uintptr_t)(lds_u16 *)(cur + of.kt[ks] + base * D);
@@ -575,10 +575,10 @@ __device__ inline int xcd_item(int b, int n) {
 
 // First token of the tiles of a job or segment that starts at token t: a KV_POOL
 // K row is copied in aligned chunks of 8 tokens (KV_TOKEN follows it, so that both
-// sum in the same order; KV_ODD starts at the job's first token).
+// sum in the same order; the odd_count layouts start at the job's first token).
 template <int L>
 __device__ inline int tile_start(int t) {
-    return L == KV_ODD ? t : t & ~7;
+    return odd_count(L) ? t : t & ~7;
 }
 
 // The waves of a work item meet at a barrier, unless one wave works alone on
@@ -801,8 +801,8 @@ struct PipeMath {
     }
 
     // Raise the running maxima where a score of the staged step exceeds them
-    // by more than TAU (wave-uniform branch, rare after the first step).  KV_ODD
-    // decides it per row block as tile() does, so that a row's result does not
+    // by more than TAU (wave-uniform branch, rare after the first step).  odd_count
+    // layouts decide it per row block as tile() does, so that a row's result does not
     // depend on the kind of item it is in.
     __device__ void rescale(float c, float rc) {  // rc = 1 / c
         if constexpr (Z::FP32) {
@@ -837,7 +837,7 @@ struct PipeMath {
 
     // One pipeline block (see above).  vs / vbase: stage and offset of V(g);
     // ks / kbase: of K(g+2) (any resident step when there is none); lo / hi:
-    // valid tokens of step g+1 (without MORE: of step g, for KV_ODD).  Every fragment register set is reloaded only
+    // valid tokens of step g+1 (without MORE: of step g, for odd_count layouts).  Every fragment register set is reloaded only
     // after its last reader: V(g) during QK(g+1), K(g+2) during PV(g).
     //
     // With MORE the order is written out, one matrix instruction per slot, and each
@@ -892,8 +892,8 @@ struct PipeMath {
             for (int j = 0; j < NP; ++j) {
                 const int db = j / NB, nb = j % NB;
                 o[nb][db] = O::mma_k32(vf[db], pb[nb], o[nb][db]);
-                if (L == KV_TOKEN ? j == 0 : j < 2 * KS) {
-                    if constexpr (L == KV_TOKEN)
+                if (token_major(L) ? j == 0 : j < 2 * KS) {
+                    if constexpr (token_major(L))
                         TM::load_k(ks, of, kbase, kf);
                     else
                         kf[j % 2][j / 2] = TM::k_pair(ks, of, kbase, j % 2, j / 2);
@@ -1232,7 +1232,7 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
     // together: one wait and one barrier per round, then every wave attends
     // the round's tiles of the segments holding its rows, side by side.  The
     // root loop (or the prologue) already issued the first tiles.
-    if constexpr (L != KV_ODD) {  // (the launcher passes no attachments for KV_ODD)
+    if constexpr (!odd_count(L)) {  // (the launcher passes no attachments for the others)
         for (int r0 = ntiles; r0 < ntot; r0 += STAGES) {
             const int r1 = min(r0 + STAGES, ntot);
             __builtin_amdgcn_s_barrier();  // every wave is done with the tiles before r0
@@ -1484,7 +1484,7 @@ hipError_t launch_d(const SegParams &sp, int kind, hipStream_t stream) {
     switch (kind) {
         case TA_TAIL:  // as TA_SMALL, merging the request into out when out is given
             if (sp.out) {
-                if constexpr (L == KV_ODD)
+                if constexpr (odd_count(L))
                     return (hipError_t)TA_ERR_ARG;
                 else
                     return launch_tail_merge<D, FP16, L>(sp, stream);

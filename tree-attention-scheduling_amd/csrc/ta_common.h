@@ -197,12 +197,19 @@ struct MixParams {
 //             8-token chunk of a K row is 16-byte aligned
 //   KV_ODD:   the same pools of any other capacity: K rows start anywhere
 //   KV_TOKEN: k, v [tokens, hk, d], as a prefill leaves them (kp, vp point at
-//             them, tcap is the number of tokens)
-enum Layout { KV_POOL, KV_ODD, KV_TOKEN };
+//             them, tcap is the number of tokens), tcap % 8 == 0
+//   KV_TOKEN_ODD: the same of any other number of tokens
+// Pools packed from token-major K and V give the same bits: KV_TOKEN those of
+// KV_POOL, KV_TOKEN_ODD those of KV_ODD.
+enum Layout { KV_POOL, KV_ODD, KV_TOKEN, KV_TOKEN_ODD };
+constexpr bool token_major(int layout) { return layout == KV_TOKEN || layout == KV_TOKEN_ODD; }
+// Tiles start at the job's first token, denominators sum FP32 exponentials, no
+// attachments and no fused merge.
+constexpr bool odd_count(int layout) { return layout == KV_ODD || layout == KV_TOKEN_ODD; }
 
 // Launchers of segment_tile.hip, which is compiled once per layout
 // (hipErrorNotSupported for a head dim they have no kernel for).
-// One segment launch of the work items of one kind; KV_ODD takes no attachments.
+// One segment launch of the work items of one kind; odd_count layouts take no attachments.
 template <int L>
 hipError_t launch_kind(const SegParams &sp, int kind, int d, bool fp16, hipStream_t stream);
 // One launch of the TA_LARGE256, TA_LARGE64 and TA_SMALL items items[k]
@@ -219,6 +226,7 @@ hipError_t launch_mix(const SegParams &sp, const int32_t *const items[3], const 
 TA_EXTERN_LAYOUT(KV_POOL)
 TA_EXTERN_LAYOUT(KV_ODD)
 TA_EXTERN_LAYOUT(KV_TOKEN)
+TA_EXTERN_LAYOUT(KV_TOKEN_ODD)
 #undef TA_EXTERN_LAYOUT
 
 }  // namespace ta

@@ -181,8 +181,9 @@ __global__ __launch_bounds__(READ_NT) void read_stream_kernel(const u32x4 *__res
 }
 
 // ------------------------------------------------------------------ launch
-// The layout of pools of `tcap` tokens.
+// The layout of pools, and of token-major K and V, of `tcap` tokens.
 int pool_layout(int32_t tcap) { return tcap % 8 == 0 ? KV_POOL : KV_ODD; }
+int token_layout(int32_t tcap) { return tcap % 8 == 0 ? KV_TOKEN : KV_TOKEN_ODD; }
 
 // nreq requests: reqs[0 .. nreq) when reqs is given, else 0 .. nreq-1
 template <int D, bool FP16>
@@ -273,18 +274,19 @@ int segment_launch(const void *q, const void *kp, const void *vp, const int32_t 
         return TA_ERR_ARG;
     if (!aligned16(q) || !aligned16(kp) || !aligned16(vp) || !aligned16(part)) return TA_ERR_ALIGN;
     if (out) {
-        if (kind != TA_TAIL || layout == KV_ODD || !slots || !counts || maxs <= 0) return TA_ERR_ARG;
+        if (kind != TA_TAIL || odd_count(layout) || !slots || !counts || maxs <= 0) return TA_ERR_ARG;
         if (!aligned16(out)) return TA_ERR_ALIGN;
     }
-    if (xtail && (kind != TA_LARGE256 || layout == KV_ODD || xtail_stride != TA_XTAIL_STRIDE)) return TA_ERR_ARG;
+    if (xtail && (kind != TA_LARGE256 || odd_count(layout) || xtail_stride != TA_XTAIL_STRIDE)) return TA_ERR_ARG;
     SegParams sp;
     fill_params(sp, q, kp, vp, qids, kstart, qlen, klen, rowbase, items, n_items, part, lse, hq, hk, d, tcap, maxr,
                 slots, counts, out, maxs, xtail, xtail_stride, qbase);
     const hipStream_t st = static_cast<hipStream_t>(stream);
     const bool fp16 = dtype == TA_FP16;
-    return (int)(layout == KV_POOL  ? ta::launch_kind<KV_POOL>(sp, kind, d, fp16, st)
-                 : layout == KV_ODD ? ta::launch_kind<KV_ODD>(sp, kind, d, fp16, st)
-                                    : ta::launch_kind<KV_TOKEN>(sp, kind, d, fp16, st));
+    return (int)(layout == KV_POOL    ? ta::launch_kind<KV_POOL>(sp, kind, d, fp16, st)
+                 : layout == KV_ODD   ? ta::launch_kind<KV_ODD>(sp, kind, d, fp16, st)
+                 : layout == KV_TOKEN ? ta::launch_kind<KV_TOKEN>(sp, kind, d, fp16, st)
+                                      : ta::launch_kind<KV_TOKEN_ODD>(sp, kind, d, fp16, st));
 }
 
 // The launch arguments every segment kernel shares.
@@ -418,7 +420,7 @@ int mix_launch(const void *q, const void *kp, const void *vp, int32_t tcap, cons
         if (plan->n_items[k] > 0 && !plan->items[k]) return TA_ERR_ARG;
     if (!aligned16(q) || !aligned16(kp) || !aligned16(vp) || !aligned16(plan->part)) return TA_ERR_ALIGN;
     const bool xt = n[0] > 0 && plan->xtail;
-    if (xt && (plan->xtail_stride != TA_XTAIL_STRIDE || layout == KV_ODD)) return TA_ERR_ARG;
+    if (xt && (plan->xtail_stride != TA_XTAIL_STRIDE || odd_count(layout))) return TA_ERR_ARG;
     SegParams sp;
     fill_params(sp, q, kp, vp, plan->qids, plan->kstart, plan->qlen, plan->klen, plan->rowbase, nullptr, 0,
                 plan->part, plan->lse, plan->hq, plan->hk, plan->d, tcap, plan->maxr, plan->slots, plan->counts,
@@ -426,16 +428,16 @@ int mix_launch(const void *q, const void *kp, const void *vp, int32_t tcap, cons
     const int32_t *const items[3] = {plan->items[TA_LARGE256], plan->items[TA_LARGE64], plan->items[TA_SMALL]};
     const hipStream_t st = static_cast<hipStream_t>(stream);
     const bool fp16 = plan->dtype == TA_FP16;
-    return (int)(layout == KV_POOL  ? ta::launch_mix<KV_POOL>(sp, items, n, plan->d, fp16, st)
-                 : layout == KV_ODD ? ta::launch_mix<KV_ODD>(sp, items, n, plan->d, fp16, st)
-                                    : ta::launch_mix<KV_TOKEN>(sp, items, n, plan->d, fp16, st));
+    return (int)(layout == KV_POOL    ? ta::launch_mix<KV_POOL>(sp, items, n, plan->d, fp16, st)
+                 : layout == KV_ODD   ? ta::launch_mix<KV_ODD>(sp, items, n, plan->d, fp16, st)
+                 : layout == KV_TOKEN ? ta::launch_mix<KV_TOKEN>(sp, items, n, plan->d, fp16, st)
+                                      : ta::launch_mix<KV_TOKEN_ODD>(sp, items, n, plan->d, fp16, st));
 }
 
 int attention_layer(const void *q, const void *kp, const void *vp, int32_t tcap, const ta_plan *plan, void *out,
                     int layout, void *stream) {
     if (!plan || !out) return TA_ERR_ARG;
-    // attachments are kept to layouts whose K the LDS DMA takes
-    if (plan->xtail && layout == KV_ODD) return TA_ERR_ARG;
+    if (plan->xtail && odd_count(layout)) return TA_ERR_ARG;
     // the partials every merge reads come first: large jobs, then small jobs,
     // in one launch when the kinds allow it
     const int mixed = mix_launch(q, kp, vp, tcap, plan, layout, stream);
@@ -446,9 +448,9 @@ int attention_layer(const void *q, const void *kp, const void *vp, int32_t tcap,
         if (plan->n_items[kind] == 0) continue;
         if (int e = plan_segment(q, kp, vp, tcap, plan, kind, nullptr, layout, stream)) return e;
     }
-    // the fused merge takes a tail's partial in FP32; pools of other capacities store every
-    // partial and merge all requests alike
-    const bool fused = layout != KV_ODD;
+    // the fused merge takes a tail's partial in FP32; other token counts than multiples of 8
+    // store every partial and merge all requests alike
+    const bool fused = !odd_count(layout);
     if (plan->n_items[TA_TAIL] > 0)
         if (int e = plan_segment(q, kp, vp, tcap, plan, TA_TAIL, fused ? out : nullptr, layout, stream)) return e;
     if (!fused) return plan_merge(plan, nullptr, plan->nreq, out, stream);
@@ -490,7 +492,7 @@ int ta_attention_matrix(const void *q, const void *kp, const void *vp, int32_t t
 
 int ta_attention_tokens(const void *q, const void *k, const void *v, int32_t tokens, const ta_plan *plan, void *out,
                         void *stream) {
-    return attention_layer(q, k, v, tokens, plan, out, KV_TOKEN, stream);
+    return attention_layer(q, k, v, tokens, plan, out, token_layout(tokens), stream);
 }
 
 int ta_attention_matrix_noalloc(const void *q, const void *kp, const void *vp, int32_t tcap, const ta_plan *plan,

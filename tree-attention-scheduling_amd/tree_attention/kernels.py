@@ -103,11 +103,15 @@ class PreparedPlan:
             self._unattached.fill_growing(length)
 
     def for_pools(self, kp: torch.Tensor) -> "PreparedPlan":
-        """The plan to launch on pools like ``kp``: this one, or, when it has
-        attached segments and the pool capacity is not a multiple of 8 (whose
-        kernels bring K through registers and take no attachments), the same
-        plan prepared without attachments, writing into the same ``out``."""
-        if not self.attached or kp.shape[-1] % 8 == 0:
+        """The plan to launch on pools like ``kp`` (``for_capacity``)."""
+        return self.for_capacity(kp.shape[-1])
+
+    def for_capacity(self, tokens: int) -> "PreparedPlan":
+        """The plan to launch on K and V of ``tokens`` tokens: this one, or, when it
+        has attached segments and the count is not a multiple of 8 (whose kernels
+        take no attachments), the same plan prepared without attachments, writing
+        into the same ``out``."""
+        if not self.attached or tokens % 8 == 0:
             return self
         if self._unattached is None:
             alt = prepare(self.plan, self.out, attach_tails=False, **self.options)
@@ -830,7 +834,12 @@ def attention(q, k, v, prepared):
     140 us packed, 37 us in place).  Anything else is packed first, and
     ``attention_matrix`` checks it.
     """
-    rc = _fastcall().attention(q, k, v, ctypes.addressof(prepared.abi), prepared.out, True)
+    call = _fastcall().attention
+    rc = call(q, k, v, ctypes.addressof(prepared.abi), prepared.out, True)
+    if rc is None and prepared.attached and getattr(k, "ndim", 0) == 3:
+        p = prepared.for_capacity(k.shape[0])
+        if p is not prepared:
+            rc = call(q, k, v, ctypes.addressof(p.abi), p.out, True)
     if rc is None:
         return attention_matrix(q, *pack_kv(k, v), prepared)
     if rc:
