@@ -15,7 +15,7 @@ import torch
 
 from oracle.attention_oracle import relative_l2, request_attention
 from tree_attention import CostModel, KVTree, schedule, shapes
-from tree_attention import _native
+from tree_attention import _native, kernels
 from tree_attention.kernels import attention, attention_matrix, pack_kv, prepare
 from tree_attention.schedule import Job, Plan
 
@@ -178,6 +178,28 @@ def test_token_major_of_any_count_equals_packed(shared, nreq, hq, hk, d, dtype, 
         assert torch.cuda.memory_stats()["allocation.all.allocated"] == before  # nothing packed
         say("any count", t, method, list(p.abi.n_items), len(p.attached))
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("hk,d,nreq,pad,packed", [(32, 32, 120, 0, True), (32, 32, 40, 0, False), (24, 32, 120, 0, True),
+                                                  (32, 32, 120, 1, False), (16, 32, 120, 0, False),
+                                                  (32, 64, 120, 0, False)])
+def test_narrow_rows_read_often_are_packed(hk, d, nreq, pad, packed, device, monkeypatch):
+    """Token-major K and V of head dim 32 under a plan that reads them many times over: packed
+    (PACK_READS), with the bits of the call in place; any other call stays in place."""
+    tree = shapes.tree(shapes.shared_prefix(nreq, 2400, 4))
+    t = -(-tree.storage_tokens // 8) * 8 + pad
+    g = torch.Generator().manual_seed(hk + nreq)
+    q = torch.randn(nreq, hk, d, generator=g).bfloat16().to(device)
+    k = torch.randn(t, hk, d, generator=g).bfloat16().to(device)
+    v = torch.randn(t, hk, d, generator=g).bfloat16().to(device)
+    p = prepare(schedule(tree, hk, hk, d, "request", CostModel.mi355x()), q)
+    calls = []
+    monkeypatch.setattr(kernels, "pack_kv", lambda *kv: calls.append(1) or pack_kv(*kv))
+    a = attention(q, k, v, p).clone()
+    say("narrow", hk, d, nreq, t, p.narrow_reads, bool(calls))
+    assert bool(calls) == packed
+    monkeypatch.setattr(kernels, "PACK_READS", 10 ** 9)
+    assert torch.equal(a, attention(q, k, v, p)) and len(calls) == packed
 
 
 @pytest.mark.parametrize("hk", [8, 4])

@@ -88,6 +88,12 @@ class PreparedPlan:
     # positions in ``metadata`` of every growing tail's length: klen of the growing
     # jobs, the token field of the records of the items the attached ones joined
     grow_offsets: torch.Tensor | None = None
+    # head dim 32 and PACK_HEADS KV heads or more: (token, KV head) rows of K its work items read, else 0
+    narrow_reads: int = 0
+
+    def packs(self, tokens: int) -> bool:
+        """Whether token-major K and V of ``tokens`` tokens are better packed (``PACK_READS``)."""
+        return tokens % 8 == 0 and self.narrow_reads > PACK_READS * tokens
 
     def fill_growing(self, length: int) -> None:
         """Set the length of every growing tail (tokens from ``fixed_from`` on) to
@@ -210,6 +216,15 @@ LARGE_MIN_TILES = 2
 # wider large jobs run as 64-row request groups when 64-row items run anyway and no wider
 # job exceeds this many rows (prepare's consolidate_rows; 0: never)
 CONSOLIDATE_ROWS = 128
+# token-major K and V of head dim 32 are packed when a plan reads each of them often: a token's
+# row of one head is then half a 128-byte line, PACK_HEADS heads or more apart from the next
+# token's.  PACK_READS is the reads of a token's rows (over all heads) from which the packing
+# pays: in place against packed at most 1.03x up to 1,600 of them, 0.95-1.53x above, growing
+# with them (per-request plans, 24-96 heads, 3,424-20,480 tokens; at 16 heads never above
+# 0.93x, at head dims 64 and 128 never above 0.84x; counts that are no multiple of 8 stay in
+# place, their packed pools are the slower ones).
+PACK_HEADS = 24
+PACK_READS = 1600
 # a launch of small-job items alone (2048 one-wave workgroups, 8 per CU) takes two-tile chunks
 # instead of one-tile chunks when those would fill at least 45 % of its waves: a wave streams
 # the second tile of an item while it computes the first, and every chunk is one more partial
@@ -436,6 +451,18 @@ def _recut(jobs, items_per_chunk, target_items, is_fixed, min_tiles=1, floor_ite
             put(job, "tokens", ids[a:a + size])
             out.append(job)
     return out
+
+
+def _narrow_reads(jobs, attached, group, kvheads, dim, tile_rows) -> int:
+    """(token, KV head) rows that the work items read, where ``PACK_READS`` looks at them."""
+    if dim != 32 or kvheads < PACK_HEADS:
+        return 0
+    reads = sum(len(job.tokens) for segs in attached.values() for job, _ in segs)
+    for job in jobs:
+        rows = len(job.requests) * group
+        tile = SMALL_ROWS if rows <= SMALL_ROWS else _native.KIND_ROWS[_large_kind(rows, tile_rows)]
+        reads += -(-rows // tile) * len(job.tokens)
+    return reads * kvheads
 
 
 def _cu_count(device) -> int:
@@ -818,7 +845,8 @@ def prepare(plan: Plan, q: torch.Tensor, tile_rows: int = 256, fixed_from: int |
                          "consolidate_rows": consolidate_rows, "large_target": large_target,
                          "small_target": small_target, "large_min_tiles": large_min_tiles}, None,
                         meta["qbase"].tolist(),
-                        grow_offsets=grow_offsets)
+                        grow_offsets=grow_offsets,
+                        narrow_reads=_narrow_reads(jobs, attached, group, kvheads, dim, tile_rows))
 
 
 def pack_kv(k: torch.Tensor, v: torch.Tensor):
@@ -830,16 +858,16 @@ def attention(q, k, v, prepared):
     """``attention_matrix`` on ``k, v [T,HK,D]`` (kernels.py:148-149).
 
     Contiguous K and V are attended where they lie (``ta_attention_tokens``):
-    packing them costs a strided pass over both (one layer of 17,424 tokens:
-    140 us packed, 37 us in place).  Anything else is packed first, and
-    ``attention_matrix`` checks it.
+    packing them costs a strided pass over both (17,424 tokens of 8 heads of
+    128: about 110 us, the layer itself 27).  Plans that read narrow rows many
+    times (``PACK_READS``) and anything that is not contiguous are packed first,
+    and ``attention_matrix`` checks them.
     """
     call = _fastcall().attention
-    rc = call(q, k, v, ctypes.addressof(prepared.abi), prepared.out, True)
-    if rc is None and prepared.attached and getattr(k, "ndim", 0) == 3:
+    rc = None
+    if getattr(k, "ndim", 0) == 3 and not prepared.packs(k.shape[0]):
         p = prepared.for_capacity(k.shape[0])
-        if p is not prepared:
-            rc = call(q, k, v, ctypes.addressof(p.abi), p.out, True)
+        rc = call(q, k, v, ctypes.addressof(p.abi), p.out, True)
     if rc is None:
         return attention_matrix(q, *pack_kv(k, v), prepared)
     if rc:
