@@ -233,6 +233,33 @@ def test_one_wave_items_in_any_order(small, hk, device):
         assert relative_l2(out, ref) <= 3e-3
 
 
+@pytest.mark.parametrize("d,hk,group,per", [(128, 8, 1, 63), (128, 8, 1, 64), (128, 8, 2, 97), (64, 8, 1, 70),
+                                            (64, 4, 4, 33), (32, 2, 8, 33), (64, 12, 4, 61), (128, 16, 8, 5)])
+def test_one_wave_items_beside_64_row_items_in_any_order(d, hk, group, per, device):
+    """Small items of one or more rows a head beside 64-row items, on both sides of the line from
+    which they go to the XCDs by KV head (2,048 items of one or two rows): every item runs once."""
+    nreq = -(-64 // group) + per
+    base = 8 * per
+    jobs = [Job((r,), tuple(range(8 * r + 4 * h, 8 * r + 4 * h + 1 + (r + h) % 3))) for h in (0, 1) for r in range(per)]
+    wide = range(per, nreq)
+    jobs += [Job((r,), tuple(range(base + 8 * i + o, base + 8 * i + o + 2))) for i, r in enumerate(wide) for o in (0, 3)]
+    root = base + 8 * len(wide)
+    jobs.append(Job(tuple(wide), tuple(range(root, root + 77))))
+    t = -(-(root + 77) // 8) * 8
+    g = torch.Generator().manual_seed(per)
+    q = torch.randn(nreq, group * hk, d, generator=g).bfloat16()
+    k = torch.randn(t, hk, d, generator=g).bfloat16()
+    v = torch.randn(t, hk, d, generator=g).bfloat16()
+    p = prepare(Plan(jobs, "x", 0.0, dict(kvheads=hk)), q.to(device), route_items=0, attach_tails=False)
+    say("one-wave beside 64 rows", d, hk, group, list(p.abi.n_items))
+    assert p.abi.n_items[_native.TA_SMALL] == 2 * nreq * hk and p.abi.n_items[_native.TA_LARGE64]
+    out = attention_matrix(q.to(device), *pack_kv(k.to(device), v.to(device)), p).cpu()
+    paths = [sum((tuple(j.tokens) for j in jobs if r in j.requests), ()) for r in range(nreq)]
+    ref = request_attention(q.float(), k.float(), v.float(), KVTree([], paths))
+    torch.testing.assert_close(out, ref.bfloat16(), atol=0.008, rtol=0.03)
+    assert relative_l2(out, ref) <= 3e-3
+
+
 @pytest.mark.parametrize("d,hq,hk,dtype", [(128, 32, 8, torch.bfloat16), (64, 8, 2, torch.float16)])
 @pytest.mark.parametrize("n", [319, 320, 321, 384, 385, 449, 1000])
 def test_copies_spread_over_steps(n, d, hq, hk, dtype, device):

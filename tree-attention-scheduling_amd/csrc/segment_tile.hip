@@ -707,16 +707,37 @@ __device__ __forceinline__ void tile_item(const SegParams &p, const int32_t *__r
     }
 }
 
-constexpr int ONE_ROUND = 5 * 256;  // one-wave workgroups that run at once at d = 128 (five 32 KiB tiles per CU)
+// One-wave items lie job by job with the KV heads inside.  Item i may go to XCD i % 8 ("by
+// head": an XCD works on one head of 8 and translates and caches an eighth of the pools)
+// or an XCD gets a range of jobs.  By head only where a head has four rows or more: items
+// of fewer rows write neighbouring pieces of the same cache lines (a row's entry of `lse`
+// is 8 bytes), and those then come from all XCDs, about 1.3 us a launch (32 requests x 128
+// tokens, 8 heads of 32, one row each: 6.9 us by job, 8.2 by head; 8 requests, 1024 shared
+// + 64 tokens, 8 heads of 128, four rows: 10.1 and 9.1).
+//
+// A launch of one-wave items alone goes by head only when they all run at once, five
+// workgroups of 32 KiB per CU at d = 128 (128 x 8192 private tokens, several rounds: 781 us
+// by job, 793 by head).  At d = 64 more of them do, but gain nothing (1,600 and 1,920 items
+// 11.1 and 11.9 us by job, 11.0 and 11.8 by head; 4,096 items 24.0 and 24.9).
+constexpr int ONE_ROUND = 5 * 256;
+__device__ inline bool tile_by_head(const SegParams &p, int items) {
+    return items <= ONE_ROUND && p.hk % 8 == 0 && p.group >= 4;
+}
+// Beside 64-row items also in several rounds (layers of 32 and 24 requests in two branches
+// 43.3 -> 42.5 us and 26.2 -> 25.1; 96 requests x 64 tokens, eight rows a head 28.8 -> 27.4),
+// and with fewer rows from two rounds of four a CU on at d = 128, whose 16-KiB runs then
+// weigh more (3,072 items of one row, 16 heads: 36.4 -> 33.7 us; 768 of them 16.6 -> 17.8;
+// d = 64 and 32 at 3,072 items 21.2 -> 22.0 and 13.5 -> 14.7).  Two heads gain nothing
+// (0.0-0.15 us slower by head), four are even.  Beside 256-row items, which fill whole CUs
+// by head already, four neighbours share a workgroup (by head 0.1-0.5 us slower).
+inline bool mix_by_head(const SegParams &p, const int n[3], int d) {
+    if (n[0] > 0 || p.hk % 4 != 0) return false;
+    return p.group >= 4 || (d == 128 && p.hk % 8 == 0 && n[2] >= 2 * 4 * 256);
+}
 template <int D, bool FP16, int NB, int NW, int STAGES, int L, bool SHORT = false>
 __global__ __launch_bounds__(64 * NW) void seg_tile_kernel(const int32_t *items, SegParams p) {
     __shared__ __attribute__((aligned(16))) u16 lds[STAGES * Tile<D>::ELEMS];
-    // One-wave items lie job by job with the KV heads inside: with item i on XCD i % 8 an
-    // XCD works on one head of 8 and translates and caches an eighth of the pools.  That
-    // helps a launch whose items all run at once (8 requests, 1024 shared + 64 tokens:
-    // layer 10.1 -> 9.1 us); a launch of several rounds keeps whole jobs on an XCD (128 x
-    // 8192 private tokens: 793 us by heads, 781 us by jobs).
-    const bool by_head = NW == 1 && p.hk % 8 == 0 && gridDim.x <= ONE_ROUND;
+    const bool by_head = NW == 1 && tile_by_head(p, gridDim.x);
     const int item = by_head ? blockIdx.x : xcd_item(blockIdx.x, gridDim.x);
     tile_item<D, FP16, NB, NW, STAGES, L, false, SHORT>(p, items, item, lds, threadIdx.x, 16 * NB * NW);
 }
@@ -1295,10 +1316,6 @@ __global__ __launch_bounds__(64 * NW) void seg_pipe_kernel(const int32_t *items,
 // waves end at once).  The bases are multiples of 8, so that the row tiles map
 // to XCDs as in their own kernels; blocks past a kind's item count end
 // at once.  The kinds run side by side instead of one launch after another.
-// Small items beside 64-row items keep item i on XCD i % 8 (one KV head of 8
-// per XCD; layers of 32 and 24 requests in two branches 43.3 -> 42.5 us and
-// 26.2 -> 25.1 us); beside 256-row items, which fill whole CUs by head already,
-// four neighbours share a workgroup (by head 0.1-0.5 us slower on two layers).
 template <int D, bool FP16, int L>
 __global__ __launch_bounds__(512) void seg_mix_kernel(const int32_t *items0, const int32_t *items1, const int32_t *items2,
                                                       MixParams mp) {
@@ -1315,7 +1332,7 @@ __global__ __launch_bounds__(512) void seg_mix_kernel(const int32_t *items0, con
         tile_item<D, FP16, 1, 8, 3, L>(mp.p, items1, xcd_item(lb, mp.n[1]), lds, tid, 64);
     } else {
         const int lb = b - mp.base[2], wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-        const int it = mp.n[0] ? 4 * lb + wave : 8 * (4 * (lb >> 3) + wave) + (lb & 7);
+        const int it = mp.by_head ? 8 * (4 * (lb >> 3) + wave) + (lb & 7) : 4 * lb + wave;
         if (wave >= 4 || it >= mp.n[2]) return;
         tile_item<D, FP16, 1, 1, 1, L, true>(mp.p, items2, it, lds + wave * T::ELEMS, tid & 63, 16);
     }
@@ -1540,7 +1557,8 @@ hipError_t launch_mix<TA_LAYOUT>(const SegParams &sp, const int32_t *const items
         mp.base[k] = base;
         base += (mp.n[k] + 7) & ~7;  // (the last kind's is not needed)
     }
-    const int small_blocks = n[0] > 0 ? (mp.n[2] + 3) / 4 : (mp.n[2] + 31) / 32 * 8;
+    mp.by_head = mix_by_head(sp, mp.n, d);
+    const int small_blocks = mp.by_head ? (mp.n[2] + 31) / 32 * 8 : (mp.n[2] + 3) / 4;
     const int blocks = mp.base[2] + small_blocks;
     if (blocks <= 0) return hipSuccess;
     TA_BY_SHAPE(launch_mix_d, TA_LAYOUT, mp, blocks, stream)

@@ -190,6 +190,7 @@ struct MixParams {
     const int32_t *items[3];
     int n[3];
     int base[3];
+    int by_head;  // small items go to the XCDs by KV head (mix_by_head)
 };
 
 // Where K and V lie (template argument of the segment kernels).
