@@ -132,6 +132,45 @@ def test_odd_capacity_same_bits_in_every_kind(n, nreq, device):
     assert relative_l2(outs[0].cpu(), ref) <= 3e-3
 
 
+@pytest.mark.parametrize("pad", [0, 3])
+@pytest.mark.parametrize("nreq,tile_rows", [(3, 256), (14, 256), (30, 128), (64, 256)])
+def test_a_job_without_requests_writes_nothing(nreq, tile_rows, pad, device):
+    """``ta_segment`` on a job whose qlen is 0 (a C caller's, ``prepare`` makes none): no row is
+    read or written for it, and the other jobs' partials are the same."""
+    n = 96
+    jobs = [Job(tuple(range(nreq)), tuple(range(n * i, n * i + 90 - i))) for i in range(3)]
+    g = torch.Generator().manual_seed(nreq)
+    q = torch.randn(nreq, 32, 128, generator=g).bfloat16().to(device)
+    k = torch.randn(3 * n + pad, 8, 128, generator=g).bfloat16().to(device)
+    v = torch.randn(3 * n + pad, 8, 128, generator=g).bfloat16().to(device)
+    kp, vp = pack_kv(k, v)
+    p = prepare(Plan(jobs, "x", 0.0, dict(kvheads=8)), q, tile_rows=tile_rows, route_items=0, consolidate_rows=0,
+                large_target=1, small_target=1, attach_tails=False)
+    abi, lib = p.abi, _native.load()
+    kind = next(i for i in range(_native.TA_NKINDS) if abi.n_items[i])
+    qlen = p.qlen.clone()
+    say("no requests", nreq, kind, pad, list(abi.n_items), qlen.tolist())
+
+    def run():
+        p.part.zero_()
+        _native.check(lib.ta_segment(q.data_ptr(), kp.data_ptr(), vp.data_ptr(), abi.qids, abi.kstart, qlen.data_ptr(),
+                                     abi.klen, abi.rowbase, abi.items[kind], abi.n_items[kind], kind, abi.part,
+                                     abi.lse, abi.nreq, abi.hq, abi.hk, abi.d, kp.shape[2], abi.maxr, abi.dtype,
+                                     torch.cuda.current_stream().cuda_stream))
+        return p.part.clone()
+
+    whole = run()
+    for job in (0, len(p.jobs) - 1):
+        qlen.copy_(p.qlen)
+        qlen[job] = 0
+        a = int(p.rowbase[job])
+        part = run()
+        assert not part[a:a + nreq].any() and whole[a:a + nreq].any()
+        whole_rest = whole.clone()
+        whole_rest[a:a + nreq] = 0
+        assert torch.equal(part, whole_rest)
+
+
 def test_token_major_equals_packed(device):
     """Token-major K/V give the bits of the packed pools of an aligned capacity (same tiles, same
     order), attachments included; views that are not contiguous are packed as before."""

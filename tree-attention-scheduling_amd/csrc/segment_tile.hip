@@ -621,15 +621,16 @@ __device__ __forceinline__ void tile_item(const SegParams &p, const int32_t *__r
     // past the item repeat its last row and are never stored).  A job over
     // consecutive requests (qbase) needs no request-id loads.  The first tile's
     // copies go out behind the Q loads, so that one wait covers both.
+    const int last = max(nrows, 1) - 1;  // (a job without requests reads a row and stores none)
     u32x4 qf[NB][KS];
     const u16 *qsrc[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-        const int rr = min(wrow0 + 16 * nb + row, nrows - 1);
+        const int rr = min(wrow0 + 16 * nb + row, last);
         const int lr = rr / p.group;
         int rq = qb + lr;
         if (qb < 0) {
-            rq = p.qids[(size_t)job * p.maxr + lr];
+            rq = nrows > 0 ? p.qids[(size_t)job * p.maxr + lr] : 0;
             asm volatile("" : "+v"(rq));  // waited for in this branch only
         }
         qsrc[nb] = p.q + ((size_t)rq * p.hq + h * p.group + (rr - lr * p.group)) * D + 8 * g4;
@@ -1030,6 +1031,8 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
     const int ntok = max(0, min(p.klen[job], p.tcap - kst));
     const int kend = kst + ntok;
     const int nrows = p.qlen[job] * p.group;
+    if constexpr (odd_count(L))
+        if (nrows <= row0) return;  // (a job without requests)
     const int wrow0 = row0 + 16 * NB * wave;
     const bool active = wrow0 < nrows;
     const float c = p.scale_log2, rc = 1.f / p.scale_log2;
