@@ -132,6 +132,30 @@ def test_odd_capacity_same_bits_in_every_kind(n, nreq, device):
     assert relative_l2(outs[0].cpu(), ref) <= 3e-3
 
 
+@pytest.mark.parametrize("start", [2 ** 31 - 400, 2 ** 31 - 100])
+@pytest.mark.parametrize("nreq", [4, 14, 40, 64])
+def test_a_job_far_beyond_the_pool_adds_nothing(nreq, start, device):
+    """Jobs whose tokens all lie past the pool, up to the largest ids there are, contribute
+    nothing in any kind (no sum of ids and tile sizes may wrap around)."""
+    n = 333
+    g = torch.Generator().manual_seed(nreq)
+    q = torch.randn(nreq, 32, 128, generator=g).bfloat16().to(device)
+    k = torch.randn(n, 8, 128, generator=g).bfloat16().to(device)
+    v = torch.randn(n, 8, 128, generator=g).bfloat16().to(device)
+    everyone = tuple(range(nreq))
+    jobs = [Job(everyone, tuple(range(n))), Job(everyone, tuple(range(start, start + 90)))]
+    for pad in (0, 3):
+        kp, vp = pack_kv(torch.cat([k, k[:pad + 3]]), torch.cat([v, v[:pad + 3]]))
+        for tile_rows in (64, 128, 256):
+            opts = dict(tile_rows=tile_rows, route_items=0, consolidate_rows=0, large_target=1, small_target=1)
+            out = []
+            for js in (jobs, jobs[:1]):
+                p = prepare(Plan(js, "x", 0.0, dict(kvheads=8)), q, **opts)
+                say("beyond", nreq, start, pad, tile_rows, list(p.abi.n_items))
+                out.append(attention_matrix(q, kp, vp, p).clone())
+            assert torch.equal(*out)
+
+
 @pytest.mark.parametrize("pad", [0, 3])
 @pytest.mark.parametrize("nreq,tile_rows", [(3, 256), (14, 256), (30, 128), (64, 256)])
 def test_a_job_without_requests_writes_nothing(nreq, tile_rows, pad, device):

@@ -1198,7 +1198,7 @@ __device__ __forceinline__ void pipe_item(const SegParams &p, const int32_t *__r
     constexpr int NH = T::KBLK / NW;  // copies of K, and of V, of one wave
     if constexpr (L == KV_POOL && SYNC == 1 && T::KBLK % NW == 0 && NH * NW == T::VBLK) {
         // (readfirstlane: a lane-dependent branch here would move `issued` to vector registers)
-        if (__builtin_amdgcn_readfirstlane(active) && p.tcap <= SHORT_CAP && tb0 + STAGES * T::TT <= kend) {
+        if (__builtin_amdgcn_readfirstlane(active) && p.tcap <= SHORT_CAP && (u32)tb0 + STAGES * T::TT <= (u32)kend) {
             constexpr int EVERY = 4;  // slots from one copy to the next
             static_assert(EVERY * NH <= 2 * KS * NB, "the copies fit the step's QK slots");
             const int w = __builtin_amdgcn_readfirstlane(wave);
