@@ -125,3 +125,20 @@ def test_native_lowering_leaves_bad_requests_to_prepare():
     plan = Plan([Job((0, 5), (0, 1, 2))], "x", 0.0, dict(kvheads=1))
     with pytest.raises(ValueError, match="names request 5"):
         prepare(plan, torch.empty(2, 4, 32, dtype=torch.float16))
+
+
+@pytest.mark.parametrize("opts", [dict(fixed_from=-1), dict(fixed_from=-7), dict(fixed_from=64.0),
+                                  dict(large_target=200.5, small_target=float("inf")), dict(large_target=10 ** 20),
+                                  dict(consolidate_rows=None)])
+def test_options_that_are_not_small_ints(opts):
+    """Targets and limits may be any numbers; a negative fixed_from keeps every job as it is."""
+    from tree_attention import kernels
+    plan = random_plan(random.Random(7), 40)
+    q = torch.empty(40, 8, 128, dtype=torch.bfloat16)
+    p = prepare(plan, q, **opts)
+    full = {**dict(tile_rows=256, fixed_from=None, attach_tails=True, route_items=kernels.ROUTE_ITEMS,
+                   fuse_rows=kernels.FUSE_ROWS, consolidate_rows=kernels.CONSOLIDATE_ROWS, large_target=256,
+                   small_target=2048, large_min_tiles=kernels.LARGE_MIN_TILES), **opts}
+    jobs, small, attached = kernels._lower_py(list(plan.jobs), 256, kvheads=2, group=4, **full)
+    assert p.jobs == jobs and p.small_jobs == small
+    assert p.attached == {(j + small, row0): segs for (j, row0), segs in attached.items()}

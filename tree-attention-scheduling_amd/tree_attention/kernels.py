@@ -601,11 +601,15 @@ def _lower(jobs, nreq, n_cu, **options):
     from . import _planner
     if _planner.available() and all(0 <= j.tokens[0] and j.tokens[0] + len(j.tokens) < 2 ** 31 for j in jobs):
         o = options
-        got = _planner.lower(jobs, nreq, (
-            o["kvheads"], o["group"], o["tile_rows"], bool(o["attach_tails"]), o["consolidate_rows"], o["large_target"],
-            o["large_min_tiles"], n_cu, -1 if o["fixed_from"] is None else o["fixed_from"], XTAIL_MAX, WAVE_ROWS,
-            ATTACH_MIN_CAP, o["small_target"], TOKEN_QUANTUM, o["route_items"], o["fuse_rows"], TAIL_KEEP_TILES,
-            TAIL_KEEP_ITEMS_PER_CU, bool(SMALL_PAIRS)))
+        fixed = -1 if o["fixed_from"] is None else max(o["fixed_from"], 0)  # (no token id is below 0)
+        try:
+            got = _planner.lower(jobs, nreq, (
+                o["kvheads"], o["group"], o["tile_rows"], bool(o["attach_tails"]), o["consolidate_rows"],
+                o["large_target"], o["large_min_tiles"], n_cu, fixed, XTAIL_MAX, WAVE_ROWS, ATTACH_MIN_CAP,
+                o["small_target"], TOKEN_QUANTUM, o["route_items"], o["fuse_rows"], TAIL_KEEP_TILES,
+                TAIL_KEEP_ITEMS_PER_CU, bool(SMALL_PAIRS)))
+        except (TypeError, OverflowError):  # options or ids that are not ints of its sizes
+            got = None
         if got is not None:
             triples, small_jobs, att = got
             out, new, put = [], object.__new__, object.__setattr__
