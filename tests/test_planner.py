@@ -246,6 +246,15 @@ def test_subclassed_cost_model_is_honoured():
     plan.validate(tree)
 
 
+def test_cost_set_on_a_model_prices_every_job():
+    """A cost function set on one model object is asked for every job, whatever its sizes."""
+    tree = KVTree.synthetic([-1, 0, 0], [100, 10, 10], [1, 2])
+    model = CostModel()
+    model.cost = lambda requests, tokens, *heads: float(tokens[0])
+    plan = schedule(tree, method="fixed", model=model)
+    assert plan.estimated_us == sum(job.tokens[0] for job in physical_jobs(plan.jobs)) == 100 + 110
+
+
 def test_calibration_coordinate_search():
     """calibrate.tune_terms scales one continuous term at a time (1/4 .. 4x), or sets a per-job
     term to an absolute level, and keeps the best change while the measured cube plans get at

@@ -214,7 +214,7 @@ def schedule(tree: KVTree, qheads=32, kvheads=8, dim=128, method="cube", model=N
         return out
 
     # the reference's cost depends on the two counts alone: one evaluation per pair
-    by_counts = {} if type(model).cost is CostModel.cost else None
+    by_counts = {} if getattr(model.cost, "__func__", None) is CostModel.cost else None
 
     def plan_cost(jobs):
         total = 0
