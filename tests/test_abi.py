@@ -5,8 +5,10 @@ import subprocess
 from pathlib import Path
 
 import pytest
+import torch
 
-from tree_attention import _native
+from tree_attention import _native, kernels
+from tree_attention.schedule import Job, Plan
 
 ROOT = Path(__file__).resolve().parent.parent
 HEADER = ROOT / "include" / "tree_attn.h"
@@ -109,3 +111,59 @@ def test_decode_append_rejects_host_slots_outside_the_pool():
             decode_append(q, k, v, cos, sin, bad, kp, vp)
     with pytest.raises(ValueError, match="one pool position per request"):
         decode_append(q, k, v, cos, sin, [0, 1], kp, vp)
+
+
+@pytest.fixture
+def fresh(monkeypatch):
+    """The module as it is before the first load."""
+    monkeypatch.setattr(_native, "_lib", None)
+    monkeypatch.setattr(_native, "fastcall", None)
+    monkeypatch.delenv("TREE_ATTN_LIB", raising=False)
+    return monkeypatch
+
+
+def test_host_module_is_the_one_that_runs(fresh):
+    lib = _native.load()
+    assert _native.fastcall is not _native.GeneralPath and _native.fastcall.BUILT_FOR.startswith("cpython")
+    assert lib is _native.load()
+
+
+def test_host_module_missing_or_built_for_another_torch(fresh, tmp_path):
+    """Every call then takes the general path, with a warning: the module is no requirement."""
+    fresh.setattr(_native, "FASTCALL_PATH", tmp_path / "_fastcall.so")
+    with pytest.warns(RuntimeWarning, match="not used"):
+        lib = _native.load()
+    assert _native.fastcall is _native.GeneralPath and lib is _native.load()
+    assert _native.fastcall.attention(1, 2, 3, 4, 5, 6) is None and _native.fastcall.fill(1, 2, 3) is None
+    fresh.undo()
+    fresh.setattr(_native, "_lib", None)
+    fresh.setattr(torch, "__version__", "0.0.0")
+    with pytest.warns(RuntimeWarning, match="built for"):
+        _native.load()
+    assert _native.fastcall is _native.GeneralPath
+
+
+def test_library_without_the_host_modules_calls(fresh, tmp_path):
+    """A library that TREE_ATTN_LIB selects may lack ta_attention_tokens and ta_fill_lengths."""
+    names = [n for n in _native.EXPORTS if n not in ("ta_attention_tokens", "ta_fill_lengths")]
+    src = tmp_path / "old.c"
+    src.write_text("".join(f"int {n}(void) {{ return 0; }}\n" for n in names))
+    old = tmp_path / "libold.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(old)], check=True)
+    fresh.setenv("TREE_ATTN_LIB", str(old))
+    with pytest.warns(RuntimeWarning, match="ta_attention_tokens"):
+        _native.load()
+    assert _native.fastcall is _native.GeneralPath
+
+
+def test_arguments_are_checked_before_the_library_is_needed(fresh, tmp_path):
+    fresh.setattr(_native, "LIB_PATH", tmp_path / "libtree_attn.so")
+    q = torch.zeros(2, 8, 32, dtype=torch.bfloat16)
+    prepared = kernels.prepare(Plan([Job((0, 1), (0, 1, 2))], "x", 0.0, dict(kvheads=2)), q)
+    kp, vp = torch.zeros(2, 32, 8, dtype=torch.bfloat16), torch.zeros(2, 8, 32, dtype=torch.bfloat16)
+    with pytest.raises(ValueError, match="share dtype"):
+        kernels.attention_matrix(q.float(), kp, vp, prepared)
+    with pytest.raises(ValueError, match="same GPU"):
+        kernels.attention(q, kp.permute(2, 0, 1).contiguous(), vp.transpose(0, 1).contiguous(), prepared)
+    with pytest.raises(RuntimeError, match="not found"):
+        kernels.merge(prepared)

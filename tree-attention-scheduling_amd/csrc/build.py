@@ -107,6 +107,7 @@ def build_fastcall(verbose: bool = False, out: Path | None = None) -> Path:
         raise RuntimeError("g++ not found; it is required to build the host module")
     lib = Path(torch.__file__).parent / "lib"
     _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          f'-DTA_BUILT_FOR="{sys.implementation.cache_tag} torch {torch.__version__}"',
           *[f"-isystem{p}" for p in include_paths()], f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}",
           str(HERE / "fastcall.cpp"), f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-o", str(tmp)],
          verbose)

@@ -224,4 +224,13 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fastcall", nullptr, -1, methods};
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__fastcall(void) { return PyModule_Create(&module); }
+// BUILT_FOR names the Python and the torch whose object layouts the module was compiled with;
+// _native uses it with no other.
+PyMODINIT_FUNC PyInit__fastcall(void) {
+    PyObject *m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "BUILT_FOR", TA_BUILT_FOR) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

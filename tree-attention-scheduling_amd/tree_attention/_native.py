@@ -12,7 +12,9 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import sys
 import threading
+import warnings
 from pathlib import Path
 
 LIB_PATH = Path(__file__).with_name("libtree_attn.so")
@@ -48,13 +50,20 @@ class TaPlan(ctypes.Structure):
 
 
 _lib = None
-fastcall = None  # the host module of the per-layer calls, set by load()
+
+
+class GeneralPath:
+    """Stands in for the host module where it cannot be used: every call takes the general path."""
+    attention = decode_append = fill = staticmethod(lambda *args: None)
+
+
+fastcall = None  # the host module of the per-layer calls or GeneralPath, set by load()
 _lock = threading.Lock()
 
 
 def load(path: Path | str | None = None) -> ctypes.CDLL:
     """Load (once) and return the native library, with prototypes set."""
-    global _lib
+    global _lib, fastcall
     if _lib is not None and path is None:
         return _lib
     with _lock:
@@ -81,9 +90,13 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
         lib.ta_attention_matrix.restype = ctypes.c_int
         lib.ta_attention_matrix.argtypes = [_c_ptr, _c_ptr, _c_ptr, _c_i32, ctypes.POINTER(TaPlan),
                                             _c_ptr, _c_ptr]
-        lib.ta_attention_tokens.restype = ctypes.c_int
-        lib.ta_attention_tokens.argtypes = [_c_ptr, _c_ptr, _c_ptr, _c_i32, ctypes.POINTER(TaPlan),
-                                            _c_ptr, _c_ptr]
+        if hasattr(lib, "ta_attention_tokens"):  # (a library built before the two calls has neither)
+            lib.ta_attention_tokens.restype = ctypes.c_int
+            lib.ta_attention_tokens.argtypes = [_c_ptr, _c_ptr, _c_ptr, _c_i32, ctypes.POINTER(TaPlan),
+                                                _c_ptr, _c_ptr]
+        if hasattr(lib, "ta_fill_lengths"):
+            lib.ta_fill_lengths.restype = ctypes.c_int
+            lib.ta_fill_lengths.argtypes = [_c_ptr, _c_ptr, _c_i32, _c_i32, _c_ptr]
         lib.ta_attention_matrix_noalloc.restype = ctypes.c_int
         lib.ta_attention_matrix_noalloc.argtypes = [_c_ptr, _c_ptr, _c_ptr, _c_i32, ctypes.POINTER(TaPlan),
                                                     _c_ptr, _c_ptr]
@@ -96,32 +109,39 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
         lib.ta_decode_append.restype = ctypes.c_int
         lib.ta_decode_append.argtypes = [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i32, _c_ptr, _c_ptr, _c_ptr,
                                          _c_ptr, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_ptr]
-        lib.ta_fill_lengths.restype = ctypes.c_int
-        lib.ta_fill_lengths.argtypes = [_c_ptr, _c_ptr, _c_i32, _c_i32, _c_ptr]
         lib.ta_time_next_launch.restype = ctypes.c_int
         lib.ta_time_next_launch.argtypes = [_c_ptr, _c_ptr]
         lib.ta_read_stream.restype = ctypes.c_int
         lib.ta_read_stream.argtypes = [_c_ptr, ctypes.c_int64, _c_ptr, _c_i32, _c_ptr]
         if path is None:
-            _bind_fastcall(lib)
+            fastcall = _host_module(lib)
             _lib = lib
         return lib
 
 
-def _bind_fastcall(lib) -> None:
-    """Load the host module of the per-layer calls (csrc/fastcall.cpp) and give it ``lib``'s functions."""
-    global fastcall
+def _host_module(lib):
+    """The host module of the per-layer calls (csrc/fastcall.cpp) with ``lib``'s functions bound.
+
+    ``GeneralPath`` and a warning where it is missing, was built for another Python or torch
+    (it holds torch's C++ layouts), or ``lib`` lacks a call of its: the results are the same,
+    the calls cost the host more (see the times in fastcall.cpp).
+    """
     import torch
-    if not FASTCALL_PATH.exists():
-        raise RuntimeError(f"tree_attn host module not found at {FASTCALL_PATH}; build it with "
-                           "`python -c 'import __graft_entry__ as g; g.build()'` from the repository root")
-    loader = importlib.machinery.ExtensionFileLoader("_fastcall", str(FASTCALL_PATH))
-    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_fastcall", loader))
-    loader.exec_module(module)
-    module.bind(*(ctypes.cast(getattr(lib, name), _c_ptr).value for name in
-                  ("ta_attention_matrix", "ta_attention_tokens", "ta_decode_append", "ta_fill_lengths")),
-                torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice)
-    fastcall = module
+    calls = ("ta_attention_matrix", "ta_attention_tokens", "ta_decode_append", "ta_fill_lengths")
+    here = f"{sys.implementation.cache_tag} torch {torch.__version__}"
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("_fastcall", str(FASTCALL_PATH))
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_fastcall", loader))
+        loader.exec_module(module)
+        if module.BUILT_FOR != here:
+            raise ImportError(f"built for {module.BUILT_FOR}, not for {here}")
+        module.bind(*(ctypes.cast(getattr(lib, name), _c_ptr).value for name in calls),
+                    torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice)
+        return module
+    except (ImportError, AttributeError) as e:
+        warnings.warn(f"tree_attn host module {FASTCALL_PATH} not used ({e}); build it with `python -c 'import "
+                      "__graft_entry__ as g; g.build()'` from the repository root", RuntimeWarning, stacklevel=3)
+        return GeneralPath
 
 
 def check(rc: int) -> None:

@@ -880,9 +880,13 @@ def attention(q, k, v, prepared):
 
 
 def _fastcall():
-    """The host module of the per-layer calls (csrc/fastcall.cpp)."""
+    """The host module of the per-layer calls (csrc/fastcall.cpp).  Without the library, the
+    general path: it checks a call's arguments before it needs the library."""
     if _native.fastcall is None:
-        _native.load()
+        try:
+            _native.load()
+        except (RuntimeError, OSError):
+            return _native.GeneralPath
     return _native.fastcall
 
 
