@@ -211,3 +211,32 @@ def test_native_metadata_equals_numpy():
         for key in ("maxr", "maxs", "nslot", "contiguous_q", "slot_stride"):
             assert a[key] == b[key], key
         assert np.array_equal(a["qbase"], b["qbase"])
+
+
+def test_arrays_live_until_the_library_has_used_them(monkeypatch):
+    """Every array whose address goes into tp_attach_tails and tp_build_metadata is alive during
+    the call, also where the binding makes it: no candidates, records that are not contiguous."""
+    import weakref
+    refs, calls, lib, address = [], [], _planner.load(), _planner._ptr
+
+    class Checked:
+        def __getattr__(self, name):
+            def call(*args):
+                calls.append(name)
+                assert all(ref() is not None for ref in refs), name
+                return getattr(lib, name)(*args)
+            return call
+
+    monkeypatch.setattr(_planner, "_ptr", lambda a: refs.append(weakref.ref(a)) or address(a))
+    monkeypatch.setattr(_planner, "load", lambda: Checked())
+    from tree_attention.schedule import Job
+    big = Job(tuple(range(64)), tuple(range(300)))
+    _planner.attach_tails([big], [], 4, [True], [5], [], [], 64, 4, 32, 256, 8)
+    refs.clear()
+    ints = [np.array(x, dtype=np.int32) for x in ([64], list(range(64)), [0], [300], [0], [0])]
+    records = np.arange(34, dtype=np.int32).reshape(1, 34)
+    a = _planner.build_metadata(*ints[:4], 0, 64, 4, 2, 256, ints[4], ints[5], records[:, ::2], 17)
+    refs.clear()
+    b = _planner.build_metadata(*ints[:4], 0, 64, 4, 2, 256, ints[4], ints[5], records[:, ::2].copy(), 17)
+    assert a[0] == b[0] and np.array_equal(a[1], b[1])
+    assert calls == ["tp_attach_tails"] + ["tp_build_metadata"] * 4

@@ -66,6 +66,7 @@ def available() -> bool:
 
 
 def _ptr(a: np.ndarray):
+    """The address of ``a``'s data; the caller keeps ``a`` alive until the library has used it."""
     return a.__array_interface__["data"][0]  # (an int: ctypes.data_as costs four times as much)
 
 
@@ -144,7 +145,7 @@ def attach_tails(large, small, group, is256, large_tiles, small_tiles, fixed, nr
     np.cumsum([len(j.requests) for j in small], out=sreq_off[1:])
     sreq = np.fromiter(chain.from_iterable(j.requests for j in small), dtype=np.int32, count=int(sreq_off[-1]))
     tiles_s = np.asarray(small_tiles, dtype=np.int32)
-    fixed = np.asarray(fixed, dtype=np.int8)
+    fixed = np.asarray(fixed, dtype=np.int8) if ns else np.zeros(1, dtype=np.int8)
     cap = int(sum(-(-len(j.requests) * group // item_rows) for j, b in zip(large, is256) if b))
     item = np.zeros(max(ns, 1), dtype=np.int32)
     lrow = np.zeros(max(ns, 1), dtype=np.int32)
@@ -154,7 +155,7 @@ def attach_tails(large, small, group, is256, large_tiles, small_tiles, fixed, nr
     one = np.zeros(1, dtype=np.int32)
     ptr = lambda a: _ptr(a if a.size else one)  # noqa: E731
     rc = lib.tp_attach_tails(nl, ptr(is256), ptr(tiles), _ptr(req_off), ptr(req), group, ns, _ptr(sreq_off), ptr(sreq),
-                             ptr(tiles_s), _ptr(fixed if fixed.size else np.zeros(1, np.int8)), nreq, xtail_max,
+                             ptr(tiles_s), _ptr(fixed), nreq, xtail_max,
                              wave_rows, item_rows, min_cap, _ptr(item), _ptr(lrow), _ptr(item_job), _ptr(item_row0),
                              _ptr(n_items))
     if rc != 0:
@@ -170,8 +171,9 @@ def build_metadata(qlen, req, kstart, klen, small_jobs, nreq, group, kvheads, ti
     one = np.zeros(1, dtype=np.int32)
     ptr = lambda a: _ptr(a if a.size else one)  # noqa: E731
     sizes = np.zeros(13, dtype=np.int32)
+    att_rec = np.ascontiguousarray(att_rec, dtype=np.int32).reshape(-1)
     args = (len(qlen), small_jobs, ptr(qlen), ptr(req), ptr(kstart), ptr(klen), nreq, group, kvheads, tile_rows,
-            len(att_job), ptr(att_job), ptr(att_row0), ptr(np.ascontiguousarray(att_rec).reshape(-1)), xstride,
+            len(att_job), ptr(att_job), ptr(att_row0), ptr(att_rec), xstride,
             _ptr(sizes))
     if lib.tp_build_metadata(*args, None, 0) != 0:
         raise ValueError("tp_build_metadata rejected its arguments")
