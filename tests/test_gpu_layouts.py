@@ -323,6 +323,57 @@ def test_one_wave_items_beside_64_row_items_in_any_order(d, hk, group, per, devi
     assert relative_l2(out, ref) <= 3e-3
 
 
+@pytest.mark.parametrize("d,cap", [(32, 2 ** 28 + 8), (64, 2 ** 28), (64, 2 ** 28 + 8)])
+def test_pools_past_the_short_offsets(d, cap, device):
+    """Pools of more than 2**28 tokens (34 and 69 GB here) take 64-bit lane addresses in one-wave
+    items and leave the spread copies of 256-row items: the bits of the same tokens in a small
+    pool, at the end of the large one and across its 2**28-th token."""
+    n, nreq, group = 700, 40, 8
+    first = cap - 1024
+    g = torch.Generator().manual_seed(d)
+    q = torch.randn(nreq, group, d, generator=g).bfloat16().to(device)
+    small = [torch.randn(1, d, 1024, generator=g).bfloat16().to(device),
+             torch.randn(1, 1024, d, generator=g).bfloat16().to(device)]
+    kp = torch.empty(1, d, cap, dtype=torch.bfloat16, device=device)
+    vp = torch.empty(1, cap, d, dtype=torch.bfloat16, device=device)
+    kp[:, :, first:] = small[0]
+    vp[:, first:] = small[1]
+    for attach in (True, False):
+        outs = []
+        for base, pools in ((first, (kp, vp)), (0, small)):
+            jobs = [Job(tuple(range(nreq)), tuple(range(base + 3, base + 3 + n)))]
+            jobs += [Job((r,), tuple(range(base + 710 + 7 * r, base + 715 + 7 * r))) for r in range(nreq)]
+            p = prepare(Plan(jobs, "x", 0.0, dict(kvheads=1)), q, attach_tails=attach, route_items=0, large_target=1)
+            say("large pool", d, cap, list(p.abi.n_items), len(p.attached))
+            outs += [attention_matrix(q, *pools, p).clone()]
+            plain = prepare(Plan(jobs[1:], "x", 0.0, dict(kvheads=1)), q, small_target=1)
+            jobs2 = [Job((r,), tuple(range(base + 9 * r + o, base + 9 * r + o + 4))) for o in (0, 5) for r in range(nreq)]
+            pair = prepare(Plan(jobs2, "x", 0.0, dict(kvheads=1)), q, small_target=1)
+            assert pair.abi.n_items[_native.TA_SMALL] == 2 * nreq
+            outs += [attention_matrix(q, *pools, plain).clone(), attention_matrix(q, *pools, pair).clone()]
+        assert all(torch.equal(a, b) for a, b in zip(outs[:3], outs[3:]))
+    del kp, vp, pools
+    torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("hk", [2 ** 18 - 1, 2 ** 18, 270_000])
+def test_token_major_rows_past_the_short_offsets(hk, device):
+    """Token-major rows so wide that 64 of them pass 4 GiB (d = 128, 2**18 heads): the bits of
+    the packed pools."""
+    n, d = 64, 128
+    q = torch.randn(1, hk, d, dtype=torch.bfloat16, device=device)
+    k = torch.randn(n, hk, d, dtype=torch.bfloat16, device=device)
+    v = torch.randn(n, hk, d, dtype=torch.bfloat16, device=device)
+    p = prepare(Plan([Job((0,), tuple(range(30))), Job((0,), tuple(range(31, n)))], "x", 0.0, dict(kvheads=hk)), q,
+                small_target=1)
+    say("wide rows", hk, list(p.abi.n_items))
+    assert p.abi.n_items[_native.TA_SMALL] == 2 * hk
+    a = attention(q, k, v, p).clone()
+    assert torch.equal(a, attention_matrix(q, *pack_kv(k, v), p))
+    del k, v
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("d,hq,hk,dtype", [(128, 32, 8, torch.bfloat16), (64, 8, 2, torch.float16)])
 @pytest.mark.parametrize("n", [319, 320, 321, 384, 385, 449, 1000])
 def test_copies_spread_over_steps(n, d, hq, hk, dtype, device):

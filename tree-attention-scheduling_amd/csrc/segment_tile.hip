@@ -180,9 +180,8 @@ struct TileCopy {
     static constexpr int NK = (T::KBLK + NW - 1) / NW;  // K blocks of a wave, V likewise (D = 32: of some waves)
     u32x4 k[L == KV_ODD ? NK : 1];
 
-    // SHORT: a copy's source is a scalar base per block plus a 32-bit lane offset that all tiles
-    // of an item share (8 K rows span 14 tcap bytes, so tcap <= SHORT_CAP); else a 64-bit address
-    // per lane.  In the one-wave kernel the short form streams 128 x 8192 private tokens in 768
+    // SHORT (short_offsets): a copy's source is a scalar base per block plus a 32-bit lane offset
+    // that all tiles of an item share; else a 64-bit address per lane.  In the one-wave kernel the short form streams 128 x 8192 private tokens in 768
     // us against 782 us; in the mixed kernel, whose scalar registers are full, it is the slower
     // one (32 requests x 4096 tokens: 42.8 us against 41.8 us).
     __device__ static void dma(u16 *dst, const u16 *base, u32 ofs) {
@@ -1499,6 +1498,13 @@ hipError_t launch_tail_merge(const SegParams &sp, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// Whether the 32-bit lane offsets of TileCopy's short form cover a tile: 8 K rows of a pool span
+// 14 tcap bytes; the 64 rows of token-major K and V 128 D hk, whatever their number.
+template <int D, int L>
+bool short_offsets(const SegParams &p) {
+    return token_major(L) ? p.hk < (1 << 25) / D : L == KV_POOL && p.tcap <= SHORT_CAP;
+}
+
 template <int D, bool FP16, int L>
 hipError_t launch_d(const SegParams &sp, int kind, hipStream_t stream) {
     switch (kind) {
@@ -1511,7 +1517,7 @@ hipError_t launch_d(const SegParams &sp, int kind, hipStream_t stream) {
             }
             [[fallthrough]];
         case TA_SMALL:  // one wave per (job, head); one stage so that five fit on a CU
-            if (L != KV_ODD && sp.tcap <= SHORT_CAP)
+            if (short_offsets<D, L>(sp))
                 TA_LAUNCH((seg_tile_kernel<D, FP16, 1, 1, 1, L, L != KV_ODD>), dim3(sp.n_items), dim3(64), stream,
                           sp.items, sp);
             else
