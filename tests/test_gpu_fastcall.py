@@ -4,11 +4,13 @@ Every form that the calls accept -- contiguous or not, any slot type, one RoPE r
 request, an output given or not, another stream -- gives the bits that the ctypes path gives,
 and what was refused is refused with the same error.
 """
+import ctypes
+
 import pytest
 import torch
 
 from tree_attention import CostModel, schedule, shapes
-from tree_attention import _native, kernels
+from tree_attention import _native
 from tree_attention.kernels import CachedDecodePlan, attention_matrix, decode_append, pack_kv, prepare
 
 pytestmark = pytest.mark.gpu
@@ -108,4 +110,87 @@ def test_fill_growing(requests, device, general):
         fast = c.update(n).metadata.clone()
         c.update(7)
         want = general(lambda: c.update(n).metadata.clone())
-        assert torch.equal(fast, want) and kernels._fastcall().fill is not None
+        assert torch.equal(fast, want)
+
+
+def test_attention_calls_that_the_module_takes(device):
+    """The ordinary call is handled by the module itself (it returns the library's code), on any
+    stream; every other form is left to the general path (None)."""
+    tree = shapes.tree(shapes.shared_prefix(32, 2043, 60))
+    for dtype in (torch.bfloat16, torch.float16):
+        g = torch.Generator().manual_seed(3)
+        q = torch.randn(32, 32, 128, generator=g).to(dtype).to(device)
+        k = torch.randn(tree.storage_tokens + 5, 8, 128, generator=g).to(dtype).to(device)
+        v = torch.randn(tree.storage_tokens + 5, 8, 128, generator=g).to(dtype).to(device)
+        assert k.shape[0] % 8 == 0
+        plan = schedule(tree, 32, 8, 128, "cube", CostModel.mi355x())
+        attached, plain = prepare(plan, q), prepare(plan, q, attach_tails=False)
+        assert attached.attached
+        _native.load()
+        call = _native.fastcall.attention
+
+        def run(p, q, k, v, tokens=False):
+            return call(q, k, v, ctypes.addressof(p.abi), p.out, tokens)
+
+        even, odd = (k, v), (k[:-3], v[:-3])
+        side = torch.cuda.Stream()
+        for p in (attached, plain):
+            assert run(p, q, *pack_kv(*even)) == 0 and run(p, q, *even, True) == 0
+            with torch.cuda.stream(side):
+                assert run(p, q, *pack_kv(*even)) == 0
+        assert run(plain, q, *pack_kv(*odd)) == 0 and run(plain, q, *odd, True) == 0
+        torch.cuda.synchronize()
+        # attachments on a count that is no multiple of 8: the unattached variant is the caller's to choose
+        assert run(attached, q, *pack_kv(*odd)) is None and run(attached, q, *odd, True) is None
+        kp, vp = pack_kv(*even)
+        strided = q.transpose(0, 1).contiguous().transpose(0, 1)
+        other = torch.float16 if dtype == torch.bfloat16 else torch.bfloat16
+        for bad in ((strided, kp, vp), (q[:5], kp, vp), (q.to(other), kp, vp), (q, kp.to(other), vp), (q, kp, vp[:, :-8]),
+                    (q, kp.transpose(1, 2), vp), (q.cpu(), kp, vp), (q, kp.cpu(), vp), (q, kp[0], vp), (q, kp, None)):
+            assert run(plain, *bad) is None
+        for bad in ((q, kp, vp), (q, k[:, :, :64], v), (q, k.transpose(0, 1), v), (q, k[:-8], v)):
+            assert run(plain, *bad, True) is None
+        shifted = torch.empty(k.numel() + 1, dtype=dtype, device=device)[1:].view(k.shape).copy_(k)
+        assert run(plain, q, shifted, v, True) is None  # 2 bytes off: a packed copy is aligned
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rope_rows", [1, 6])
+def test_decode_append_calls_that_the_module_takes(dtype, rope_rows, device):
+    nreq, hq, hk, d, cap = 6, 8, 2, 64, 40
+    q, k, v = (torch.randn(nreq, 1, h, d, device=device).to(dtype) for h in (hq, hk, hk))
+    cos, sin = (torch.randn(rope_rows, 1, d, device=device).to(dtype) for _ in range(2))
+    kp, vp = torch.zeros(hk, d, cap, dtype=dtype, device=device), torch.zeros(hk, cap, d, dtype=dtype, device=device)
+    slots = torch.arange(nreq, dtype=torch.int32, device=device)
+    _native.load()
+    call = _native.fastcall.decode_append
+    flat = [t.reshape(nreq, -1, d) for t in (q, k, v)]
+    for args in ((q, k, v, cos, sin, slots, kp, vp), (*flat, cos[:, 0], sin[:, 0], slots, kp, vp)):
+        out = call(*args)
+        assert isinstance(out, torch.Tensor) and out.shape == (nreq, hq, d)
+        with torch.cuda.stream(torch.cuda.Stream()):
+            assert isinstance(call(*args), torch.Tensor)
+    torch.cuda.synchronize()
+    strided = torch.stack([q, q], dim=-1)[..., 0]
+    for bad in ((strided, k, v, cos, sin, slots, kp, vp), (q, k, v, cos, sin, slots.long(), kp, vp),
+                (q, k, v, cos, sin, slots[:3], kp, vp), (q, k, v, cos.float(), sin, slots, kp, vp),
+                (q, k[:3], v, cos, sin, slots, kp, vp), (q, k, v, cos, sin, slots.cpu(), kp, vp),
+                (q, k, v, cos, sin, slots, kp.transpose(1, 2), vp), (q, k, v, cos, sin, slots, kp, vp[:, :-1]),
+                (q, k, v, cos, sin, slots.tolist(), kp, vp)):
+        assert call(*bad) is None
+
+
+def test_fill_calls_that_the_module_takes(device):
+    _native.load()
+    call = _native.fastcall.fill
+    meta = torch.zeros(12, dtype=torch.int32, device=device)
+    at = torch.tensor([1, 5, 11], device=device)
+    assert call(meta, at, 7) == 0
+    with torch.cuda.stream(torch.cuda.Stream()):
+        assert call(meta, at[:0], 7) == 0
+    torch.cuda.synchronize()
+    assert meta.tolist() == [0, 7, 0, 0, 0, 7, 0, 0, 0, 0, 0, 7]
+    for bad in ((meta, at, -1), (meta, at, 2 ** 31), (meta, at, 1.5), (meta, at.int(), 7), (meta.long(), at, 7),
+                (meta.cpu(), at, 7), (meta, at.cpu(), 7), (meta, [1], 7)):
+        assert call(*bad) is None
+    assert meta.tolist() == [0, 7, 0, 0, 0, 7, 0, 0, 0, 0, 0, 7]
