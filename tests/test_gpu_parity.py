@@ -320,7 +320,7 @@ def test_attached_tails(hq, hk, d, dtype, pad, device):
     """Private tails folded into 256-row root items: ragged lengths (1..200 tokens, unaligned
     starts, several tiles), several per item, GQA groups 4/8/16; equal to the oracle, to the
     unattached plan, and to the explicit segment + merge launches.  pad 3 (pool capacity not a
-    multiple of 8) runs the unattached variant on the register-staged kernels."""
+    multiple of 8) runs the unattached variant on the kernels of those pools."""
     group = hq // hk
     nreq, root = {4: (96, 3001), 8: (48, 6001), 16: (24, 12001)}[group]
     tails = [1 + (37 * r) % 200 for r in range(nreq)]

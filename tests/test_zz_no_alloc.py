@@ -78,7 +78,7 @@ def test_noalloc_equals_attention_matrix(device):
 
 
 def test_noalloc_on_register_staged_pools(device):
-    """Pools whose capacity is not a multiple of 8 run the register-staged kernels and the
+    """Pools whose capacity is not a multiple of 8 bring K through registers and take the
     unfused order (every kind writes partials, then all requests merge): the variant keeps
     those partials in the array too.  Mixed kinds with up to 24 slots per request; two calls,
     the second on a smaller layer, each bit-identical to ta_attention_matrix."""
@@ -95,7 +95,7 @@ def test_noalloc_on_register_staged_pools(device):
         prepared = prepare(schedule(tree, 32, 8, 128, "cube", CostModel()), q).for_pools(kp)
         abi = prepared.abi
         assert not abi.xtail
-        say("noalloc register-staged", name, "slots", abi.nslot, "per request", abi.maxs, "items",
+        say("noalloc odd capacity", name, "slots", abi.nslot, "per request", abi.maxs, "items",
             list(abi.n_items))
         bare = _native.TaPlan.from_buffer_copy(abi)
         bare.part, bare.lse = None, None

@@ -1,6 +1,6 @@
-// segment_tile.hip -- gfx950 kernel for large segment jobs (more than 16 query rows).
+// segment_tile.hip -- gfx950 kernels of the segment launches: work items of every kind.
 //
-// Replaces the large phase of the reference's Triton _segment
+// Replaces the reference's Triton _segment
 // (src/tree_attention/kernels.py:8-55, launched at :158-165): grouped partial
 // attention of one physical KV segment for all requests of a job, online
 // softmax in fp32, P rounded to the input dtype before PV (kernels.py:49),
@@ -40,8 +40,9 @@
 // The kernels are templates over the layout of K and V (enum Layout): pools whose
 // capacity is a multiple of 8 (every 8-token chunk of a K row is one aligned
 // 16-byte copy), pools of any other capacity (K through registers) and
-// token-major K and V (K's operand read without transposing).  The text above
-// describes the first; TileCopy and KTokens say where the others differ.
+// token-major K and V (K's operand read without transposing) of a count that is a
+// multiple of 8 or any other.  The text above describes the first; TileCopy,
+// KTokens and RowSum say where the others differ.
 #include "ta_common.h"
 #include "tree_attn.h"
 
@@ -171,8 +172,8 @@ struct KTokens {
 // DMA, finish() waits for both and writes K to LDS at the slots the DMA would have
 // filled.  The tile's compute runs between the two and hides the loads.  Moving both
 // operands through registers with an 8 x 8 transpose took twice as long (24 ragged
-// requests in two branches, 10,839 tokens, d = 128: layer 49.2 us, here 26.7 us; 32
-// ragged requests, 1,745 tokens, d = 64: 14.2 us, here 8.4 us).
+// requests in two branches, 10,839 tokens, d = 128: layer 49.2 us, here 25.0 us; 32
+// ragged requests, 1,745 tokens, d = 64: 14.4 us, here 8.4 us).
 constexpr int SHORT_CAP = 1 << 28;
 template <int D, int NW, int L, bool SHORT = false>
 struct TileCopy {

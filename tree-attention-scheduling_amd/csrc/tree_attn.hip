@@ -389,6 +389,7 @@ int ta_segment_plan(const void *q, const void *kp, const void *vp, int32_t tcap,
 
 int ta_tail_merge(const void *q, const void *kp, const void *vp, int32_t tcap, const ta_plan *plan, void *out,
                   void *stream) {
+    // (pools of other capacities store a tail's partial like any other and merge all requests alike)
     if (!plan || !out || tcap % 8 != 0) return TA_ERR_ARG;
     return plan_segment(q, kp, vp, tcap, plan, TA_TAIL, out, KV_POOL, stream);
 }
