@@ -11,7 +11,7 @@ import torch
 
 from tree_attention import CostModel, schedule, shapes
 from tree_attention import _native
-from tree_attention.kernels import CachedDecodePlan, attention_matrix, decode_append, pack_kv, prepare
+from tree_attention.kernels import CachedDecodePlan, attention, attention_matrix, decode_append, pack_kv, prepare
 
 pytestmark = pytest.mark.gpu
 
@@ -194,3 +194,31 @@ def test_fill_calls_that_the_module_takes(device):
                 (meta.cpu(), at, 7), (meta, at.cpu(), 7), (meta, [1], 7)):
         assert call(*bad) is None
     assert meta.tolist() == [0, 7, 0, 0, 0, 7, 0, 0, 0, 0, 0, 7]
+
+
+def test_plans_with_attachments_on_any_count_stay_on_the_module(device, monkeypatch):
+    """attention_matrix and attention on a count that is no multiple of 8 under a plan with
+    attachments: the module runs the unattached variant, the Python path is not taken."""
+    tree = shapes.tree(shapes.shared_prefix(64, 2000, 5))
+    t = tree.storage_tokens + (tree.storage_tokens % 8 == 0)
+    q = torch.randn(64, 8, 64, device=device).half()
+    k, v = (torch.randn(t, 2, 64, device=device).half() for _ in range(2))
+    p = prepare(schedule(tree, 8, 2, 64, "cube", CostModel.mi355x()), q)
+    assert p.attached
+    codes = []
+    _native.load()
+
+    class Spy:
+        @staticmethod
+        def attention(*args):
+            codes.append(_native_call(*args))
+            return codes[-1]
+
+    _native_call = _native.fastcall.attention
+    kp, vp = pack_kv(k, v)
+    monkeypatch.setattr(_native, "fastcall", Spy)
+    a = attention_matrix(q, kp, vp, p).clone()
+    assert codes == [None, 0]
+    assert torch.equal(a, attention(q, k, v, p)) and codes == [None, 0] * 2
+    with pytest.raises(ValueError, match="share dtype"):
+        attention_matrix(q.bfloat16(), kp, vp, p)

@@ -867,11 +867,8 @@ def attention(q, k, v, prepared):
     times (``PACK_READS``) and anything that is not contiguous are packed first,
     and ``attention_matrix`` checks them.
     """
-    call = _fastcall().attention
-    rc = None
-    if getattr(k, "ndim", 0) == 3 and not prepared.packs(k.shape[0]):
-        p = prepared.for_capacity(k.shape[0])
-        rc = call(q, k, v, ctypes.addressof(p.abi), p.out, True)
+    narrow = prepared.narrow_reads and getattr(k, "ndim", 0) == 3 and prepared.packs(k.shape[0])
+    rc = None if narrow else _fast_layer(q, k, v, prepared, True)
     if rc is None:
         return attention_matrix(q, *pack_kv(k, v), prepared)
     if rc:
@@ -888,6 +885,18 @@ def _fastcall():
         except (RuntimeError, OSError):
             return _native.GeneralPath
     return _native.fastcall
+
+
+def _fast_layer(q, k, v, prepared, token_major):
+    """The layer through the host module: the library's code, or None for the general path.
+    A plan with attachments that does not go with K's token count runs its unattached variant."""
+    call = _fastcall().attention
+    rc = call(q, k, v, ctypes.addressof(prepared.abi), prepared.out, token_major)
+    if rc is None and prepared.attached and getattr(k, "ndim", 0) == 3:
+        p = prepared.for_capacity(k.shape[0 if token_major else 2])
+        if p is not prepared:
+            rc = call(q, k, v, ctypes.addressof(p.abi), p.out, token_major)
+    return rc
 
 
 def _check_inputs(q, kp, vp, p):
@@ -914,7 +923,7 @@ def attention_matrix(q, kp, vp, prepared):
     Returns ``prepared.out`` (``[R, HQ, D]`` in q's dtype), which every call
     overwrites, as in the reference.
     """
-    rc = _fastcall().attention(q, kp, vp, ctypes.addressof(prepared.abi), prepared.out, False)
+    rc = _fast_layer(q, kp, vp, prepared, False)
     if rc is not None:  # the ordinary call; None: the general path below
         if rc:
             _native.check(rc)
