@@ -229,7 +229,8 @@ int ta_fill_lengths(int32_t *metadata, const int64_t *offsets, int32_t n, int32_
  * with device events around whole launches (scripts/profile_kernel.py:17-33).
  * The next kernel this library launches on the calling host thread records
  * `start_event` when its dispatch begins and `stop_event` when it ends
- * (hipExtLaunchKernel); the hook then clears itself.  Both are hipEvent_t
+ * (hipExtLaunchKernel); the hook then clears itself (ta_fill_lengths, a plan's
+ * bookkeeping, leaves it to the kernel after it).  Both are hipEvent_t
  * created with timing enabled, or both NULL to clear the hook.  Not for use
  * under stream capture. */
 int ta_time_next_launch(void *start_event, void *stop_event);

@@ -11,7 +11,8 @@ import torch
 
 from tree_attention import CostModel, schedule, shapes
 from tree_attention import _native
-from tree_attention.kernels import CachedDecodePlan, attention, attention_matrix, decode_append, pack_kv, prepare
+from tree_attention.kernels import (CachedDecodePlan, attention, attention_matrix, decode_append, launch_durations_us,
+                                    pack_kv, prepare)
 
 pytestmark = pytest.mark.gpu
 
@@ -222,3 +223,15 @@ def test_plans_with_attachments_on_any_count_stay_on_the_module(device, monkeypa
     assert torch.equal(a, attention(q, k, v, p)) and codes == [None, 0] * 2
     with pytest.raises(ValueError, match="share dtype"):
         attention_matrix(q.bfloat16(), kp, vp, p)
+
+
+def test_timing_hook_passes_over_the_tails_update(device):
+    """launch_durations_us of a step that sets the tails' lengths first stamps the layer's kernel
+    (25 us and more here), not the update's (4 us, what any stamp of an empty kernel reads)."""
+    tree = shapes.tree(shapes.headline())
+    q = torch.randn(128, 32, 128, device=device).bfloat16()
+    cached = CachedDecodePlan(schedule(tree, 32, 8, 128, "cube", CostModel.mi355x()), q, tree.storage_tokens, 8)
+    t = tree.storage_tokens + 128 * 8
+    kp, vp = (torch.randn(*s, device=device).bfloat16() for s in ((8, 128, t), (8, t, 128)))
+    us = launch_durations_us(lambda i: attention_matrix(q, kp, vp, cached.update(i % 8)), 16)
+    assert min(us) > 15.0

