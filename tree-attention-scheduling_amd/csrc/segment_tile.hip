@@ -182,9 +182,10 @@ struct TileCopy {
     u32x4 k[L == KV_ODD ? NK : 1];
 
     // SHORT (short_offsets): a copy's source is a scalar base per block plus a 32-bit lane offset
-    // that all tiles of an item share; else a 64-bit address per lane.  In the one-wave kernel the short form streams 128 x 8192 private tokens in 768
-    // us against 782 us; in the mixed kernel, whose scalar registers are full, it is the slower
-    // one (32 requests x 4096 tokens: 42.8 us against 41.8 us).
+    // that all tiles of an item share; else a 64-bit address per lane.  In the one-wave kernel the
+    // short form streams 128 x 8192 private tokens in 768 us against 782 us; in the mixed kernel,
+    // whose scalar registers are full, it is the slower one (32 requests x 4096 tokens: 42.8 us
+    // against 41.8 us).
     __device__ static void dma(u16 *dst, const u16 *base, u32 ofs) {
         __builtin_amdgcn_global_load_lds((const void *)((const char *)base + ofs), (lds_void *)dst, 16, 0, 0);
     }
